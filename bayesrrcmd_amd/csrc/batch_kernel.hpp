@@ -29,6 +29,7 @@
 
 #include <type_traits>
 
+#include "mixture.hpp"
 #include "sweep_kernel.hpp"
 
 namespace brr {
@@ -81,7 +82,7 @@ struct BBlock {
     uint8_t codes[kBB][kBRow];        // byte b of row k: individuals lo + 4b .. 4b + 3 of marker k
     double wt[kBB][4];                // dot weight per 2-bit code (0 for markers past the block)
     double ut[kBB][4];                // residual change per unit beta change, per code
-    double mstat[kBB][3];             // ragged: mean, sd, Zsum
+    double mstat[kBB][4];             // ragged: mean, sd, Zsum, 1 / sd
     double bo[kBB][kMaxT];            // beta before the block
     uint32_t mk[kBB];                 // marker ids
 };
@@ -98,7 +99,7 @@ struct BShared {
     uint64_t zw[kBB][kMaxT];          // its normal: Philox words (chain) or the given z's bits
     uint16_t plist[kBB * kMaxT];      // pending pairs of a round after the first: k << 8 | t
     double gc[kMaxK][kMaxT];          // log pi_k - 0.5 log(logLScale S_k + 1)
-    double gden[kMaxK][kMaxT];        // denom_k
+    double grd[kMaxK][kMaxT];         // 1 / denom_k
     double gbsd[kMaxK][kMaxT];        // sqrt(sigmaE / denom_k)
     double dg[kMaxK][kMaxT];          // logL_k - logL_0 = dg_k + num^2 hk_k
     double hk[kMaxK][kMaxT];
@@ -282,7 +283,7 @@ __device__ __forceinline__ void bstore(const BatchParams& p, BBlock& L, const BN
         if (k >= nb) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) { L.wt[k][c] = 0.0; L.ut[k][c] = 0.0; }
-            L.mstat[k][0] = 0.0; L.mstat[k][1] = 1.0; L.mstat[k][2] = 0.0;
+            L.mstat[k][0] = 0.0; L.mstat[k][1] = 1.0; L.mstat[k][2] = 0.0; L.mstat[k][3] = 1.0;
         } else if (p.layout == kLayoutDense) {
             // 2-bit code v -> dosage: 0->2, 1->missing, 2->1, 3->0
             L.wt[k][0] = x.m2; L.wt[k][1] = x.m3; L.wt[k][2] = x.m1; L.wt[k][3] = x.m0;
@@ -296,6 +297,7 @@ __device__ __forceinline__ void bstore(const BatchParams& p, BBlock& L, const BN
             L.wt[k][1] = (p.layout == kLayoutEigen) ? mean : 0.0;   // EigenBayesRKernel: missing at the mean
             const double meanAdjustment = mean / sd;
             const double oneAdjustment = 1.0 / sd;
+            L.mstat[k][3] = oneAdjustment;
             L.ut[k][0] = -meanAdjustment + 2 * oneAdjustment;
             L.ut[k][1] = 0.0;
             L.ut[k][2] = -meanAdjustment + oneAdjustment;
@@ -319,111 +321,38 @@ __device__ __forceinline__ double bnum(const BShared& L, const BBlock& B, int k,
 {
     const double beta_old = B.bo[k][t];
     if (kDenseMath) return L.cd[k][t] + beta_old * NM1;
-    const double mean = B.mstat[k][0], sd = B.mstat[k][1];
-    return beta_old * (dN - 1.0) - mean * L.epsSum[t] / sd + L.cd[k][t] / sd;
+    const double mean = B.mstat[k][0], rsd = B.mstat[k][3];
+    return beta_old * (dN - 1.0) - mean * L.epsSum[t] * rsd + L.cd[k][t] * rsd;
 }
 
-// logL and mu of every component (BayesRBase.cpp:309-333)
-template <int kK>
-__device__ __forceinline__ void blogl(const BShared& L, int t, int K, double num, double (&logL)[kK],
-                                      double (&muk)[kK])
-{
-    const double sigmaE = L.sigmaE[t];
-    logL[0] = L.gc[0][t];
-    muk[0] = 0.0;
-#pragma unroll
-    for (int c = 1; c < kK; ++c) {
-        muk[c] = 0.0;
-        logL[c] = 0.0;
-        if (c < K) {
-            muk[c] = num / L.gden[c][t];
-            logL[c] = L.gc[c][t] + 0.5 * (muk[c] * num) / sigmaE;
-        }
-    }
-}
-
-// The draw of processColumn (BayesRBase.cpp:335-366) from num, u and z. With
-// d_k = logL_k - logL_0 = dg_k + num^2 hk_k, the probability terms
-// 1 / sum_i exp(logL_i - logL_c) equal exp(d_c) / sum_i exp(d_i); while every
-// |d_k| <= 350 no 700 guard can fire and no exponential overflows, so they are
-// formed from one set of K - 1 exponentials. Otherwise the reference's own
-// formulation, guards included, is evaluated.
+// The draw of processColumn (BayesRBase.cpp:335-366) from num, u and z.
 struct BDraw {
     double bnew, acum0;
     int sel;
 };
 
-template <int kK>
+template <int kK, bool kExact>
 __device__ __forceinline__ BDraw bdraw_k(const BShared& L, int t, int K, double num, double beta_old, double u,
                                        uint64_t zw, bool zwords)
 {
-    const double n2 = num * num;
-    double d[kK];
-    d[0] = 0.0;
-    bool far = false;
-#pragma unroll
-    for (int c = 1; c < kK; ++c) {
-        d[c] = 0.0;
-        if (c < K) {
-            d[c] = L.dg[c][t] + n2 * L.hk[c][t];
-            far = far || fabs(d[c]) > 350.0;
-        }
-    }
-    BDraw r{beta_old, 0.0, -1};
-    if (!far) {
-        double e[kK];
-        double S = 1.0;
-        e[0] = 1.0;
-#pragma unroll
-        for (int c = 1; c < kK; ++c) {
-            e[c] = 0.0;
-            if (c < K) {
-                e[c] = exp(d[c]);
-                S += e[c];
-            }
-        }
-        const double invS = 1.0 / S;
-        double acum = invS;
-        r.acum0 = acum;
-#pragma unroll
-        for (int c = 0; c < kK; ++c) {
-            if (c < K && r.sel < 0) {
-                if (u <= acum) r.sel = c;
-                else if (c + 1 < kK && c + 1 < K) acum += e[c + 1 < kK ? c + 1 : 0] * invS;
-            }
-        }
-    } else {
-        double logL[kK], muk[kK];
-        blogl<kK>(L, t, K, num, logL, muk);
-        double acum = guard700(logL, K, logL[0]) ? 0.0 : inv_sum_exp(logL, K, logL[0]);
-        r.acum0 = acum;
-#pragma unroll 1
-        for (int c = 0; c < K; ++c) {
-            if (u <= acum) { r.sel = c; break; }
-            if (c + 1 < K) {
-                double ref = 0.0;
-#pragma unroll
-                for (int q = 1; q < kK; ++q)
-                    if (q == c + 1) ref = logL[q];
-                if (!guard700(logL, K, ref)) acum += inv_sum_exp(logL, K, ref);
-            }
-        }
-    }
+    const MixDraw m = mix_draw<kK, kExact>(K, num * num, u, [&](int c) { return L.dg[c][t]; },
+                                   [&](int c) { return L.hk[c][t]; }, [&](int c) { return L.gc[c][t]; });
+    BDraw r{beta_old, m.acum0(), m.sel};
     if (r.sel == 0) {
         r.bnew = 0.0;
     } else if (r.sel > 0) {
         const double z = zwords ? unit_normal((uint32_t)(zw >> 32), (uint32_t)zw) : bits_as_double(zw);
-        r.bnew = z * L.gbsd[r.sel][t] + num / L.gden[r.sel][t];
+        r.bnew = z * L.gbsd[r.sel][t] + num * L.grd[r.sel][t];
     }
     return r;
 }
 
-// The loops unrolled to 4 components when K <= 4 (the usual mixture), else to kMaxK.
+// Four components (the usual mixture) as straight-line code, else room for kMaxK.
 __device__ __forceinline__ BDraw bdraw(const BShared& L, int t, int K, double num, double beta_old, double u,
                                        uint64_t zw, bool zwords)
 {
-    return K <= 4 ? bdraw_k<4>(L, t, K, num, beta_old, u, zw, zwords)
-                  : bdraw_k<kMaxK>(L, t, K, num, beta_old, u, zw, zwords);
+    return K == 4 ? bdraw_k<4, true>(L, t, K, num, beta_old, u, zw, zwords)
+                  : bdraw_k<kMaxK, false>(L, t, K, num, beta_old, u, zw, zwords);
 }
 
 // -------------------------------------------------------------------- kernel --
@@ -562,17 +491,17 @@ bayesr_batch_kernel(BatchParams p)
             const double sigmaG = L.sigmaG[t], sigmaE = L.sigmaE[t];
             if (k == 0) {
                 L.gc[0][t] = log(L.pi[0][t]);
-                L.gden[0][t] = 0.0;
+                L.grd[0][t] = 0.0;
                 L.gbsd[0][t] = 0.0;
             } else {
                 const double S = L.cva[k];
                 const double sigmaEOverSigmaG = sigmaE / sigmaG;
                 const double den = NM1 + sigmaEOverSigmaG * (1.0 / S);
                 const double logLScale = sigmaG / sigmaE * NM1;
-                L.gden[k][t] = den;
+                L.grd[k][t] = 1.0 / den;
                 L.gc[k][t] = log(L.pi[k][t]) - 0.5 * log(logLScale * S + 1.0);
                 L.gbsd[k][t] = __dsqrt_rn(sigmaE / den);
-                L.hk[k][t] = 0.5 / (den * sigmaE);
+                L.hk[k][t] = 0.5 / (den * sigmaE);   // logL_k = gc_k + num^2 hk_k
             }
         }
         __syncthreads();
