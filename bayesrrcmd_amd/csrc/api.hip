@@ -14,16 +14,20 @@
 
 #include "brr_hip.h"
 #include "sweep_kernel.hpp"
+#include "pipe_kernel.hpp"
 #include "batch_kernel.hpp"
 #include "bayesw_kernel.hpp"
 #include "bed_kernels.hpp"
 #include "kernels.hpp"
 
 namespace brr {
-// instantiated in kern_sweep_seq.hip, kern_sweep_async.hip, kern_batch.hip, kern_bayesw.hip
-BRR_SWEEP_KERNELS_OF(BRR_SWEEP_DECL, false)
-BRR_SWEEP_KERNELS_OF(BRR_SWEEP_DECL, true)
-BRR_SWEEP_F32_KERNELS(BRR_SWEEP_DECL)
+// instantiated in the kern_*.hip files
+BRR_SWEEP_SEQ_KERNELS(BRR_SWEEP_DECL)
+BRR_SWEEP_ASYNC_KERNELS(BRR_SWEEP_DECL)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, false)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, true)
+BRR_GRAM_DECL(false)
+BRR_GRAM_DECL(true)
 BRR_COHORT_KERNELS(BRR_COHORT_DECL)
 BRR_BATCH_KERNELS(BRR_BATCH_DECL)
 BRR_BATCH_F32_KERNELS(BRR_BATCH_DECL)
@@ -62,7 +66,16 @@ struct brr_hip_ctx {
     double* d_num = nullptr;     // per-marker num of the last sweep (brr_hip_record_num)
     double* d_keps = nullptr;    // N: a host residual / residual change of the per-marker kernel calls
     SweepParams* d_cohort = nullptr;   // brr_hip_run_cohorts: the cohorts' parameter blocks
+    GramEntry* d_cohort_gram = nullptr;
     uint32_t cohort_cap = 0;
+    // pipelined sweep (gram_kernel.hpp): individuals per 2-bit value of each column, whether a call is missing,
+    // and the Gram rows (with shared counts where few blocks split the individuals) kept between launches
+    uint32_t* d_counts = nullptr;
+    bool missing = false;
+    double* d_gram = nullptr;
+    size_t gram_cap = 0;         // rows
+    int32_t* d_gram_acc = nullptr;
+    size_t gram_acc_cap = 0;     // rows x products
     uint64_t* h_status = nullptr; // pinned: control words, counters and order flag of brr_hip_sweep_noalloc
     bool record_num = false;
     uint32_t refresh_markers = 1024;
@@ -322,41 +335,72 @@ SweepParams base_params(brr_hip_ctx* c)
     return p;
 }
 
-template <int R, bool kAsync>
-const void* kernel_ra(int layout, bool codes)
+template <int R>
+const void* async_kernel(int layout, bool codes)
 {
-    if (layout == kLayoutDense) return (const void*)bayesr_sweep_kernel<R, kLayoutDense, true, kAsync, false>;
+    if (layout == kLayoutDense) return (const void*)bayesr_sweep_kernel<R, kLayoutDense, true, true, false>;
     if (layout == kLayoutEigen)   // Eigen contexts hold codes
-        return codes ? (const void*)bayesr_sweep_kernel<R, kLayoutEigen, true, kAsync, false> : nullptr;
-    return codes ? (const void*)bayesr_sweep_kernel<R, kLayoutRagged, true, kAsync, false>
-                 : (const void*)bayesr_sweep_kernel<R, kLayoutRagged, false, kAsync, false>;
+        return codes ? (const void*)bayesr_sweep_kernel<R, kLayoutEigen, true, true, false> : nullptr;
+    return codes ? (const void*)bayesr_sweep_kernel<R, kLayoutRagged, true, true, false>
+                 : (const void*)bayesr_sweep_kernel<R, kLayoutRagged, false, true, false>;
 }
 
-// FP32 residual kernels: sequential sweeps over 2-bit codes only
-template <int R>
-const void* kernel_f32(int layout, bool codes)
+template <int R, bool kF32>
+const void* pipe_kernel(int layout)
 {
-    if (!codes) return nullptr;
-    if (layout == kLayoutDense) return (const void*)bayesr_sweep_kernel<R, kLayoutDense, true, false, true>;
-    if (layout == kLayoutEigen) return (const void*)bayesr_sweep_kernel<R, kLayoutEigen, true, false, true>;
-    return (const void*)bayesr_sweep_kernel<R, kLayoutRagged, true, false, true>;
+    if (layout == kLayoutDense) return (const void*)bayesr_pipe_kernel<R, kLayoutDense, kF32>;
+    if (layout == kLayoutEigen) return (const void*)bayesr_pipe_kernel<R, kLayoutEigen, kF32>;
+    return (const void*)bayesr_pipe_kernel<R, kLayoutRagged, kF32>;
 }
 
-template <int R>
-const void* kernel_r(int layout, bool codes, bool async, bool f32)
+template <bool kF32>
+const void* four_run_kernel(int layout)
 {
-    if (f32) return async ? nullptr : kernel_f32<R>(layout, codes);
-    return async ? kernel_ra<R, true>(layout, codes) : kernel_ra<R, false>(layout, codes);
+    if (layout == kLayoutDense) return (const void*)bayesr_sweep_kernel<4, kLayoutDense, true, false, kF32>;
+    if (layout == kLayoutEigen) return (const void*)bayesr_sweep_kernel<4, kLayoutEigen, true, false, kF32>;
+    return (const void*)bayesr_sweep_kernel<4, kLayoutRagged, true, false, kF32>;
 }
 
-const void* kernel_for(uint32_t R, int layout, bool codes, bool async = false, bool f32 = false)
+// The kernel of a single-chain context and its workgroup size.
+struct SweepKernel {
+    const void* fn;
+    uint32_t threads;
+    bool pipe;
+};
+
+// Sequential sweeps over 2-bit codes take the pipelined kernel while a slice is one or two lane runs (four runs'
+// columns do not fit its LDS ring: N above 262,144 on 256 workgroups). A sequential sweep in FP64 blocks of one
+// marker is the asynchronous sweep with windows of one, without dots to correct.
+SweepKernel kernel_for(uint32_t R, int layout, bool codes, bool async, bool f32, uint32_t B)
 {
-    switch (R) {
-    case 1: return kernel_r<1>(layout, codes, async, f32);
-    case 2: return kernel_r<2>(layout, codes, async, f32);
-    case 4: return kernel_r<4>(layout, codes, async, f32);
-    default: return nullptr;
+    if (f32 && (async || !codes)) return {nullptr, kThreads, false};
+    if (async || (codes && !f32 && B == 1)) {
+        switch (R) {
+        case 1: return {async_kernel<1>(layout, codes), kThreads, false};
+        case 2: return {async_kernel<2>(layout, codes), kThreads, false};
+        case 4: return {async_kernel<4>(layout, codes), kThreads, false};
+        default: return {nullptr, kThreads, false};
+        }
     }
+    if (!codes) {
+        switch (R) {
+        case 1: return {(const void*)bayesr_sweep_kernel<1, kLayoutRagged, false, false, false>, kThreads, false};
+        case 2: return {(const void*)bayesr_sweep_kernel<2, kLayoutRagged, false, false, false>, kThreads, false};
+        case 4: return {(const void*)bayesr_sweep_kernel<4, kLayoutRagged, false, false, false>, kThreads, false};
+        default: return {nullptr, kThreads, false};
+        }
+    }
+    switch (R) {
+    case 1: return {f32 ? pipe_kernel<1, true>(layout) : pipe_kernel<1, false>(layout), kPipeThreads, true};
+    case 2: return {f32 ? pipe_kernel<2, true>(layout) : pipe_kernel<2, false>(layout), kPipeThreads, true};
+    case 4: return {f32 ? four_run_kernel<true>(layout) : four_run_kernel<false>(layout), kThreads, false};
+    default: return {nullptr, kThreads, false};
+    }
+}
+
+SweepKernel kernel_of(const brr_hip_ctx* c)
+{
+    return kernel_for(c->R, c->layout, c->codes, c->async != 0, c->f32, c->B);
 }
 
 const void* cohort_kernel_for(uint32_t R, bool f32)
@@ -542,15 +586,15 @@ int reset_exchange(brr_hip_ctx* c)
     return BRR_HIP_OK;
 }
 
-// One cooperative launch of the context's kernel with argument block `param`.
-int launch_fn(brr_hip_ctx* c, const void* fn, void* param)
+// Runs enqueue() -- the launches of one call -- on the context's stream between two events and reads the control
+// words and counters back.
+template <class Enqueue>
+int run_launches(brr_hip_ctx* c, Enqueue&& enqueue)
 {
-    if (!fn) return fail(c, BRR_HIP_EINVAL, "unsupported slice size");
     HIP_TRY(c, hipMemsetAsync(c->d_ctl + kCtlAbort, 0, sizeof(uint32_t) * 2, c->stream));
     HIP_TRY(c, hipMemsetAsync(c->d_counters, 0, sizeof(unsigned long long) * kCounters, c->stream));
-    void* args[] = {param};
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
-    HIP_TRY(c, hipLaunchCooperativeKernel(fn, dim3(c->P), dim3(kThreads), args, 0, c->stream));
+    HIP_TRY(c, enqueue());
     HIP_TRY(c, hipEventRecord(c->ev1, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     float ms = 0.f;
@@ -581,13 +625,147 @@ int launch_fn(brr_hip_ctx* c, const void* fn, void* param)
     return BRR_HIP_OK;
 }
 
+// One cooperative launch of the context's kernel with argument block `param`.
+int launch_fn(brr_hip_ctx* c, const void* fn, void* param, uint32_t threads = kThreads)
+{
+    if (!fn) return fail(c, BRR_HIP_EINVAL, "unsupported slice size");
+    void* args[] = {param};
+    return run_launches(c, [&] {
+        return hipLaunchCooperativeKernel(fn, dim3(c->P), dim3(threads), args, 0, c->stream);
+    });
+}
+
+// ------------------------------------------------------ pipelined sweep --
+
+// Rows of the Gram workspace one launch may fill when it runs several iterations (1 KB a row).
+constexpr size_t kGramRowsPerLaunch = 65536;
+// Blocks from which a Gram launch fills the chip without splitting the individuals.
+constexpr uint32_t kGramBlocks = 128;
+
+uint32_t gram_iterations(const brr_hip_ctx* c, uint32_t iterations)
+{
+    return (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, kGramRowsPerLaunch / c->cfg.num_snps));
+}
+
+uint32_t gram_splits(const brr_hip_ctx* c, uint32_t iterations)
+{
+    const uint32_t blocks = iterations * ((c->cfg.num_snps + c->B - 1) / c->B);
+    const uint32_t chunks = (c->cfg.num_inds + kGramChunk - 1) / kGramChunk;
+    return blocks >= kGramBlocks ? 1u : std::max(1u, std::min(2 * kGramBlocks / blocks, chunks));
+}
+
+int gram_products_of(const brr_hip_ctx* c) { return c->missing ? gram_products(c->layout) : 1; }
+
+// The workspace of a launch of `iterations` iterations.
+int gram_reserve(brr_hip_ctx* c, uint32_t iterations)
+{
+    const size_t rows = (size_t)iterations * c->cfg.num_snps;
+    int rc;
+    if (c->gram_cap < rows) {
+        c->gram_cap = 0;
+        if ((rc = dalloc(c, &c->d_gram, rows * kGramCols))) return rc;
+        c->gram_cap = rows;
+    }
+    // (a block is at most 64 rows; whether it is split depends on the block size, which may change later)
+    const size_t acc = rows <= (size_t)kGramBlocks * kMaxB ? rows * gram_products_of(c) : 0;
+    if (c->gram_acc_cap < acc) {
+        c->gram_acc_cap = 0;
+        if ((rc = dalloc(c, &c->d_gram_acc, acc * kGramCols))) return rc;
+        HIP_TRY(c, hipMemsetAsync(c->d_gram_acc, 0, sizeof(int32_t) * acc * kGramCols, c->stream));
+        c->gram_acc_cap = acc;
+    }
+    return BRR_HIP_OK;
+}
+
+GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t iterations, const uint32_t* gate)
+{
+    GramParams g{};
+    g.N = c->cfg.num_inds;
+    g.M = c->cfg.num_snps;
+    g.B = c->B;
+    g.iterations = iterations;
+    g.layout = c->layout;
+    g.splits = gram_splits(c, iterations);
+    g.codes = c->d_dense;
+    g.col_words = c->col_words;
+    g.counts = c->d_counts;
+    g.lut = c->d_lut;
+    g.stats = c->d_stats;
+    g.order = order;
+    g.gram = c->d_gram;
+    g.acc = c->d_gram_acc;
+    g.gate = gate;
+    return g;
+}
+
+// The Gram rows of `iterations` iterations, then the pipelined kernel over them.
+hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, uint32_t iterations)
+{
+    if (p.mode == kModeSweep || p.mode == kModeChain) {
+        GramParams g = gram_params(c, p.order, iterations, p.gate);
+        const uint32_t items = iterations * ((g.M + g.B - 1) / g.B) * g.splits;
+        if (c->missing) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
+        else gram_kernel<false><<<items, kGramThreads, 0, c->stream>>>(g);
+        if (hipError_t e = hipGetLastError()) return e;
+        if (g.splits > 1) {
+            gram_finish_kernel<<<iterations * g.M, kGramCols, 0, c->stream>>>(g, gram_products_of(c));
+            if (hipError_t e = hipGetLastError()) return e;
+        }
+    }
+    p.gram = c->d_gram;
+    void* args[] = {&p};
+    return hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream);
+}
+
+// Per-marker counts of the columns just stored, and the Gram workspace of a sweep (so that sweeps allocate
+// nothing). `counted`: the caller has the counts in place (and `missing` set).
+int prepare_pipe(brr_hip_ctx* c, bool counted)
+{
+    if (c->T || c->bw || !c->codes) return BRR_HIP_OK;
+    int rc;
+    const uint32_t M = c->cfg.num_snps;
+    if (!counted) {
+        if ((rc = dalloc(c, &c->d_counts, (size_t)4 * M + 1))) return rc;
+        uint32_t* any = c->d_counts + 4 * (size_t)M;
+        uint32_t got = 0;
+        HIP_TRY(c, hipMemsetAsync(any, 0, sizeof(uint32_t), c->stream));
+        marker_counts_kernel<<<M, 256, 0, c->stream>>>(c->d_dense, c->col_words, c->cfg.num_inds, c->d_counts, any);
+        HIP_TRY(c, hipGetLastError());
+        HIP_TRY(c, hipMemcpyAsync(&got, any, sizeof(got), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        c->missing = got != 0;
+    }
+    if ((rc = gram_reserve(c, 1))) return rc;
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    return BRR_HIP_OK;
+}
+
 int launch(brr_hip_ctx* c, SweepParams& p)
 {
     p.refresh_blocks = std::max(1u, c->refresh_markers / c->B);
     if (c->f32 && !c->codes)
         return fail(c, BRR_HIP_ESTATE, "the FP32 residual mode needs the columns held as 2-bit codes "
                                        "(ragged_storage 0 or 2)");
-    return launch_fn(c, kernel_for(c->R, c->layout, c->codes, c->async != 0, c->f32), &p);
+    const SweepKernel k = kernel_of(c);
+    if (!k.pipe) return launch_fn(c, k.fn, &p, k.threads);
+    if (p.mode != kModeChain) {
+        if (int rc = gram_reserve(c, 1)) return rc;
+        return run_launches(c, [&] { return enqueue_pipe(c, k, p, 1); });
+    }
+    // a chain in launches of as many iterations as the Gram workspace holds
+    const uint32_t total = p.iterations, step = gram_iterations(c, total);
+    if (int rc = gram_reserve(c, step)) return rc;
+    return run_launches(c, [&] {
+        for (uint32_t it = 0; it < total; it += step) {
+            SweepParams q = p;
+            q.iterations = std::min(step, total - it);
+            q.iter_base = p.iter_base + it;
+            q.order = p.order + (size_t)it * p.M;
+            q.hist = p.hist ? p.hist + (size_t)it * (4 + p.G) : nullptr;
+            if (hipError_t e = enqueue_pipe(c, k, q, q.iterations)) return e;
+        }
+        return hipSuccess;
+    });
 }
 
 // Batched contexts: the same launch with the sweep-mode / chain-mode fields of p.
@@ -705,6 +883,7 @@ int configure_shape(brr_hip_ctx* c, uint32_t workgroups, uint32_t block)
     if (block > (uint32_t)kMaxB) return fail(c, BRR_HIP_EINVAL, "block_markers must be 0..64");
     uint32_t S, R = 0, nt = 0, NT = 0;
     const void* probe;
+    uint32_t threads = kThreads;
     if (c->T) {
         const uint32_t Preq = workgroups ? std::min(workgroups, Pmax) : Pmax;
         S = (N + Preq - 1) / Preq;
@@ -718,11 +897,14 @@ int configure_shape(brr_hip_ctx* c, uint32_t workgroups, uint32_t block)
         R = (S + kRun - 1) / kRun;
         if (R == 3) R = 4;
         if (R > (uint32_t)kMaxRuns) return fail(c, BRR_HIP_EINVAL, "slices hold at most 2048 individuals");
-        probe = kernel_for(R, c->layout, c->codes || c->layout == kLayoutEigen, c->async != 0, c->f32);
+        const SweepKernel k = kernel_for(R, c->layout, c->codes || c->layout == kLayoutEigen, c->async != 0, c->f32,
+                                         block && !c->async ? block : c->B);
+        probe = k.fn;
+        threads = k.threads;
     }
     const uint32_t P = (N + S - 1) / S;
     int occ = 0;
-    if (!probe || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, probe, kThreads, 0) != hipSuccess ||
+    if (!probe || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, probe, (int)threads, 0) != hipSuccess ||
         (uint64_t)occ * c->cus < P)
         return fail(c, BRR_HIP_EDEVICE, "the launch shape does not fit the device");
     const size_t x1 = c->T ? (size_t)2 * P * kBVmax * 2 : (size_t)2 * kSlots * P * 2;
@@ -845,6 +1027,7 @@ int brr_hip_create(const brr_hip_config* cfg, brr_hip_ctx** out)
     c->T = cfg->num_traits;
     c->Tn = c->T ? c->T : 1u;
     const void* probe = nullptr;
+    uint32_t threads = kThreads;
     if (c->T) {
         // batched traits: residuals of a slice in registers as 16-row tiles;
         // ragged columns are held as 2-bit codes
@@ -862,7 +1045,11 @@ int brr_hip_create(const brr_hip_config* cfg, brr_hip_ctx** out)
         c->R = R;
         c->B = cfg->block_markers ? cfg->block_markers : 64u;
         c->B_seq = c->B;
-        probe = kernel_for(R, (int)cfg->layout, c->layout == kLayoutEigen);
+        // (a ragged context's storage is chosen at its upload: 2-bit codes unless lists are asked for)
+        const SweepKernel k = kernel_for(R, (int)cfg->layout, c->layout != kLayoutRagged || cfg->ragged_storage != 1, false,
+                                         false, c->B);
+        probe = k.fn;
+        threads = k.threads;
     }
     c->S = S;
     c->P = (N + S - 1) / S;
@@ -871,7 +1058,7 @@ int brr_hip_create(const brr_hip_config* cfg, brr_hip_ctx** out)
     c->x2_words = c->T ? kCopies * kBCopyWords : kCopies * kCopyWords;
 
     int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, probe, kThreads, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, probe, (int)threads, 0) != hipSuccess ||
         (uint64_t)occ * cus < c->P) {
         delete c;
         return BRR_HIP_EDEVICE;
@@ -923,6 +1110,7 @@ void brr_hip_destroy(brr_hip_ctx* c)
     dfree(c->d_scal); dfree(c->d_hist); dfree(c->d_order); dfree(c->d_u); dfree(c->d_z);
     dfree(c->d_xchg1); dfree(c->d_xchg2); dfree(c->d_ctl); dfree(c->d_counters); dfree(c->d_tmp);
     dfree(c->d_fail); dfree(c->d_sumf); dfree(c->d_num); dfree(c->d_keps); dfree(c->d_cohort);
+    dfree(c->d_cohort_gram); dfree(c->d_counts); dfree(c->d_gram); dfree(c->d_gram_acc);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -953,6 +1141,7 @@ int brr_hip_upload_dense(brr_hip_ctx* c, const uint8_t* bed, uint64_t column_str
     HIP_TRY(c, hipMemcpy2D(c->d_dense, c->col_words * 4, bed, column_stride, col_bytes, M,
                            hipMemcpyHostToDevice));
     HIP_TRY(c, hipMemcpy(c->d_lut, lut, sizeof(double) * 4 * M, hipMemcpyHostToDevice));
+    if (!c->bw && (rc = prepare_pipe(c, false))) return rc;
     c->have_markers = true;
     if (c->bw) {
         // a BayesW context takes its layout from the markers it is given
@@ -1036,6 +1225,7 @@ int brr_hip_upload_ragged(brr_hip_ctx* c, const int32_t* ones, const uint64_t* o
         // BayesR kernels too, once the lists are gone)
         dfree(c->d_ones); dfree(c->d_twos); dfree(c->d_miss);
     }
+    if ((rc = prepare_pipe(c, false))) return rc;
     c->have_markers = true;
     c->have_model = c->have_model && !c->bw;   // sum_failure depends on the columns
     return BRR_HIP_OK;
@@ -1064,14 +1254,13 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
     const uint64_t payload = cb * M;
     const uint64_t stage_words = (payload + 32 + 3) / 4;
     uint32_t* d_stage = nullptr;
-    uint32_t* d_cnt = nullptr;
+    uint32_t*& d_cnt = c->d_counts;
     int rc;
-    if ((rc = dalloc(c, &d_stage, stage_words)) || (rc = dalloc(c, &d_cnt, (size_t)4 * M + 1))) {
+    if ((rc = dalloc(c, &d_stage, stage_words)) || (rc = dalloc(c, &d_cnt, (size_t)4 * M + 2))) {
         dfree(d_stage);
-        dfree(d_cnt);
         return rc;
     }
-    auto cleanup = [&]() { dfree(d_stage); dfree(d_cnt); };
+    auto cleanup = [&]() { dfree(d_stage); };
     auto hip_ok = [&](hipError_t e, const char* what) {
         if (e == hipSuccess) return true;
         fail(c, BRR_HIP_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
@@ -1092,8 +1281,9 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
         cleanup();
         return rc;
     }
-    uint32_t* d_bad = d_cnt + 4 * (size_t)M;
+    uint32_t* d_bad = d_cnt + 4 * (size_t)M;   // first unusable marker; whether any call is missing
     if (!hip_ok(hipMemsetAsync(d_bad, 0xFF, sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
+        !hip_ok(hipMemsetAsync(d_bad + 1, 0, sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
         !hip_ok(hipEventRecord(c->ev0, c->stream), "hipEventRecord"))
         return BRR_HIP_EDEVICE;
     bed_unpack_kernel<<<M, kBedThreads, 0, c->stream>>>(d_stage, cb, N, c->col_words, c->d_dense, d_cnt,
@@ -1114,8 +1304,10 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
             return BRR_HIP_EDEVICE;
         (void)hipEventElapsedTime(&ms_table, c->ev0, c->ev1);
     }
-    uint32_t bad = 0xFFFFFFFFu;
-    if (!hip_ok(hipMemcpy(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost), "hipMemcpy")) return BRR_HIP_EDEVICE;
+    uint32_t found[2] = {0xFFFFFFFFu, 0u};
+    if (!hip_ok(hipMemcpy(found, d_bad, sizeof(found), hipMemcpyDeviceToHost), "hipMemcpy")) return BRR_HIP_EDEVICE;
+    const uint32_t bad = found[0];
+    c->missing = found[1] != 0;
     cleanup();
     c->stats = brr_hip_stats{};
     shape_stats(c);
@@ -1129,6 +1321,7 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
                                            (layout == BRR_HIP_LAYOUT_EIGEN_SPARSE ? " has no nonzero call"
                                                                                   : " has no genotype 1 or 2 calls"));
     c->codes = true;
+    if ((rc = prepare_pipe(c, true))) return rc;
     if (c->bw) {
         c->layout = dense ? kLayoutDense : kLayoutRagged;
         c->cfg.layout = (uint32_t)layout;
@@ -1359,18 +1552,50 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
         launches[l].push_back(q);
         used[l] += ctxs[q]->P;
     }
-    // parameter blocks in launch order, on the device
-    std::vector<SweepParams> packed;
-    for (auto& L : launches)
-        for (uint32_t q : L) packed.push_back(params[q]);
-    if (c0->cohort_cap < n) {
-        c0->cohort_cap = 0;
-        if ((rc = dalloc(c0, &c0->d_cohort, n))) return rc;
-        c0->cohort_cap = n;
+    // Iterations per launch: as many as fit the cohorts' Gram workspaces (together at most eight launches' worth of
+    // one context, at least one iteration)
+    size_t rows1 = 0;
+    bool missing = false;
+    for (uint32_t q = 0; q < n; ++q) {
+        rows1 += ctxs[q]->cfg.num_snps;
+        missing = missing || ctxs[q]->missing;
     }
-    HIP_TRY(c0, hipMemcpy(c0->d_cohort, packed.data(), sizeof(SweepParams) * n, hipMemcpyHostToDevice));
-    // per launch, the counters' reset and the cooperative cohort kernel: recorded into
-    // one graph (or, with BRR_HIP_COHORTS_DIRECT, launched one after another)
+    const uint32_t step = (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, 8 * kGramRowsPerLaunch / rows1));
+    const uint32_t steps = (iterations + step - 1) / step;
+    for (uint32_t q = 0; q < n; ++q)
+        if ((rc = gram_reserve(ctxs[q], step))) return fail(c0, rc, ctxs[q]->err);
+    HIP_TRY(c0, hipDeviceSynchronize());
+    // parameter blocks by step in launch order, on the device; the Gram entries of all cohorts of a step in one launch
+    std::vector<SweepParams> packed;
+    std::vector<GramEntry> grams;
+    std::vector<uint32_t> gram_items(steps, 0);
+    for (uint32_t st = 0; st < steps; ++st) {
+        const uint32_t it0 = st * step, its = std::min(step, iterations - it0);
+        for (auto& L : launches)
+            for (uint32_t q : L) {
+                const brr_hip_ctx* c = ctxs[q];
+                SweepParams p = params[q];
+                p.iterations = its;
+                p.iter_base += it0;
+                p.order += (size_t)it0 * p.M;
+                p.hist += (size_t)it0 * (4 + p.G);
+                p.gram = c->d_gram;
+                packed.push_back(p);
+                GramEntry g{gram_params(c, p.order, its, nullptr), gram_items[st]};
+                g.p.splits = 1;
+                grams.push_back(g);
+                gram_items[st] += its * ((g.p.M + g.p.B - 1) / g.p.B);
+            }
+    }
+    if (c0->cohort_cap < packed.size()) {
+        c0->cohort_cap = 0;
+        if ((rc = dalloc(c0, &c0->d_cohort, packed.size())) || (rc = dalloc(c0, &c0->d_cohort_gram, grams.size()))) return rc;
+        c0->cohort_cap = (uint32_t)packed.size();
+    }
+    HIP_TRY(c0, hipMemcpy(c0->d_cohort, packed.data(), sizeof(SweepParams) * packed.size(), hipMemcpyHostToDevice));
+    HIP_TRY(c0, hipMemcpy(c0->d_cohort_gram, grams.data(), sizeof(GramEntry) * grams.size(), hipMemcpyHostToDevice));
+    // the cooperative cohort kernel of each launch: recorded into one graph with the counters' reset and the Gram
+    // launches (or, with BRR_HIP_COHORTS_DIRECT, launched one after another)
     std::vector<CohortTable> tables(launches.size());
     std::vector<const void*> fns(launches.size());
     uint32_t base = 0;
@@ -1387,20 +1612,27 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
         for (uint32_t q : launches[l]) R = std::max(R, ctxs[q]->R);
         fns[l] = cohort_kernel_for(R, c0->f32);
         int occ = 0;
-        if (!fns[l] || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fns[l], kThreads, 0) != hipSuccess ||
+        if (!fns[l] || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fns[l], kPipeThreads, 0) != hipSuccess ||
             (uint64_t)occ * c0->cus < wg)
             return fail(c0, BRR_HIP_EDEVICE, "a cohort launch does not fit the device");
         base += t.n;
     }
     auto enqueue = [&]() -> hipError_t {
-        for (size_t l = 0; l < launches.size(); ++l) {
-            CohortTable& t = tables[l];
-            cohort_reset_kernel<<<t.n, 64, 0, c0->stream>>>(t.params);
-            hipError_t e2 = hipGetLastError();
-            if (e2 != hipSuccess) return e2;
-            void* args[] = {&t};
-            e2 = hipLaunchCooperativeKernel(fns[l], dim3(t.first[t.n]), dim3(kThreads), args, 0, c0->stream);
-            if (e2 != hipSuccess) return e2;
+        cohort_reset_kernel<<<n, 64, 0, c0->stream>>>(c0->d_cohort);
+        if (hipError_t e2 = hipGetLastError()) return e2;
+        for (uint32_t st = 0; st < steps; ++st) {
+            const GramEntry* g = c0->d_cohort_gram + (size_t)st * n;
+            if (missing) gram_cohort_kernel<true><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
+            else gram_cohort_kernel<false><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
+            if (hipError_t e2 = hipGetLastError()) return e2;
+            for (size_t l = 0; l < launches.size(); ++l) {
+                CohortTable t = tables[l];
+                t.params += (size_t)st * n;
+                void* args[] = {&t};
+                const hipError_t e2 = hipLaunchCooperativeKernel(fns[l], dim3(t.first[t.n]), dim3(kPipeThreads), args, 0,
+                                                                 c0->stream);
+                if (e2 != hipSuccess) return e2;
+            }
         }
         return hipSuccess;
     };
@@ -1763,8 +1995,8 @@ int brr_hip_sweep_noalloc(brr_hip_ctx* c, const uint32_t* d_order, const double*
     if (c->f32 && !c->codes)
         return fail(c, BRR_HIP_ESTATE, "the FP32 residual mode needs the columns held as 2-bit codes "
                                        "(ragged_storage 0 or 2)");
-    const void* fn = kernel_for(c->R, c->layout, c->codes, c->async != 0, c->f32);
-    if (!fn) return fail(c, BRR_HIP_EINVAL, "unsupported slice size");
+    const SweepKernel k = kernel_of(c);
+    if (!k.fn) return fail(c, BRR_HIP_EINVAL, "unsupported slice size");
     HIP_TRY(c, hipSetDevice(c->device));
     uint64_t* base = nullptr;
     if ((rc = scratch_for(c, &base))) return rc;
@@ -1785,9 +2017,13 @@ int brr_hip_sweep_noalloc(brr_hip_ctx* c, const uint32_t* d_order, const double*
     p.counters = (unsigned long long*)(base + kOffCnt);
     p.gate = (const uint32_t*)(base + kOffFlag);
     p.refresh_blocks = std::max(1u, c->refresh_markers / c->B);
-    void* args[] = {&p};
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
-    HIP_TRY(c, hipLaunchCooperativeKernel(fn, dim3(c->P), dim3(kThreads), args, 0, c->stream));
+    if (k.pipe) {
+        HIP_TRY(c, enqueue_pipe(c, k, p, 1));   // (the Gram workspace was allocated with the markers)
+    } else {
+        void* args[] = {&p};
+        HIP_TRY(c, hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream));
+    }
     HIP_TRY(c, hipEventRecord(c->ev1, c->stream));
     HIP_TRY(c, hipMemcpyAsync(c->h_status, base + kOffCtl, sizeof(uint64_t) * kStatusWords, hipMemcpyDeviceToHost,
                               c->stream));

@@ -1,6 +1,6 @@
 // kern_cohort.hip -- the kernels that run several BayesR contexts (cohorts) in
 // one persistent launch (see kernels.hpp).
-#include "sweep_kernel.hpp"
+#include "pipe_kernel.hpp"
 #include "kernels.hpp"
 
 namespace brr {

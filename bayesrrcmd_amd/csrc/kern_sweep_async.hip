@@ -3,5 +3,5 @@
 #include "kernels.hpp"
 
 namespace brr {
-BRR_SWEEP_KERNELS_OF(BRR_SWEEP_INST, true)
+BRR_SWEEP_ASYNC_KERNELS(BRR_SWEEP_INST)
 } // namespace brr

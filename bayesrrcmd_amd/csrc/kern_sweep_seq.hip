@@ -1,7 +1,7 @@
-// kern_sweep_seq.hip -- the sequential BayesR sweep kernels (see kernels.hpp).
+// kern_sweep_seq.hip -- the round-by-round BayesR sweep kernels (see kernels.hpp).
 #include "sweep_kernel.hpp"
 #include "kernels.hpp"
 
 namespace brr {
-BRR_SWEEP_KERNELS_OF(BRR_SWEEP_INST, false)
+BRR_SWEEP_SEQ_KERNELS(BRR_SWEEP_INST)
 } // namespace brr

@@ -5,22 +5,28 @@
 // addresses for the launches and occupancy queries.
 #pragma once
 
-// bayesr_sweep_kernel<R, layout, codes, async, fp32>: FP64 residual
-#define BRR_SWEEP_KERNELS_OF(X, A)                                                                      \
-    X(1, kLayoutDense, true, A, false) X(1, kLayoutRagged, true, A, false)                              \
-    X(1, kLayoutRagged, false, A, false) X(1, kLayoutEigen, true, A, false)                             \
-    X(2, kLayoutDense, true, A, false) X(2, kLayoutRagged, true, A, false)                              \
-    X(2, kLayoutRagged, false, A, false) X(2, kLayoutEigen, true, A, false)                             \
-    X(4, kLayoutDense, true, A, false) X(4, kLayoutRagged, true, A, false)                              \
-    X(4, kLayoutRagged, false, A, false) X(4, kLayoutEigen, true, A, false)
+// bayesr_pipe_kernel<R, layout, fp32>: sequential sweeps over 2-bit codes, slices of up to 1,024 individuals
+#define BRR_PIPE_KERNELS_OF(X, F)                                                                       \
+    X(1, kLayoutDense, F) X(1, kLayoutRagged, F) X(1, kLayoutEigen, F)                                  \
+    X(2, kLayoutDense, F) X(2, kLayoutRagged, F) X(2, kLayoutEigen, F)
 
-// FP32 residual with FP64 refresh: sequential sweeps over 2-bit codes
-#define BRR_SWEEP_F32_KERNELS(X)                                                                        \
-    X(1, kLayoutDense, true, false, true) X(1, kLayoutRagged, true, false, true)                        \
-    X(1, kLayoutEigen, true, false, true) X(2, kLayoutDense, true, false, true)                         \
-    X(2, kLayoutRagged, true, false, true) X(2, kLayoutEigen, true, false, true)                        \
+// bayesr_sweep_kernel<R, layout, codes, async, fp32>: the sequential sweeps that the pipelined kernel does not
+// take (index lists; four lane runs, whose columns do not fit its LDS ring)
+#define BRR_SWEEP_SEQ_KERNELS(X)                                                                        \
+    X(1, kLayoutRagged, false, false, false) X(2, kLayoutRagged, false, false, false)                   \
+    X(4, kLayoutRagged, false, false, false) X(4, kLayoutDense, true, false, false)                     \
+    X(4, kLayoutRagged, true, false, false) X(4, kLayoutEigen, true, false, false)                      \
     X(4, kLayoutDense, true, false, true) X(4, kLayoutRagged, true, false, true)                        \
     X(4, kLayoutEigen, true, false, true)
+
+// asynchronous windows
+#define BRR_SWEEP_ASYNC_KERNELS(X)                                                                      \
+    X(1, kLayoutDense, true, true, false) X(1, kLayoutRagged, true, true, false)                        \
+    X(1, kLayoutRagged, false, true, false) X(1, kLayoutEigen, true, true, false)                       \
+    X(2, kLayoutDense, true, true, false) X(2, kLayoutRagged, true, true, false)                        \
+    X(2, kLayoutRagged, false, true, false) X(2, kLayoutEigen, true, true, false)                       \
+    X(4, kLayoutDense, true, true, false) X(4, kLayoutRagged, true, true, false)                        \
+    X(4, kLayoutRagged, false, true, false) X(4, kLayoutEigen, true, true, false)
 
 // bayesr_cohort_kernel<R, fp32>: one or two lane runs per slice (a four-run
 // variant gave chains that differ from run to run and stays out)
@@ -38,6 +44,12 @@
 
 #define BRR_SWEEP_INST(R, L, C, A, F) template __global__ void bayesr_sweep_kernel<R, L, C, A, F>(SweepParams);
 #define BRR_SWEEP_DECL(R, L, C, A, F) extern template __global__ void bayesr_sweep_kernel<R, L, C, A, F>(SweepParams);
+#define BRR_PIPE_INST(R, L, F) template __global__ void bayesr_pipe_kernel<R, L, F>(SweepParams);
+#define BRR_PIPE_DECL(R, L, F) extern template __global__ void bayesr_pipe_kernel<R, L, F>(SweepParams);
+#define BRR_GRAM_INST(M) template __global__ void gram_kernel<M>(GramParams); \
+    template __global__ void gram_cohort_kernel<M>(const GramEntry*, uint32_t);
+#define BRR_GRAM_DECL(M) extern template __global__ void gram_kernel<M>(GramParams); \
+    extern template __global__ void gram_cohort_kernel<M>(const GramEntry*, uint32_t);
 #define BRR_COHORT_INST(R, F) template __global__ void bayesr_cohort_kernel<R, F>(CohortTable);
 #define BRR_COHORT_DECL(R, F) extern template __global__ void bayesr_cohort_kernel<R, F>(CohortTable);
 #define BRR_BATCH_INST(NT, D, F) template __global__ void bayesr_batch_kernel<NT, D, F>(BatchParams);

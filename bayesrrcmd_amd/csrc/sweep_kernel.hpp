@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "brr_rng.h"
+#include "mixture.hpp"
 
 namespace brr {
 
@@ -94,6 +95,7 @@ struct SweepParams {
     // dense arena: column j at dense + j * col_words (32-bit words)
     const uint32_t* dense;
     uint64_t col_words, col_bytes;
+    const double* gram;           // pipelined sweep: the Gram rows of the launch's iterations (gram_kernel.hpp)
     const double* lut;            // M x 4, by dosage 0,1,2,missing
     // ragged arena
     const int32_t* ones;
@@ -145,7 +147,7 @@ struct Shared {
     // current block's per-marker constants
     double beta_old[kMaxB];
     double wt[kMaxB][4];                // column value per 2-bit code
-    double mstat[kMaxB][3];             // ragged: mean, sd, Zsum
+    double mstat[kMaxB][4];             // ragged: mean, sd, Zsum, 1 / sd
     double uu[kMaxB];
     uint64_t zw[kMaxB];                // z (bits)
     // chain: the next block's u and z, formed by wave 1 while wave 0 decides
@@ -174,7 +176,7 @@ struct Shared {
     double betasqn[kMaxG];
     double cva[kMaxG * (kMaxK - 1)];
     double gc[kMaxG * kMaxK];           // log pi_k - 0.5 log(logLScale S_k + 1)
-    double gden[kMaxG * kMaxK];         // denom_k (index k >= 1)
+    double grd[kMaxG * kMaxK];          // 1 / denom_k (index k >= 1)
     double gbsd[kMaxG * kMaxK];         // sqrt(sigmaE / denom_k)
     double gdg[kMaxG * kMaxK];          // logL_k - logL_0 = gdg_k + num^2 ghk_k
     double ghk[kMaxG * kMaxK];
@@ -330,6 +332,16 @@ struct IntC {
     static constexpr int value = N;
 };
 
+// f(IntC<kK>, BoolC<exact>) for K mixture components: exact for the usual sizes, else room for kMaxK
+template <class F>
+__device__ __forceinline__ void with_components(int K, F&& f)
+{
+    if (K == 4) f(IntC<4>{}, BoolC<true>{});
+    else if (K == 3) f(IntC<3>{}, BoolC<true>{});
+    else if (K == 2) f(IntC<2>{}, BoolC<true>{});
+    else f(IntC<kMaxK>{}, BoolC<false>{});
+}
+
 // Value of a 2-bit code: two flat selects on 64-bit halves (no control flow).
 __device__ __forceinline__ double wt_of(uint32_t v, double w0, double w1, double w2, double w3)
 {
@@ -379,8 +391,8 @@ __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e)
 // FP32 word and exchanged alongside, so the wave total is hi + lo, accurate to
 // about 2^-48 of the summed magnitudes instead of 2^-24 (Ogita, Rump & Oishi,
 // "Accurate sum and dot product", SIAM J. Sci. Comput. 26, 2005: Sum2).
-template <int kHalf, int kBit>
-__device__ __forceinline__ void transpose_stage_c(float (&hi)[16], float (&lo)[16], int lane)
+template <int kHalf, int kBit, int kN>
+__device__ __forceinline__ void transpose_stage_c(float (&hi)[kN], float (&lo)[kN], int lane)
 {
     const bool up = (lane & kBit) != 0;
 #pragma unroll
@@ -417,6 +429,27 @@ __device__ __forceinline__ double transpose_reduce16_c(float (&v)[16], int lane)
     step(lane_xor<2>(h, lane), lane_xor<2>(l, lane));
     step(lane_xor<1>(h, lane), lane_xor<1>(l, lane));
     return (double)h + (double)l;   // total of value ((lane >> 2) & 15)
+}
+
+__device__ __forceinline__ double transpose_reduce8_c(float (&v)[8], int lane)
+{
+    float lo[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) lo[i] = 0.f;
+    transpose_stage_c<4, 32>(v, lo, lane);
+    transpose_stage_c<2, 16>(v, lo, lane);
+    transpose_stage_c<1, 8>(v, lo, lane);
+    float h = v[0], l = lo[0];
+    auto step = [&](float rh, float rl) {
+        float s, e;
+        two_sum(h, rh, s, e);
+        h = s;
+        l = (l + rl) + e;
+    };
+    step(lane_xor<4>(h, lane), lane_xor<4>(l, lane));
+    step(lane_xor<2>(h, lane), lane_xor<2>(l, lane));
+    step(lane_xor<1>(h, lane), lane_xor<1>(l, lane));
+    return (double)h + (double)l;   // total of value ((lane >> 3) & 7)
 }
 
 // FP32-residual mode: the residual changes applied since the last FP64
@@ -671,11 +704,9 @@ __device__ __forceinline__ bool allreduce_scalar(const SweepParams& p, Shared<R>
 // order (carried across iterations like the reference's xI) takes the
 // libstdc++ random_shuffle rule on its own stream; gamma_f is scalar draw
 // 2 + G + G K + f. epsilonSum is left as is, as in the reference.
-template <int R>
-__device__ __forceinline__ bool fixed_effects(const SweepParams& p, Shared<R>& L, uint32_t& rnd,
-                                              unsigned long long& n_rounds, double (&eps)[R][8],
-                                              uint32_t iteration, uint32_t lo, uint32_t hi, uint32_t w,
-                                              int wave, int lane)
+template <int R, class LDS, class AllReduce>
+__device__ __forceinline__ bool fixed_effects(const SweepParams& p, LDS& L, double (&eps)[R][8], uint32_t iteration,
+                                              uint32_t lo, uint32_t hi, int lane, AllReduce&& allreduce)
 {
     const int tid = threadIdx.x;
     if (tid == 0) {
@@ -709,8 +740,7 @@ __device__ __forceinline__ bool fixed_effects(const SweepParams& p, Shared<R>& L
                 part += xv[r][e] * (eps[r][e] + gamma_old * xv[r][e]);
             }
         double num;
-        if (!allreduce_scalar<R>(p, L, rnd, part, w, wave, lane, &num)) return false;
-        ++n_rounds;
+        if (!allreduce(part, &num)) return false;
         const double denom = dNm1 + sigE_sigF;
         const double g = norm_rng(p.seed, iteration, draw0 + f, p.chain, num / denom, L.sigmaE / denom);
 #pragma unroll
@@ -729,20 +759,20 @@ __device__ __forceinline__ bool fixed_effects(const SweepParams& p, Shared<R>& L
     return true;
 }
 
-template <int R>
-__device__ __forceinline__ void group_constants(const SweepParams& p, Shared<R>& L)
+template <class LDS>
+__device__ __forceinline__ void group_constants(const SweepParams& p, LDS& L)
 {
     // Per-iteration constants of processColumn (BayesRBase.cpp:309-333); they
     // depend only on sigmaE, sigmaG[g], pi[g], S[g].
     const uint32_t K = p.K;
     const double NM1 = (double)(p.N - 1u);
-    for (uint32_t t = threadIdx.x; t < p.G * K; t += kThreads) {
+    for (uint32_t t = threadIdx.x; t < p.G * K; t += blockDim.x) {
         const uint32_t g = t / K, k = t % K;
         const double sigmaG = L.sigmaG[g];
         const double sigmaE = L.sigmaE;
         if (k == 0) {
             L.gc[t] = log(L.pi[t]);
-            L.gden[t] = 0.0;
+            L.grd[t] = 0.0;
             L.gbsd[t] = 0.0;
             L.gdg[t] = 0.0;
             L.ghk[t] = 0.0;
@@ -751,7 +781,7 @@ __device__ __forceinline__ void group_constants(const SweepParams& p, Shared<R>&
             const double sigmaEOverSigmaG = sigmaE / sigmaG;
             const double den = NM1 + sigmaEOverSigmaG * (1.0 / S);
             const double logLScale = sigmaG / sigmaE * NM1;
-            L.gden[t] = den;
+            L.grd[t] = 1.0 / den;
             L.gc[t] = log(L.pi[t]) - 0.5 * log(logLScale * S + 1.0);
             L.gbsd[t] = __dsqrt_rn(sigmaE / den);
             L.gdg[t] = L.gc[t] - log(L.pi[g * K]);
@@ -760,27 +790,50 @@ __device__ __forceinline__ void group_constants(const SweepParams& p, Shared<R>&
     }
 }
 
-// any_{i=1..K-1} |logL[i] - logL[r]| > 700 (BayesRBase.cpp:335, 360); loops run
-// to the array size N >= K with a predicate so the arrays stay in registers
-template <int N>
-__device__ __forceinline__ bool guard700(const double (&logL)[N], int K, double ref)
+// sigmaE, sigmaG and pi draws (BayesRBase.cpp:237-247), the same in every workgroup, and the iteration's history
+// row (all threads). Every draw has its own place in the stream, so they are formed side by side: one thread
+// per gamma of the Dirichlet draws and per variance (one thread after the other took 25 us an iteration).
+template <class LDS>
+__device__ __forceinline__ void scalar_draws(const SweepParams& p, LDS& L, uint32_t iteration, uint32_t it, double e2,
+                                             uint32_t w)
 {
-    bool g = false;
-#pragma unroll
-    for (int i = 1; i < N; ++i)
-        if (i < K) g = g || (fabs(logL[i] - ref) > 700.0);
-    return g;
-}
-
-// 1 / sum_k exp(logL[k] - ref) in index order (BayesRBase.cpp:338, 363)
-template <int N>
-__device__ __forceinline__ double inv_sum_exp(const double (&logL)[N], int K, double ref)
-{
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-        if (k < K) s += exp(logL[k] - ref);
-    return 1.0 / s;
+    const int K = (int)p.K;
+    for (uint32_t t = threadIdx.x; t < p.G * p.K + p.G + 1u; t += blockDim.x) {
+        if (t < p.G * p.K) {
+            L.pi[t] = rgamma(p.seed, iteration, 2u + p.G + t, p.chain, L.v[t] + 1.0, 1.0);
+        } else if (t < p.G * p.K + p.G) {
+            const uint32_t g = t - p.G * p.K;
+            double vsum = 0.0;
+            for (int k = 0; k < K; ++k) vsum += L.v[g * K + k];
+            const double m0 = vsum - L.v[g * K];
+            L.sigmaG[g] = inv_scaled_chisq_rng(p.seed, iteration, kDrawSigmaG0 + g, p.chain, p.v0G + m0,
+                                               (L.betasqn[g] * m0 + p.v0G * p.s02G) / (p.v0G + m0));
+        } else {
+            L.sigmaE = inv_scaled_chisq_rng(p.seed, iteration, kDrawSigmaE, p.chain, p.v0E + p.N,
+                                            (e2 + p.v0E * p.s02E) / (p.v0E + p.N));
+        }
+    }
+    __syncthreads();
+    for (uint32_t g = threadIdx.x; g < p.G; g += blockDim.x) {
+        double sum = 0.0;
+        for (int k = 0; k < K; ++k) sum += L.pi[g * K + k];
+        for (int k = 0; k < K; ++k) L.pi[g * K + k] = L.pi[g * K + k] / sum;
+    }
+    if (w == 0 && threadIdx.x == 0 && p.hist) {
+        double m0 = 0.0;
+        for (uint32_t g = 0; g < p.G; ++g) {
+            double vsum = 0.0;
+            for (int k = 0; k < K; ++k) vsum += L.v[g * K + k];
+            m0 += vsum - L.v[g * K];
+        }
+        double* h = p.hist + (size_t)it * (4u + p.G);
+        h[0] = L.mu;
+        h[1] = L.sigmaE;
+        h[2] = m0;
+        h[3] = e2;
+        for (uint32_t g = 0; g < p.G; ++g) h[4 + g] = L.sigmaG[g];
+    }
+    __syncthreads();
 }
 
 // ------------------------------------------------------------ block loading --
@@ -797,7 +850,8 @@ struct MetaNext {
 };
 
 // A marker's u and z in a chain (as marker_uz).
-__device__ __forceinline__ void chain_draws(const SweepParams& p, uint32_t j, uint32_t iteration, double& u,
+template <class Params>
+__device__ __forceinline__ void chain_draws(const Params& p, uint32_t j, uint32_t iteration, double& u,
                                             uint64_t& zw)
 {
     const U4 x = draw_block(p.seed, j, iteration, kStreamMarker, p.chain);
@@ -869,6 +923,7 @@ __device__ __forceinline__ void meta_store(const SweepParams& p, Shared<R>& L, i
         L.mstat[t][0] = m.w0;
         L.mstat[t][1] = m.w1;
         L.mstat[t][2] = m.w2;
+        L.mstat[t][3] = 1.0 / m.w1;
         L.wt[t][0] = 2.0;   // genotype 2
         // missing: absent from the ragged dot, at the marker mean in EigenBayesRKernel's
         L.wt[t][1] = (kLay == kLayoutEigen) ? m.w0 : 0.0;
@@ -1249,6 +1304,11 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
         return;
     }
 
+    auto reduce = [&](double part, double* total) -> bool {
+        if (!allreduce_scalar<R>(p, L, rnd, part, w, wave, lane, total)) return false;
+        ++n_rounds;
+        return true;
+    };
     const uint32_t iters = (p.mode == kModeChain) ? p.iterations : 1u;
     const uint32_t nblocks = (p.M + p.B - 1) / p.B;
     for (uint32_t it = 0; it < iters; ++it) {
@@ -1256,7 +1316,7 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
         const uint32_t* order = p.order + (size_t)((p.mode == kModeChain) ? it : 0u) * p.M;
         if (p.mode == kModeFixed) {
             if (!fp64_region([&](double (&ed)[R][8]) {
-                    return fixed_effects<R>(p, L, rnd, n_rounds, ed, iteration, lo, hi, w, wave, lane);
+                    return fixed_effects<R>(p, L, ed, iteration, lo, hi, lane, reduce);
                 }))
                 goto done;
             break;
@@ -1311,7 +1371,7 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
             for (uint32_t t = tid; t < p.G * p.K; t += kThreads) L.v[t] = 0.0;
             __syncthreads();
         }
-        group_constants<R>(p, L);
+        group_constants(p, L);
         __syncthreads();
 
         // ---- block 0 of this iteration, loaded in place; the ids (and for
@@ -1508,103 +1568,31 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
                         bool changed = false;
                         double bnew = 0.0, acum0 = 0.0, ed = 0.0, numk = 0.0;
                         int sel = -1, g = 0;
-                        // the decision, with its per-component loops unrolled to 4 components
-                        // when K <= 4 (the usual mixture) and to kMaxK otherwise
-                        auto decide = [&](auto kc) {
+                        auto decide = [&](auto kc, auto exact) {
                             constexpr int kK = decltype(kc)::value;
                             g = L.gr[k];
-                            const double* gc = L.gc + g * K;
-                            const double* gden = L.gden + g * K;
-                            const double* gbsd = L.gbsd + g * K;
                             const double beta_old = L.beta_old[k];
                             const double dotk = pass ? L.dot[k] + dcorr * L.gram[k] : L.dot[k];
                             double num;
                             if (dense) {
                                 num = dotk + beta_old * NM1;
                             } else {
-                                const double mean = L.mstat[k][0], sd = L.mstat[k][1];
-                                num = beta_old * (dN - 1.0) - mean * eS / sd + dotk / sd;
+                                const double mean = L.mstat[k][0], rsd = L.mstat[k][3];
+                                num = beta_old * (dN - 1.0) - mean * eS * rsd + dotk * rsd;
                             }
                             numk = num;
-                            // d_c = logL_c - logL_0 = gdg_c + num^2 ghk_c. While every |d_c| <= 350
-                            // no 700 guard can fire and no exponential overflows, and the
-                            // probability terms 1 / sum_i exp(logL_i - logL_c) equal
-                            // exp(d_c) / sum_i exp(d_i): one set of K - 1 exponentials.
-                            // Otherwise the reference's own formulation, guards included.
-                            const double n2 = num * num;
-                            double dd[kK];
-                            dd[0] = 0.0;
-                            bool far = false;
-#pragma unroll
-                            for (int c = 1; c < kK; ++c) {
-                                dd[c] = 0.0;
-                                if (c < K) {
-                                    dd[c] = L.gdg[g * K + c] + n2 * L.ghk[g * K + c];
-                                    far = far || fabs(dd[c]) > 350.0;
-                                }
-                            }
-                            const double uu = L.uu[k];
-                            if (!far) {
-                                double ee[kK];
-                                double esum = 1.0;
-                                ee[0] = 1.0;
-#pragma unroll
-                                for (int c = 1; c < kK; ++c) {
-                                    ee[c] = 0.0;
-                                    if (c < K) {
-                                        ee[c] = exp(dd[c]);
-                                        esum += ee[c];
-                                    }
-                                }
-                                const double inv = 1.0 / esum;
-                                double acum = inv;
-                                acum0 = acum;
-#pragma unroll
-                                for (int c = 0; c < kK; ++c) {
-                                    if (c < K && sel < 0) {
-                                        if (uu <= acum) sel = c;
-                                        else if (c + 1 < K) acum += ee[c + 1 < kK ? c + 1 : 0] * inv;
-                                    }
-                                }
-                            } else {
-                                double logL[kK], muk[kK];
-                                logL[0] = gc[0];
-                                muk[0] = 0.0;
-#pragma unroll
-                                for (int c = 1; c < kK; ++c) {
-                                    muk[c] = 0.0;
-                                    logL[c] = 0.0;
-                                    if (c < K) {
-                                        muk[c] = num / gden[c];
-                                        logL[c] = gc[c] + 0.5 * (muk[c] * num) / L.sigmaE;
-                                    }
-                                }
-                                double acum = guard700(logL, K, logL[0]) ? 0.0 : inv_sum_exp(logL, K, logL[0]);
-                                acum0 = acum;
-#pragma unroll
-                                for (int c = 0; c < kK; ++c) {
-                                    if (c < K && sel < 0) {
-                                        if (uu <= acum) {
-                                            sel = c;
-                                        } else if (c + 1 < K) {
-                                            const double ref = logL[c + 1 < kK ? c + 1 : 0];
-                                            if (!guard700(logL, K, ref)) acum += inv_sum_exp(logL, K, ref);
-                                        }
-                                    }
-                                }
-                            }
+                            const MixDraw md = mix_draw<kK, decltype(exact)::value>(
+                                K, num * num, L.uu[k], [&](int c) { return L.gdg[g * K + c]; },
+                                [&](int c) { return L.ghk[g * K + c]; }, [&](int c) { return L.gc[g * K + c]; });
+                            sel = md.sel;
+                            acum0 = md.acum0();
                             // the beta draw of the chosen component (BayesRBase.cpp:343-352)
                             bnew = beta_old;
                             if (sel == 0) bnew = 0.0;
-                            else if (sel > 0) {
-                                bnew = bits_as_double(L.zw[k]) * gbsd[sel] + num / gden[sel];
-                            }
+                            else if (sel > 0) bnew = bits_as_double(L.zw[k]) * L.gbsd[g * K + sel] + num * L.grd[g * K + sel];
                             changed = (bnew != beta_old);
                         };
-                        if (act) {
-                            if (K <= 4) decide(IntC<4>{});
-                            else decide(IntC<kMaxK>{});
-                        }
+                        if (act) with_components(K, decide);
                         const unsigned long long cm = __ballot(changed);
                         // sequential sweep: the first change ends the pass; asynchronous
                         // window (pos = 0): every slot decides on the window-start residual
@@ -1793,8 +1781,7 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
             double e2 = 0.0;
             const bool ok = fp64_region([&](double (&ed)[R][8]) {
                 // ---- fixed effects (BayesRBase.cpp:212-235)
-                if (p.F && !fixed_effects<R>(p, L, rnd, n_rounds, ed, iteration, lo, hi, w, wave, lane))
-                    return false;
+                if (p.F && !fixed_effects<R>(p, L, ed, iteration, lo, hi, lane, reduce)) return false;
                 // ---- |eps|^2 of the sigmaE draw
                 double part = 0.0;
 #pragma unroll
@@ -1806,37 +1793,7 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
                 return true;
             });
             if (!ok) goto done;
-            // ---- sigmaE, sigmaG, pi draws (BayesRBase.cpp:237-247)
-            if (tid == 0) {
-                L.sigmaE = inv_scaled_chisq_rng(p.seed, iteration, kDrawSigmaE, p.chain, p.v0E + p.N,
-                                                (e2 + p.v0E * p.s02E) / (p.v0E + p.N));
-                double m0_total = 0.0;
-                for (uint32_t g = 0; g < p.G; ++g) {
-                    double vsum = 0.0;
-                    for (int k = 0; k < K; ++k) vsum += L.v[g * K + k];
-                    const double m0 = vsum - L.v[g * K];
-                    m0_total += m0;
-                    L.sigmaG[g] = inv_scaled_chisq_rng(p.seed, iteration, kDrawSigmaG0 + g, p.chain,
-                                                       p.v0G + m0,
-                                                       (L.betasqn[g] * m0 + p.v0G * p.s02G) / (p.v0G + m0));
-                    double gs[kMaxK];
-                    double sum = 0.0;
-                    for (int k = 0; k < K; ++k)
-                        gs[k] = rgamma(p.seed, iteration, 2u + p.G + g * (uint32_t)K + (uint32_t)k,
-                                       p.chain, L.v[g * K + k] + 1.0, 1.0);
-                    for (int k = 0; k < K; ++k) sum += gs[k];
-                    for (int k = 0; k < K; ++k) L.pi[g * K + k] = gs[k] / sum;
-                }
-                if (w == 0 && p.hist) {
-                    double* h = p.hist + (size_t)it * (4u + p.G);
-                    h[0] = L.mu;
-                    h[1] = L.sigmaE;
-                    h[2] = m0_total;
-                    h[3] = e2;
-                    for (uint32_t g = 0; g < p.G; ++g) h[4 + g] = L.sigmaG[g];
-                }
-            }
-            __syncthreads();
+            scalar_draws(p, L, iteration, it, e2, w);
             BRR_TICK(5);
         }
     }
@@ -1888,38 +1845,6 @@ bayesr_sweep_kernel(SweepParams p)
     __shared__ Shared<R> L;
     __shared__ RefreshLog<kF32, R> RL;
     sweep_body<R, kLay, kCodes, kAsync, kF32>(p, L, RL, blockIdx.x);
-}
-
-// ------------------------------------------------------- cohorts in one launch --
-
-// Independent single-chain contexts (cohorts of uneven N and M) in one
-// persistent cooperative launch: cohort c owns workgroups [first[c], first[c+1])
-// and runs its own context's sweep or chain on them -- its own slices,
-// exchange words, state and counters -- so small cohorts, whose rounds cost as
-// much as a large one's, run side by side instead of one after another. Every
-// cohort of a launch has the same lane runs R and residual precision; the
-// layout (dense / ragged / EigenSparse formulas over 2-bit codes) is per cohort.
-constexpr int kMaxCohorts = 64;
-
-struct CohortTable {
-    const SweepParams* params;          // device array, one per cohort
-    uint32_t n;
-    uint32_t first[kMaxCohorts + 1];    // first workgroup of each cohort; first[n] = grid size
-};
-
-template <int R, bool kF32>
-__global__ void __launch_bounds__(kThreads)
-bayesr_cohort_kernel(CohortTable t)
-{
-    __shared__ Shared<R> L;
-    __shared__ RefreshLog<kF32, R> RL;
-    uint32_t c = 0;
-    while (c + 1 < t.n && blockIdx.x >= t.first[c + 1]) ++c;
-    const SweepParams p = t.params[c];
-    const uint32_t w = blockIdx.x - t.first[c];
-    if (p.layout == kLayoutDense) sweep_body<R, kLayoutDense, true, false, kF32>(p, L, RL, w);
-    else if (p.layout == kLayoutEigen) sweep_body<R, kLayoutEigen, true, false, kF32>(p, L, RL, w);
-    else sweep_body<R, kLayoutRagged, true, false, kF32>(p, L, RL, w);
 }
 
 } // namespace brr
