@@ -27,8 +27,10 @@ namespace brr {
 constexpr int kDotWaves = 8;
 constexpr int kDecWave = 8;
 constexpr int kRedWave = 9;
+constexpr int kLoadWave = 10;
+constexpr int kMetaWave = 11;
 constexpr int kDotThreads = 64 * kDotWaves;
-constexpr int kPipeThreads = kDotThreads + 128;
+constexpr int kPipeThreads = kDotThreads + 256;
 constexpr int kSlotsPerWave = kMaxB / kDotWaves;
 constexpr int kRing = 4;                 // blocks of columns and constants held at once
 constexpr uint32_t kDirectP = 16;        // workgroups up to which the partials are summed without a reduce hop
@@ -81,6 +83,7 @@ struct PipeShared {
     PipeMeta meta[kRing];
     uint32_t ids[kRing][kMaxB];
     double du[2][kMaxB], dz[2][kMaxB];         // chain draws, by block parity
+    double tots[2][kMaxB];                     // a block's totals gathered ahead, by parity
     // a block's decisions, by parity
     double ob[2][kMaxB], oa[2][kMaxB], on[2][kMaxB];
     int os[2][kMaxB];
@@ -98,6 +101,7 @@ struct PipeShared {
     uint32_t forder[kMaxF];
     double sigmaF;
     int decided;                               // last block decided
+    int got[2];                                // the block whose totals `tots` holds
     int abort;
 };
 
@@ -115,7 +119,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
     constexpr int kRows = gram_rows<R, kLay>();
     if (p.gate && __hip_atomic_load(p.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lo = w * p.S;
     const uint32_t hi = min(lo + p.S, p.N);
@@ -123,7 +127,6 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
     const int K = (int)p.K;
     const ScalarLayout SL{p.G, p.K};
     const double dN = (double)p.N;
-    const double NM1 = (double)(p.N - 1u);
     const bool direct = P <= kDirectP;
     const uint32_t copy = w % kCopies;
 
@@ -144,7 +147,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
         }
     }
 
-    // body(ed) on the FP64 slice ed[R][8], between iterations (all waves; waves 8 and 9 hold no current slice
+    // body(ed) on the FP64 slice ed[R][8], between iterations (all waves; waves 8 to 11 hold no current slice
     // and store nothing)
     auto fp64_region = [&](auto&& body) -> bool {
         if constexpr (!kF32) {
@@ -223,72 +226,87 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
     // r + 2 only after deciding round r, whose totals show that every partial of it has been read. Without the
     // reduce hop (direct) it only knows that they were written: a workgroup may publish round r + 3 while another
     // still reads round r, so four buffers take turns.
-    // They are laid out by workgroup then, so that a wave's reads of 64 slots are contiguous.
-    auto part_slot = [&](uint32_t r, int k, uint32_t w2) {
-        return q->xchg1 + 2u * (direct ? ((size_t)(r & 3u) * P + w2) * kMaxB + (size_t)k
-                                        : ((size_t)(r & 1u) * kSlots + (size_t)k) * P + w2);
+    // Laid out so that a publishing wave writes whole sectors and a reading wave reads them: direct, by workgroup;
+    // else by groups of 2 slots (4 with less than 32 workgroups), which one workgroup reduces, and by workgroup
+    // within the group.
+    const uint32_t gl = direct ? 6u : P >= 32 ? 1u : 2u;   // log2 of the slots in a group
+    auto part_slot = [&](uint32_t r, uint32_t k, uint32_t w2) {
+        const uint32_t buf = direct ? r & 3u : (r & 1u) * ((uint32_t)kMaxB >> gl);
+        return q->xchg1 + 2u * ((((size_t)(buf + (k >> gl)) * P + w2) << gl) + (k & ((1u << gl) - 1u)));
     };
-    auto tot_slot = [&](uint32_t r, int k, uint32_t c) {
+    auto tot_slot = [&](uint32_t r, uint32_t k, uint32_t c) {
         return q->xchg2 + c * kCopyWords + (((size_t)(r & 1u) * kSlots + (size_t)k) * 2u);
     };
-    // Wave 9: the slots of [0, nb) with k % P == w, reduced in a fixed order and published: one slot by all lanes,
-    // or (P < 64) up to four at once, 16 lanes each. `leave()` ends the wait (for a round that need not be reduced
-    // yet). 1: done, 0: left, -1: abort or timeout.
-    auto reduce_round = [&](uint32_t r, int nb, auto&& leave) -> int {
-        if (direct) return 1;
-        const bool wide = P >= 64;
-        const int k = wide ? (int)w : (int)(w + P * (uint32_t)(lane >> 4));
-        const uint32_t first = wide ? (uint32_t)lane : (uint32_t)(lane & 15), stride = wide ? 64u : 16u;
-        const bool act = k < nb;
-        if (!__any(act)) return 1;
-        uint64_t h[4] = {0, 0, 0, 0}, l[4] = {0, 0, 0, 0};
-        uint32_t live = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (act && first + stride * i < P) live |= 1u << i;
-        uint32_t stale = live;
+    // The sum of the lane's words at offsets at, at + step, .. (n of them, at most kN; cnt is the largest n of a
+    // lane) once all carry tag r. A lane without words reads the one at `at` and does not wait. All loads are in
+    // flight at once: their addresses come from one register, as each address kept and spilled for itself is a
+    // wait for the loads before it. `leave()` ends the wait (for a round that is not needed yet).
+    // 1: done, 0: left, -1: abort or timeout.
+    auto wait_words = [&](auto kn, const uint64_t* base, uint32_t at, uint32_t step, uint32_t n, uint32_t cnt, uint32_t r,
+                          auto&& leave, double* acc) -> int {
+        constexpr uint32_t kN = decltype(kn)::value;
+        const auto buf = xbuf(base);
+        const uint32_t last = at + (n ? n - 1u : 0u) * step;
+        u32x4 x[kN];
         for (uint64_t spins = 0;; ++spins) {
+            uint32_t from = at;
+            asm volatile("" : "+v"(from));   // opaque offset: every poll issues fresh loads
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if ((stale >> i) & 1u) ld_pair(q->xchg1, part_slot(r, k, first + stride * i), h[i], l[i]);
-            stale = 0;
+            for (uint32_t i = 0; i < kN; ++i)
+                if (i < cnt) x[i] = __builtin_amdgcn_raw_buffer_load_b128(buf, min(from + i * step, last), 0, kCpolDevice);
+            bool stale = false;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (((live >> i) & 1u) && ((uint32_t)(h[i] >> 32) != r || (uint32_t)(l[i] >> 32) != r)) stale |= 1u << i;
-            if (!__any(stale != 0)) break;
+            for (uint32_t i = 0; i < kN; ++i)
+                if (i < cnt) stale |= x[i].y != r || x[i].w != r;
+            if (!__any(stale && n != 0u)) break;
             if (leave()) return 0;
             if (spins > kSpinLimit || ((spins & 255u) == 255u &&
                                        __hip_atomic_load(q->ctl + kCtlAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
                 return -1;
         }
-        double acc = 0.0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if ((live >> i) & 1u) acc += bits_as_double((h[i] << 32) | (l[i] & 0xFFFFFFFFull));
-        if (wide) {
-            acc += lane_xor<32>(acc, lane);
-            acc += lane_xor<16>(acc, lane);
-        }
+        for (uint32_t i = 0; i < kN; ++i)
+            if (i < n) *acc += bits_as_double(((uint64_t)x[i].x << 32) | x[i].z);
+        return 1;
+    };
+    // Wave 9 of the workgroups that own a group: its slots of [0, nb), reduced in a fixed order and published.
+    auto reduce_round = [&](uint32_t r, int nb, auto&& leave) -> int {
+        if (direct || (int)(w << gl) >= nb) return 1;
+        const uint32_t k = (w << gl) + ((uint32_t)lane & ((1u << gl) - 1u));
+        const uint32_t first = (uint32_t)lane >> gl, stride = 64u >> gl;
+        constexpr uint32_t kN = 8;
+        static_assert(kN * 32 >= kMaxP, "two slots over 64 lanes");
+        double acc = 0.0;
+        const int st = wait_words(std::integral_constant<uint32_t, kN>(), q->xchg1,
+                                  (uint32_t)((const char*)part_slot(r, k, min(first, P - 1u)) - (const char*)q->xchg1),
+                                  16u * 64u, (int)k < nb && first < P ? (P - first + stride - 1u) / stride : 0u,
+                                  (P + stride - 1u) / stride, r, leave, &acc);
+        if (st != 1) return st;
+        acc += lane_xor<32>(acc, lane);
+        acc += lane_xor<16>(acc, lane);
         acc += lane_xor<8>(acc, lane);
         acc += lane_xor<4>(acc, lane);
-        acc += lane_xor<2>(acc, lane);
-        acc += lane_xor<1>(acc, lane);
-        const uint32_t cp = first;
-        if (act && cp < (uint32_t)kCopies) publish_pair(q->xchg2, tot_slot(r, k, cp), r, acc);
+        if (gl == 1) acc += lane_xor<2>(acc, lane);
+        if ((int)k < nb && first < (uint32_t)kCopies) publish_pair(q->xchg2, tot_slot(r, k, first), r, acc);
         return 1;
     };
     auto never = [] { return false; };
-    // Wave 8: slot k's total in lane k < nb.
-    auto gather_round = [&](uint32_t r, int nb, double* out) -> bool {
-        bool ok = true;
+    // Slot k's total in lane k < nb.
+    auto gather_round = [&](uint32_t r, int nb, double* out, auto&& leave) -> int {
         *out = 0.0;
-        if (direct)
-            for (uint32_t w0 = 0; ok && w0 < P; w0 += 8)
-                ok = wait_sum_strided<8>(q->xchg1, [&](uint32_t w2) { return part_slot(r, lane, w2); }, w0, 1u,
-                                         lane < nb ? P : 0u, r, q->ctl, out);
-        else if (lane < nb)
-            ok = wait_pair(q->xchg2, tot_slot(r, lane, copy), r, q->ctl, out);
-        return !__any(!ok);
+        const bool act = lane < nb;
+        if (!direct)
+            return wait_words(std::integral_constant<uint32_t, 1>(), q->xchg2,
+                              (uint32_t)((const char*)tot_slot(r, (uint32_t)lane, copy) - (const char*)q->xchg2), 0u,
+                              act ? 1u : 0u, 1u, r, leave, out);
+        int st = 1;
+        for (uint32_t w0 = 0; st == 1 && w0 < P; w0 += 8) {
+            const uint32_t n = min(P - w0, 8u);
+            st = wait_words(std::integral_constant<uint32_t, 8>(), q->xchg1,
+                            (uint32_t)((const char*)part_slot(r, (uint32_t)lane, w0) - (const char*)q->xchg1), 16u * kMaxB,
+                            act ? n : 0u, n, r, leave, out);
+        }
+        return st;
     };
     // A scalar all-reduce of wave 0's slice sum (all threads call it).
     auto allreduce = [&](double part, double* total) -> bool {
@@ -299,7 +317,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
         if (wave == kRedWave && reduce_round(rnd, 1, never) < 0 && lane == 0) { L.abort = 1; raise_abort(*q, 1); }
         if (wave == kDecWave) {
             double x;
-            if (!gather_round(rnd, 1, &x)) {
+            if (gather_round(rnd, 1, &x, never) < 0) {
                 if (lane == 0) { L.abort = 1; raise_abort(*q, 2); }
             } else if (lane == 0) {
                 L.tot = x;
@@ -323,8 +341,8 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                 if ((lane & 7) == 0 && k < nb) publish_pair(p.xchg1, part_slot(rnd, k, w), rnd, 0.0);
             } else if (wave == kDecWave) {
                 double x;
-                if (!gather_round(rnd, nb, &x) && lane == 0) { L.abort = 1; raise_abort(p, 2); }
-            } else if (reduce_round(rnd, nb, never) < 0 && lane == 0) {
+                if (gather_round(rnd, nb, &x, never) < 0 && lane == 0) { L.abort = 1; raise_abort(p, 2); }
+            } else if (wave == kRedWave && reduce_round(rnd, nb, never) < 0 && lane == 0) {
                 L.abort = 1;
                 raise_abort(p, 1);
             }
@@ -389,13 +407,13 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
         }
         group_constants(p, L);
         if (tid < count(0)) L.ids[0][tid] = order[tid];
-        if (tid == 0) L.decided = -1;
+        if (tid == 0) L.decided = L.got[0] = L.got[1] = -1;
         __syncthreads();
 
         double eS = L.epsSum;        // wave 8: epsilonSum
         double xc = 0.0;             // wave 8: correction of the next block's dot in this lane
         const uint32_t rnd0 = rnd + 1;   // block b's exchange round is rnd0 + b
-        // the outputs of block b and its counts (wave 6, lane = slot)
+        // the outputs of block b and its counts (wave 11, lane = slot)
         auto outputs = [&](int b) {
             const int nb = count(b), par = b & 1;
             const PipeMeta& m = L.meta[b & (kRing - 1)];
@@ -487,12 +505,14 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                     rd[c] = L.grd[at];
                 }
             }
-            const double base = bo * NM1;
+            const double base = bo * (double)(q->N - 1u);
             // epsilonSum's change per unit of beta (sparsebayesrkernel.cpp:29-34)
-            const double dS = dense ? 0.0 : w2 * w3 - w0 * dN * w3;
+            const double dS = dense ? 0.0 : w2 * w3 - w0 * (double)q->N * w3;
             const unsigned long long im = __ballot(bo != 0.0);
             double dot;
-            if (!gather_round(rnd0 + (uint32_t)b, nb, &dot)) {
+            if (__builtin_amdgcn_readfirstlane(L.got[par]) == b) {
+                dot = L.tots[par][lane];
+            } else if (gather_round(rnd0 + (uint32_t)b, nb, &dot, never) < 0) {
                 if (lane == 0) { L.abort = 1; raise_abort(*q, 2); }
                 return;
             }
@@ -585,88 +605,23 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
         tick(5);
         // ---- the sweep (AnalysisGraph::exec over the order). Step b decides block b; steps -2 and -1 fill
         // the pipeline.
+        if (wave >= kDotWaves) {
+            // these waves hold no slice from here on: none of its registers is kept over their loops
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) eps[r][e] = 0;
+                if constexpr (kF32) e64[r] = 0.0;
+            }
+        }
         if (wave < kDotWaves) {
             int due = (int)q->refresh_blocks;   // blocks until the FP32 slice is re-rounded
             bool fresh = false;
             for (int b = -2; b < nblocks; ++b) {
-                asm volatile("" : "+s"(q));
-                const int b1 = b + 1, b2 = b + 2, b3 = b + 3;
-                const int nb1 = count(b1), nb2 = count(b2);
-                // loads: columns of block b + 2 and Gram rows of block b + 1 straight into LDS, constants of block
-                // b + 2 and ids of block b + 3 through registers
-                // (columns: word 512 i + tid of the flattened [slot][R][32] array; a word past the column's end
-                // is its last word, of individuals that hold no residual; a slot past the block is column 0)
-                constexpr int kW = 4 * R;
-                constexpr uint32_t per = (uint32_t)R * 32u, kStep = kDotThreads / per;
-                if (nb2 > 0) {
-                    const uint32_t* ids = L.ids[b2 & (kRing - 1)];
-                    const uint32_t at = min((lo >> 4) + (uint32_t)tid % per, (uint32_t)q->col_words - 1u);
-                    uint32_t* dst = &L.codes[b2 & (kRing - 1)][0][0][0] + 64 * wave;
-#pragma unroll
-                    for (int i = 0; i < kW; ++i) {
-                        const uint32_t k = (uint32_t)tid / per + (uint32_t)i * kStep;
-                        const uint32_t j = k < (uint32_t)nb2 ? ids[k] : 0u;
-                        load_to_lds<4>(q->dense + (size_t)j * q->col_words + at, dst + i * kDotThreads);
-                    }
-                }
-                double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
-                if constexpr (kLay != kLayoutRagged) {
-                    // the values of slot tid / 8's pair table entries
-                    const uint32_t k = (uint32_t)tid >> 3;
-                    const uint32_t j = k < (uint32_t)nb2 ? L.ids[b2 & (kRing - 1)][k] : 0u;
-                    if constexpr (dense) {
-                        const double* lt = q->lut + 4 * (size_t)j;
-                        t0 = lt[2];
-                        t1 = lt[3];
-                        t2 = lt[1];
-                        t3 = lt[0];
-                    } else {
-                        t0 = 2.0;
-                        t1 = q->stats[4 * (size_t)j];   // EigenBayesRKernel: missing calls at the mean
-                        t2 = 1.0;
-                    }
-                }
-                if (nb1 > 0) {
-                    // row i of the in-model slots by wave i mod 8
-                    const PipeMeta& m = L.meta[b1 & (kRing - 1)];
-                    const bool in = lane < nb1 && m.bo[lane < nb1 ? lane : 0] != 0.0;
-                    unsigned long long im = __ballot(in);
-                    const int have = min((int)__popcll(im), kRows);
-                    for (int i = 0; i < have; ++i, im &= im - 1) {
-                        if ((i & (kDotWaves - 1)) != wave) continue;
-                        const int h = (int)__ffsll((long long)im) - 1;
-                        load_to_lds<16>(gram + ((size_t)b1 * B + (size_t)h) * kGramCols + 2 * lane, &L.rows[b1 & 1][i][0]);
-                    }
-                }
-                PipeMeta* const ms = &L.meta[b2 & (kRing - 1)];
-                uint32_t mj = 0;
-                int32_t mg = 0;
-                uint64_t mbo = 0;
-                double m0 = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0, mu_ = 0.0, mz = 0.0;
-                uint32_t nid = 0;
-                if (wave == 7) {
-                    mj = lane < nb2 ? L.ids[b2 & (kRing - 1)][lane] : 0u;
-                    mbo = ld_agent((const uint64_t*)(q->beta + mj));
-                    mg = q->group ? q->group[mj] : 0;
-                    mu_ = q->u[mj];
-                    mz = q->z[mj];
-                    if constexpr (dense) {
-                        const double* lt = q->lut + 4 * (size_t)mj;
-                        m0 = lt[2];
-                        m1 = lt[3];
-                        m2 = lt[1];
-                        m3 = lt[0];
-                    } else {
-                        const double* st = q->stats + 4 * (size_t)mj;
-                        m0 = st[0];
-                        m1 = st[1];
-                        m2 = st[3];
-                    }
-                } else if (wave == 5) {
-                    nid = order[min((uint32_t)b3 * B + (uint32_t)lane, M - 1u)];
-                }
+                asm volatile("" : "+s"(q), "+v"(lane));
+                const int nb1 = count(b + 1);
+                const int b1 = b + 1;
                 if (wave == 0) tick(0);
-
                 if (b >= 1) {
                     if constexpr (kF32) {
                         // the slice re-rounded from the FP64 residual in the step before
@@ -730,70 +685,41 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                         publish_pair(q->xchg1, part_slot(rnd0 + (uint32_t)b1, k, w), rnd0 + (uint32_t)b1, tot);
                 }
                 if (wave == 0) tick(1);
-                if (wave == 6 && b >= 1) outputs(b - 1);
-
-                // ---- the loads into LDS
-                if (nb2 > 0) {
-                    if constexpr (kLay != kLayoutRagged) {
-                        const int k = tid >> 3;
-                        if (k < nb2)
-#pragma unroll
-                            for (int i = 0; i < 2; ++i) {
-                                const uint32_t n = 2u * (uint32_t)(tid & 7) + (uint32_t)i;
-                                L.pt[b2 & 1][k][n][0] = (E)wt_of(n & 3u, t0, t1, t2, t3);
-                                L.pt[b2 & 1][k][n][1] = (E)wt_of(n >> 2, t0, t1, t2, t3);
-                            }
-                    }
-                    if (wave == 7 && lane < nb2) {
-                        ms->mk[lane] = mj;
-                        ms->gr[lane] = mg;
-                        ms->bo[lane] = bits_as_double(mbo);
-                        ms->w[lane][0] = m0;
-                        ms->w[lane][1] = m1;
-                        ms->w[lane][2] = m2;
-                        ms->w[lane][3] = dense ? m3 : 1.0 / m1;
-                        ms->u[lane] = mu_;
-                        ms->z[lane] = mz;
-                    }
-                }
-                if (wave == 5 && lane < count(b3)) L.ids[b3 & (kRing - 1)][lane] = nid;
-                // the loads into LDS are done; a publish after them may be on its way
-                if (kSlotsPerWave * wave < nb1 && wave != 6) wait_vm<1>();
-                else wait_vm<0>();
                 __syncthreads();
                 if (L.abort) goto done;
             }
         } else if (wave == kDecWave) {
+            __builtin_amdgcn_s_setprio(3);
             __syncthreads();
             __syncthreads();
             for (int b = 0; b < nblocks; ++b) {
-                asm volatile("" : "+s"(q));
+                asm volatile("" : "+s"(q), "+v"(lane));
                 t_last = w == 0 ? __builtin_amdgcn_s_memrealtime() : 0;
                 with_components(K, [&](auto kc, auto exact) { decide(b, kc, exact); });
                 if (lane == 0) L.decided = b;
                 __syncthreads();
                 if (L.abort) goto done;
             }
-        } else {
+        } else if (wave == kRedWave) {
+            __builtin_amdgcn_s_setprio(2);
             bool reduced = true;             // block b's slots were reduced in the step before
             for (int b = -2; b < nblocks; ++b) {
-                asm volatile("" : "+s"(q));
-                const int b1 = b + 1;
+                asm volatile("" : "+s"(q), "+v"(lane));
+                const int b1 = b + 1, nb1 = count(b1);
                 int st = 1;
                 if (!reduced) st = reduce_round(rnd0 + (uint32_t)b, count(b), never);
-                if (q->mode == kModeChain && lane < count(b1)) {
-                    double u;
-                    uint64_t zw;
-                    chain_draws(*q, L.ids[b1 & (kRing - 1)][lane], iteration, u, zw);
-                    L.du[b1 & 1][lane] = u;
-                    L.dz[b1 & 1][lane] = bits_as_double(zw);
-                }
-                reduced = b1 < 0;
-                if (st > 0 && b >= 0 && b1 < nblocks) {
-                    // block b + 1's slots already in this step if their partials arrive before block b is decided
+                reduced = true;
+                if (st > 0 && b1 >= 0 && nb1 > 0) {
+                    // block b + 1 already in this step, as far as its words arrive before block b is decided
                     const volatile int* dec = &L.decided;
-                    st = reduce_round(rnd0 + (uint32_t)b1, count(b1), [&] { return *dec >= b; });
+                    auto leave = [&] { return *dec >= b; };
+                    st = reduce_round(rnd0 + (uint32_t)b1, nb1, leave);
                     reduced = st == 1;
+                    double x;
+                    if (st == 1 && b >= 0 && (st = gather_round(rnd0 + (uint32_t)b1, nb1, &x, leave)) == 1) {
+                        L.tots[b1 & 1][lane] = x;
+                        if (lane == 0) L.got[b1 & 1] = b1;
+                    }
                 }
                 if (st < 0 && lane == 0) {
                     L.abort = 1;
@@ -802,12 +728,114 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                 __syncthreads();
                 if (L.abort) goto done;
             }
+        } else if (wave == kLoadWave) {
+            __builtin_amdgcn_s_setprio(2);
+            for (int b = -2; b < nblocks; ++b) {
+                asm volatile("" : "+s"(q), "+v"(lane));
+                const int b1 = b + 1, b2 = b + 2;
+                const int nb1 = count(b1), nb2 = count(b2);
+                // columns of block b + 2, the flattened [slot][R][32] words: four to a lane where slices start on 16
+                // bytes of their columns. A load past the column's end is of its last words, of individuals that
+                // hold no residual; a slot past the block is column 0.
+                if (nb2 > 0) {
+                    const uint32_t* ids = L.ids[b2 & (kRing - 1)];
+                    uint32_t* dst = &L.codes[b2 & (kRing - 1)][0][0][0];
+                    auto columns = [&](auto wc) {
+                        constexpr uint32_t kWords = decltype(wc)::value, per = (uint32_t)R * 32u / kWords;
+                        const uint32_t words = (uint32_t)q->col_words;
+                        const uint32_t at = min((lo >> 4) + kWords * ((uint32_t)lane % per), words - kWords);
+#pragma unroll 8
+                        for (uint32_t i = 0; i < per; ++i) {
+                            const uint32_t k = ((uint32_t)lane + 64u * i) / per;
+                            const uint32_t j = k < (uint32_t)nb2 ? ids[k] : 0u;
+                            load_to_lds<4 * (int)kWords>(q->dense + (size_t)j * words + at, dst + 64u * kWords * i);
+                        }
+                    };
+                    if (p.S % 64u == 0u) columns(std::integral_constant<uint32_t, 4>());
+                    else columns(std::integral_constant<uint32_t, 1>());
+                }
+                // Gram rows of block b + 1's in-model slots
+                if (nb1 > 0) {
+                    const PipeMeta& m = L.meta[b1 & (kRing - 1)];
+                    const bool in = lane < nb1 && m.bo[lane < nb1 ? lane : 0] != 0.0;
+                    unsigned long long im = __ballot(in);
+                    const int have = min((int)__popcll(im), kRows);
+                    for (int i = 0; i < have; ++i, im &= im - 1) {
+                        const int h = (int)__ffsll((long long)im) - 1;
+                        load_to_lds<16>(gram + ((size_t)b1 * B + (size_t)h) * kGramCols + 2 * lane, &L.rows[b1 & 1][i][0]);
+                    }
+                }
+                if (q->mode == kModeChain && lane < nb1) {
+                    double u;
+                    uint64_t zw;
+                    chain_draws(*q, L.ids[b1 & (kRing - 1)][lane], iteration, u, zw);
+                    L.du[b1 & 1][lane] = u;
+                    L.dz[b1 & 1][lane] = bits_as_double(zw);
+                }
+                wait_vm<0>();   // the loads into LDS are done
+                __syncthreads();
+                if (L.abort) goto done;
+            }
+        } else {
+            __builtin_amdgcn_s_setprio(2);
+            for (int b = -2; b < nblocks; ++b) {
+                asm volatile("" : "+s"(q), "+v"(lane));
+                const int b2 = b + 2, b3 = b + 3;
+                const int nb2 = count(b2);
+                // constants of block b + 2 and ids of block b + 3
+                const uint32_t j = lane < nb2 ? L.ids[b2 & (kRing - 1)][lane] : 0u;
+                const uint64_t bo = ld_agent((const uint64_t*)(q->beta + j));
+                const int32_t g = q->group ? q->group[j] : 0;
+                const double u_ = q->u[j], z_ = q->z[j];
+                double m0, m1, m2, m3 = 0.0;
+                if constexpr (dense) {
+                    const double* lt = q->lut + 4 * (size_t)j;
+                    m0 = lt[2];
+                    m1 = lt[3];
+                    m2 = lt[1];
+                    m3 = lt[0];
+                } else {
+                    const double* st = q->stats + 4 * (size_t)j;
+                    m0 = st[0];
+                    m1 = st[1];
+                    m2 = st[3];
+                }
+                const uint32_t id = order[min((uint32_t)b3 * B + (uint32_t)lane, M - 1u)];
+                if (lane < nb2) {
+                    PipeMeta& m = L.meta[b2 & (kRing - 1)];
+                    m.mk[lane] = j;
+                    m.gr[lane] = g;
+                    m.bo[lane] = bits_as_double(bo);
+                    m.w[lane][0] = m0;
+                    m.w[lane][1] = m1;
+                    m.w[lane][2] = m2;
+                    m.w[lane][3] = dense ? m3 : 1.0 / m1;
+                    m.u[lane] = u_;
+                    m.z[lane] = z_;
+                    if constexpr (kLay != kLayoutRagged) {
+                        // EigenBayesRKernel: missing calls at the mean
+                        const double t0 = dense ? m0 : 2.0, t1 = dense ? m1 : m0, t2 = dense ? m2 : 1.0, t3 = dense ? m3 : 0.0;
+                        // (entry order turned by the lane: the lanes' tables are a multiple of all banks apart)
+#pragma unroll 4
+                        for (int i = 0; i < 16; ++i) {
+                            const uint32_t n = (uint32_t)(i + lane) & 15u;
+                            L.pt[b2 & 1][lane][n][0] = (E)wt_of(n & 3u, t0, t1, t2, t3);
+                            L.pt[b2 & 1][lane][n][1] = (E)wt_of(n >> 2, t0, t1, t2, t3);
+                        }
+                    }
+                }
+                if (lane < count(b3)) L.ids[b3 & (kRing - 1)][lane] = id;
+                if (b >= 1) outputs(b - 1);
+                __syncthreads();
+                if (L.abort) goto done;
+            }
         }
         rnd += (uint32_t)nblocks;
         n_rounds += (unsigned long long)nblocks;
         if (wave < kDotWaves) {
             apply(nblocks - 1);
-            if (wave == 6) outputs(nblocks - 1);
+        } else if (wave == kMetaWave) {
+            outputs(nblocks - 1);
         } else if (wave == kDecWave && lane == 0) {
             L.epsSum = eS;
         }
