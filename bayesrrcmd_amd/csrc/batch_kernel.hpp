@@ -82,6 +82,7 @@ struct BBlock {
     uint8_t codes[kBB][kBRow];        // byte b of row k: individuals lo + 4b .. 4b + 3 of marker k
     double wt[kBB][4];                // dot weight per 2-bit code (0 for markers past the block)
     double ut[kBB][4];                // residual change per unit beta change, per code
+    float wtf[kBB][4], utf[kBB][4];   // the same for FP32 residual tiles
     double mstat[kBB][4];             // ragged: mean, sd, Zsum, 1 / sd
     double bo[kBB][kMaxT];            // beta before the block
     uint32_t mk[kBB];                 // marker ids
@@ -129,7 +130,8 @@ struct BShared {
         }                                                                        \
     } while (0)
 
-__device__ __forceinline__ uint64_t* bslot1(const BatchParams& p, uint32_t rnd, uint32_t w, uint32_t v)
+template <class Params>
+__device__ __forceinline__ uint64_t* bslot1(const Params& p, uint32_t rnd, uint32_t w, uint32_t v)
 {
     return p.xchg1 + ((((size_t)(rnd & 1u) * p.P + w) * kBVmax + v) * 2u);
 }
@@ -137,7 +139,8 @@ __device__ __forceinline__ uint64_t* bslot1(const BatchParams& p, uint32_t rnd, 
 // totals in kCopies copies, as the BayesR sweep's (copy w % kCopies is read by workgroup w)
 constexpr size_t kBCopyWords = 2 * (size_t)kBVmax * 2 + 32;
 
-__device__ __forceinline__ uint64_t* bslot2(const BatchParams& p, uint32_t rnd, uint32_t v, uint32_t copy)
+template <class Params>
+__device__ __forceinline__ uint64_t* bslot2(const Params& p, uint32_t rnd, uint32_t v, uint32_t copy)
 {
     return p.xchg2 + copy * kBCopyWords + (((size_t)(rnd & 1u) * kBVmax + v) * 2u);
 }
@@ -178,7 +181,8 @@ __device__ __forceinline__ dbl4 to_dbl4(dbl4 x) { return x; }
 // 8 lane groups of a wave are folded by a fixed butterfly, the 4 waves in
 // index order, and the total is published. Every total is formed once, so all
 // workgroups read the same bits. Returns false (in all threads) on abort.
-__device__ __forceinline__ bool breduce(const BatchParams& p, BShared& L, uint32_t rnd, uint32_t V,
+template <class Params>
+__device__ __forceinline__ bool breduce(const Params& p, BShared& L, uint32_t rnd, uint32_t V,
                                         uint32_t w, int tid)
 {
     const int lane = tid & 63, wave = tid >> 6;
@@ -210,7 +214,8 @@ __device__ __forceinline__ bool breduce(const BatchParams& p, BShared& L, uint32
 }
 
 // All-reduce of one value per trait (published at v = trait): totals to L.tvec.
-__device__ __forceinline__ bool ballreduce_traits(const BatchParams& p, BShared& L, uint32_t rnd, uint32_t w,
+template <class Params>
+__device__ __forceinline__ bool ballreduce_traits(const Params& p, BShared& L, uint32_t rnd, uint32_t w,
                                                   int tid)
 {
     if (!breduce(p, L, rnd, p.T, w, tid)) return false;
@@ -235,7 +240,8 @@ struct BNext {
     double b[8];                // beta of pair u * 256 + tid = (k = e >> 6, t = e & 63)
 };
 
-__device__ __forceinline__ void bissue(const BatchParams& p, const uint32_t* ids, int nb, uint32_t lo, int tid,
+template <class Params>
+__device__ __forceinline__ void bissue(const Params& p, const uint32_t* ids, int nb, uint32_t lo, int tid,
                                        BNext& x)
 {
     const uint32_t per = p.nt;   // 32-bit words (16 individuals each) per marker row
@@ -270,7 +276,8 @@ __device__ __forceinline__ void bissue(const BatchParams& p, const uint32_t* ids
     }
 }
 
-__device__ __forceinline__ void bstore(const BatchParams& p, BBlock& L, const BNext& x, int nb, int tid)
+template <class Params>
+__device__ __forceinline__ void bstore(const Params& p, BBlock& L, const BNext& x, int nb, int tid)
 {
     const uint32_t per = p.nt;
 #pragma unroll
@@ -302,6 +309,11 @@ __device__ __forceinline__ void bstore(const BatchParams& p, BBlock& L, const BN
             L.ut[k][1] = 0.0;
             L.ut[k][2] = -meanAdjustment + oneAdjustment;
             L.ut[k][3] = -meanAdjustment;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            L.wtf[k][c] = (float)L.wt[k][c];
+            L.utf[k][c] = (float)L.ut[k][c];
         }
     }
 #pragma unroll
@@ -362,6 +374,9 @@ __device__ __forceinline__ BDraw bdraw(const BShared& L, int t, int K, double nu
 // tile's FP32 dot and Gram products are accumulated across tiles in FP64, and
 // the decisions, exchange and scalar draws stay FP64. The residual is not
 // refreshed: its FP32 rounding accumulates over the chain.
+// The parameter block in constant memory, read again in each block (pipe_kernel.hpp's ConstParams).
+typedef const __attribute__((address_space(4))) BatchParams* ConstBatchParams;
+
 template <int NT, bool kDenseMath, bool kF32>
 __global__ void __launch_bounds__(kThreads)
 bayesr_batch_kernel(BatchParams p)
@@ -370,17 +385,17 @@ bayesr_batch_kernel(BatchParams p)
     using ET4 = typename std::conditional<kF32, flt4, dbl4>::type;
     __shared__ BShared L;
     const uint32_t w = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int tq = lane & 15;          // matrix-core row / column index of this lane
-    const int kq = lane >> 4;          // matrix-core k index of this lane
+    int tid = threadIdx.x;
+    int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tq = lane & 15;                // matrix-core row / column index of this lane
+    int kq = lane >> 4;                // matrix-core k index of this lane
     const uint32_t lo = w * p.S;
-    const uint32_t nloc = min(p.S, p.N - lo);
+    uint32_t nloc = min(p.S, p.N - lo);
     const int T = (int)p.T;
     const int K = (int)p.K;
     const int nt = (int)p.nt;
-    const int tl = 16 * wave + tq;     // trait of this lane's residual column
+    int tl = 16 * wave + tq;           // trait of this lane's residual column
     const bool tval = tl < T;
     const ScalarLayout SL{1u, p.K};
     const uint32_t sls = SL.size();
@@ -426,6 +441,7 @@ bayesr_batch_kernel(BatchParams p)
     if (tid == 0) { L.sum_changes = 0; L.sum_drounds = 0; }
     if (tid == 0) L.tlast = __builtin_amdgcn_s_memrealtime();
     int cb = 0;     // current block buffer
+    ConstBatchParams q = (ConstBatchParams)__builtin_amdgcn_kernarg_segment_ptr();
     __syncthreads();
 
     const uint32_t iters = (p.mode == kModeChain) ? p.iterations : 1u;
@@ -526,6 +542,12 @@ bayesr_batch_kernel(BatchParams p)
         BRR_BTICK(5);
 
         for (uint32_t blk = 0; blk < nblocks; ++blk) {
+            // Lane indexes, the slice's length and the parameters are opaque in each block: addresses, row masks
+            // and fields formed from them once and kept over the unrolled tiles spilled (up to 2,900 registers
+            // of a lane, and each reload waits for all loads before it).
+            asm volatile("" : "+s"(q), "+s"(nloc), "+v"(tid), "+v"(lane), "+v"(tq), "+v"(kq), "+v"(tl));
+            const auto& p = *q;
+            const bool tval = tl < T;
             const uint32_t b0 = blk * kBB;
             const int nb = (int)min((uint32_t)kBB, p.M - b0);
             const bool has1 = blk + 1 < nblocks;
@@ -545,76 +567,78 @@ bayesr_batch_kernel(BatchParams p)
             BRR_BTICK(0);
 
             // ---- 1. partial dots C[k][t] over this slice (wave q: traits 16q..16q+15)
-            // and the partial Gram tiles (0,0), (0,1), (1,1) on waves 0, 1, 2. The
-            // lane's code rows (markers tq and 16 + tq) and their tables sit in
-            // registers, so each matrix-core step decodes its operand with a few
-            // VALU selects instead of dependent LDS reads.
+            // and the partial Gram tiles (0,0), (0,1), (1,1) on waves 0, 1, 2. A step's operand
+            // is looked up in the marker's four values in LDS: selected from registers it costs
+            // seven VALU operations, more than the product itself (16 lanes' values lie in
+            // different banks, equal ones are broadcast).
             {
-                // (FP32 tiles: up to 32 of them, so their code words are read from LDS
-                // tile by tile instead of being held in registers)
-                constexpr int NR = kF32 ? 1 : NT;
-                uint32_t rw0[NR], rw1[NR];
-                if constexpr (!kF32) {
-#pragma unroll
-                    for (int s = 0; s < NT; ++s) {
-                        rw0[s] = (s < nt) ? *(const uint32_t*)&B.codes[tq][4 * s] : 0u;
-                        rw1[s] = (s < nt) ? *(const uint32_t*)&B.codes[16 + tq][4 * s] : 0u;
-                    }
+                const ET* tw0;
+                const ET* tw1;
+                if constexpr (kF32) {
+                    tw0 = B.wtf[tq];
+                    tw1 = B.wtf[16 + tq];
+                } else {
+                    tw0 = B.wt[tq];
+                    tw1 = B.wt[16 + tq];
                 }
-                const double w00 = B.wt[tq][0], w01 = B.wt[tq][1], w02 = B.wt[tq][2], w03 = B.wt[tq][3];
-                const double w10 = B.wt[16 + tq][0], w11 = B.wt[16 + tq][1], w12 = B.wt[16 + tq][2],
-                             w13 = B.wt[16 + tq][3];
                 if (wave < (int)p.nq) {
                     dbl4 c0, c1;
-                    if constexpr (!kF32) {
-                        // two accumulator chains per marker tile (even / odd residual tiles)
-                        dbl4 acc0[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-                        dbl4 acc1[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-                        // straight-line code (no per-step branches, which would force the
-                        // accumulators out of the matrix-core registers at each join):
-                        // tiles past the slice hold zero residuals, slots past the block
-                        // zero weights
+                    // straight-line code (no per-step branches, which would force the
+                    // accumulators out of the matrix-core registers at each join): tiles past
+                    // the slice hold zero residuals, slots past the block zero weights (every
+                    // row holds kMaxNT words). A tile's operands are looked up while the tile
+                    // before is multiplied; left to itself the compiler waits for each.
+                    constexpr int kLane = kF32 ? 8 : 2, kStep = kF32 ? 2 : 8;   // bits of kq, of r
+                    ET a0[2][4], a1[2][4];
+                    uint32_t x0[2], x1[2];
+                    auto word = [&](int s) {
+                        x0[s & 1] = *(const uint32_t*)&B.codes[tq][4 * s];
+                        x1[s & 1] = *(const uint32_t*)&B.codes[16 + tq][4 * s];
+                    };
+                    auto look = [&](int s) {
+                        const uint32_t y0 = x0[s & 1] >> (kLane * kq), y1 = x1[s & 1] >> (kLane * kq);
 #pragma unroll
-                        for (int s = 0; s < NT; ++s) {
+                        for (int r = 0; r < 4; ++r) {
+                            a0[s & 1][r] = tw0[(y0 >> (kStep * r)) & 3u];
+                            a1[s & 1][r] = tw1[(y1 >> (kStep * r)) & 3u];
+                        }
+                    };
+                    word(0);
+                    look(0);
+                    if (NT > 1) word(1);
+                    // FP64: two accumulator chains per marker tile (even / odd residual tiles). FP32: a product
+                    // of 16 individuals per residual tile, the tiles summed in FP64 (one tile late).
+                    ET4 t0[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, t1[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+                    c0 = dbl4{0.0, 0.0, 0.0, 0.0};
+                    c1 = dbl4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                const uint32_t sh = 8u * (uint32_t)r + 2u * (uint32_t)kq;
-                                acc0[s & 1] = mfma16x16x4(wt_of((rw0[s < NR ? s : 0] >> sh) & 3u, w00, w01, w02, w03), E[s][r],
-                                                          acc0[s & 1]);
-                                acc1[s & 1] = mfma16x16x4(wt_of((rw1[s < NR ? s : 0] >> sh) & 3u, w10, w11, w12, w13), E[s][r],
-                                                          acc1[s & 1]);
+                    for (int s = 0; s < NT; ++s) {
+                        if (s + 1 < NT) look(s + 1);
+                        if (s + 2 < NT) word(s + 2);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (kF32) {
+                            t0[s & 1] = ET4{0, 0, 0, 0};
+                            t1[s & 1] = ET4{0, 0, 0, 0};
+                        }
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            t0[s & 1] = mfma16x16x4(a0[s & 1][r], E[s][r], t0[s & 1]);
+                            t1[s & 1] = mfma16x16x4(a1[s & 1][r], E[s][r], t1[s & 1]);
+                        }
+                        if constexpr (kF32) {
+                            if (s > 0) {
+                                c0 += to_dbl4(t0[(s - 1) & 1]);
+                                c1 += to_dbl4(t1[(s - 1) & 1]);
                             }
                         }
-                        c0 = acc0[0] + acc0[1];
-                        c1 = acc1[0] + acc1[1];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if constexpr (kF32) {
+                        c0 += to_dbl4(t0[(NT - 1) & 1]);
+                        c1 += to_dbl4(t1[(NT - 1) & 1]);
                     } else {
-                        // per residual tile an FP32 product of 16 individuals, the tiles
-                        // summed in FP64; entry r of the B operand is individual 4 kq + r
-                        float f00 = (float)w00, f01 = (float)w01, f02 = (float)w02, f03 = (float)w03;
-                        float f10 = (float)w10, f11 = (float)w11, f12 = (float)w12, f13 = (float)w13;
-                        // converted once here (an empty asm keeps the compiler from selecting
-                        // among the FP64 values and converting per step)
-                        asm volatile("" : "+v"(f00), "+v"(f01), "+v"(f02), "+v"(f03));
-                        asm volatile("" : "+v"(f10), "+v"(f11), "+v"(f12), "+v"(f13));
-                        c0 = dbl4{0.0, 0.0, 0.0, 0.0};
-                        c1 = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                        for (int s = 0; s < NT; ++s) {
-                            // loaded without a branch (every row holds kMaxNT words), masked after
-                            const uint32_t x0 = *(const uint32_t*)&B.codes[tq][4 * s];
-                            const uint32_t x1 = *(const uint32_t*)&B.codes[16 + tq][4 * s];
-                            const uint32_t a0 = (s < nt) ? x0 : 0u;
-                            const uint32_t a1 = (s < nt) ? x1 : 0u;
-                            flt4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                const uint32_t sh = 8u * (uint32_t)kq + 2u * (uint32_t)r;
-                                t0 = mfma16x16x4(wt_of_f((a0 >> sh) & 3u, f00, f01, f02, f03), (float)E[s][r], t0);
-                                t1 = mfma16x16x4(wt_of_f((a1 >> sh) & 3u, f10, f11, f12, f13), (float)E[s][r], t1);
-                            }
-                            c0 += to_dbl4(t0);
-                            c1 += to_dbl4(t1);
-                        }
+                        c0 = t0[0] + t0[1];
+                        c1 = t1[0] + t1[1];
                     }
                     if (tval) {
 #pragma unroll
@@ -631,51 +655,53 @@ bayesr_batch_kernel(BatchParams p)
                     const bool mi = wave == 2;        // row tile of u (A operand)
                     const bool mc = wave != 0;        // column tile of w (B operand)
                     if (16 * (int)mc < nb) {
-                        const int ra = 16 * (int)mi + tq;
-                        const double u0 = B.ut[ra][0], u1 = B.ut[ra][1], u2 = B.ut[ra][2], u3 = B.ut[ra][3];
-                        const double b0 = mc ? w10 : w00, b1 = mc ? w11 : w01, b2 = mc ? w12 : w02,
-                                     b3 = mc ? w13 : w03;
-                        dbl4 g;
-                        if constexpr (!kF32) {
-                            dbl4 gg[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+                        const ET* tu;
+                        if constexpr (kF32) tu = B.utf[16 * (int)mi + tq];
+                        else tu = B.ut[16 * (int)mi + tq];
+                        const ET* tb = mc ? tw1 : tw0;
+                        const uint8_t* ca = B.codes[16 * (int)mi + tq];
+                        const uint8_t* cw = B.codes[16 * (int)mc + tq];
+                        dbl4 g = {0.0, 0.0, 0.0, 0.0};
+                        ET4 gg[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+                        ET au[2][4], bw[2][4];
+                        uint32_t xa[2], xb[2];
+                        auto word = [&](int s) {
+                            xa[s & 1] = *(const uint32_t*)&ca[4 * s];
+                            xb[s & 1] = *(const uint32_t*)&cw[4 * s];
+                        };
+                        auto look = [&](int s) {
+                            const uint32_t ya = xa[s & 1] >> (2 * kq), yb = xb[s & 1] >> (2 * kq);
 #pragma unroll
-                            for (int s = 0; s < NT; ++s) {
-                                const uint32_t rowa = mi ? rw1[s < NR ? s : 0] : rw0[s < NR ? s : 0];
-                                const uint32_t rowb = mc ? rw1[s < NR ? s : 0] : rw0[s < NR ? s : 0];
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) {
-                                    const uint32_t sh = 8u * (uint32_t)r + 2u * (uint32_t)kq;
-                                    const uint32_t i = 16u * (uint32_t)s + 4u * (uint32_t)r + (uint32_t)kq;
-                                    const double av = (i < nloc) ? wt_of((rowa >> sh) & 3u, u0, u1, u2, u3) : 0.0;
-                                    gg[r & 1] = mfma16x16x4(av, wt_of((rowb >> sh) & 3u, b0, b1, b2, b3), gg[r & 1]);
-                                }
+                            for (int r = 0; r < 4; ++r) {
+                                au[s & 1][r] = tu[(ya >> (8 * r)) & 3u];
+                                bw[s & 1][r] = tb[(yb >> (8 * r)) & 3u];
                             }
-                            g = gg[0] + gg[1];
-                        } else {
-                            // per tile an FP32 product, the tiles summed in FP64
-                            float fu0 = (float)u0, fu1 = (float)u1, fu2 = (float)u2, fu3 = (float)u3;
-                            float fb0 = (float)b0, fb1 = (float)b1, fb2 = (float)b2, fb3 = (float)b3;
-                            // converted once (as for the dot tiles)
-                            asm volatile("" : "+v"(fu0), "+v"(fu1), "+v"(fu2), "+v"(fu3));
-                            asm volatile("" : "+v"(fb0), "+v"(fb1), "+v"(fb2), "+v"(fb3));
-                            g = dbl4{0.0, 0.0, 0.0, 0.0};
+                        };
+                        word(0);
+                        look(0);
+                        if (NT > 1) word(1);
 #pragma unroll
-                            for (int s = 0; s < NT; ++s) {
-                                // loaded without a branch (every row holds kMaxNT words), masked after
-                                const uint32_t xa = *(const uint32_t*)&B.codes[16 * (int)mi + tq][4 * s];
-                                const uint32_t xb = *(const uint32_t*)&B.codes[16 * (int)mc + tq][4 * s];
-                                const uint32_t rowa = (s < nt) ? xa : 0u, rowb = (s < nt) ? xb : 0u;
-                                flt4 gt = {0.f, 0.f, 0.f, 0.f};
+                        for (int s = 0; s < NT; ++s) {
+                            if (s + 1 < NT) look(s + 1);
+                            if (s + 2 < NT) word(s + 2);
+                            __builtin_amdgcn_sched_barrier(0);
+                            if constexpr (kF32) gg[s & 1] = ET4{0, 0, 0, 0};
 #pragma unroll
-                                for (int r = 0; r < 4; ++r) {
-                                    const uint32_t sh = 8u * (uint32_t)r + 2u * (uint32_t)kq;
-                                    const uint32_t i = 16u * (uint32_t)s + 4u * (uint32_t)r + (uint32_t)kq;
-                                    const float av = (i < nloc) ? wt_of_f((rowa >> sh) & 3u, fu0, fu1, fu2, fu3) : 0.f;
-                                    gt = mfma16x16x4(av, wt_of_f((rowb >> sh) & 3u, fb0, fb1, fb2, fb3), gt);
-                                }
-                                g += to_dbl4(gt);
+                            for (int r = 0; r < 4; ++r) {
+                                // individuals past the slice are other workgroups'
+                                const uint32_t i = 16u * (uint32_t)s + 4u * (uint32_t)r + (uint32_t)kq;
+                                const ET av = (i < nloc) ? au[s & 1][r] : (ET)0;
+                                const int c = kF32 ? s & 1 : r & 1;
+                                gg[c] = mfma16x16x4(av, bw[s & 1][r], gg[c]);
                             }
+                            // FP32: a product per tile, the tiles summed in FP64 (one tile late)
+                            if constexpr (kF32) {
+                                if (s > 0) g += to_dbl4(gg[(s - 1) & 1]);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
                         }
+                        if constexpr (kF32) g += to_dbl4(gg[(NT - 1) & 1]);
+                        else g = gg[0] + gg[1];
                         const int CT = nb * T;
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
@@ -906,39 +932,35 @@ bayesr_batch_kernel(BatchParams p)
                         for (int i2 = 0; i2 < HS; ++i2) acc[i2] = ET4{0, 0, 0, 0};
                         for (uint32_t m = fmask; m; m &= m - 1u) {
                             const int km = 4 * __builtin_ctz(m) + kq;   // < kBB: the rows read below exist
-                            const bool kv = km < nb;
-                            // straight-line loads: a row past the slice's tiles or past the block
-                            // reads what the buffer holds and is masked to zero after the load
-                            uint32_t row[HS];
-#pragma unroll
-                            for (int i2 = 0; i2 < HS; ++i2) {
-                                const int s2 = h * HS + i2;
-                                const uint32_t wrow = *(const uint32_t*)&B.codes[km][4 * (s2 < NT ? s2 : 0)];
-                                row[i2] = (s2 < nt && kv) ? wrow : 0u;
-                            }
-                            ET u0 = (ET)B.ut[km][0], u1 = (ET)B.ut[km][1], u2 = (ET)B.ut[km][2],
-                               u3 = (ET)B.ut[km][3];
-                            // FP32 tiles: the four values converted once here (an empty asm keeps the
-                            // compiler from selecting among the FP64 values and converting per tile)
-                            if constexpr (kF32) asm volatile("" : "+v"(u0), "+v"(u1), "+v"(u2), "+v"(u3));
+                            const ET* tu;
+                            if constexpr (kF32) tu = B.utf[km];
+                            else tu = B.ut[km];
+                            const uint8_t* cu = B.codes[km];
                             const ET cdv = (ET)L.cd[km][16 * wave + tq];
-                            const ET bv = kv ? cdv : (ET)0;
-                            // rows past the slice are masked to zero by i < nloc (a select, not a branch)
+                            const ET bv = km < nb ? cdv : (ET)0;
+                            // (straight-line loads: a row past the slice's tiles or past the block reads
+                            // what the buffer holds)
 #pragma unroll
                             for (int i2 = 0; i2 < HS; ++i2) {
                                 const int s2 = h * HS + i2;
                                 if (s2 < NT) {
-                                    const uint32_t i = 16u * (uint32_t)s2 + (uint32_t)tq;
-                                    const ET wv = wt_t((row[i2] >> (2u * (uint32_t)tq)) & 3u, u0, u1, u2, u3);
-                                    const ET av = (i < nloc) ? wv : (ET)0;
-                                    acc[i2] = mfma16x16x4(av, bv, acc[i2]);
+                                    const uint32_t x = *(const uint32_t*)&cu[4 * s2];
+                                    acc[i2] = mfma16x16x4(tu[(x >> (2 * tq)) & 3u], bv, acc[i2]);
                                 }
                             }
                         }
 #pragma unroll
                         for (int i2 = 0; i2 < HS; ++i2) {
                             const int s2 = h * HS + i2;
-                            if (s2 < NT) E[s2 < NT ? s2 : 0] += acc[i2];
+                            if (s2 < NT) {
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) {
+                                    // rows past the slice stay zero
+                                    const uint32_t i = 16u * (uint32_t)s2 + (uint32_t)acc_row<kF32>(r, kq);
+                                    const ET e = E[s2 < NT ? s2 : 0][r] + acc[i2][r];
+                                    E[s2 < NT ? s2 : 0][r] = (i < nloc) ? e : (ET)0;
+                                }
+                            }
                         }
                     }
                 }
