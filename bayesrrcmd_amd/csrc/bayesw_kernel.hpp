@@ -89,6 +89,19 @@ struct ArmsEnv {
     int n, state, kinit, q, wq, guard;
 };
 
+// The same run with its scalars in registers and the envelope in the ArmsEnv's arrays, for the per-marker draws:
+// in LDS every scalar costs its latency at every use.
+struct ArmsRegs {
+    double *x, *y, *ey, *cum, *area;
+    double ymax, yu, ynew;
+    double wx, wy, wey;
+    double xout;
+    uint64_t seed;
+    uint32_t site, iteration, chain, k;
+    int n, state, kinit, q, wq, guard;
+    __device__ __forceinline__ explicit ArmsRegs(ArmsEnv& e) : x(e.x), y(e.y), ey(e.ey), cum(e.cum), area(e.area) {}
+};
+
 template <int R>
 struct BwShared {
     double theta[kMaxF];          // fixed effects
@@ -106,6 +119,7 @@ struct BwShared {
     double cls[kMaxK], pi[kMaxK], v[kMaxK];
     double gv[kBwB][kMaxK - 1][14];   // weighted integrand terms per slot, slab class and node
     double ml[kBwB][kMaxK];            // class likelihoods per slot
+    double sg[kBwB][kMaxK - 1];        // sigma per slot and slab class
     double ghx[14], ghw[14], ghwc;     // the rule's nodes in summation order
     double mu, alpha, sigma_b, d, visum, betasq;
     int stop;                     // first slot that changes eps this round
@@ -121,13 +135,17 @@ struct BwShared {
 // on the wave's envelope with identical data, so the lockstep lanes store
 // identical values.
 
-__device__ __forceinline__ double arms_u(ArmsEnv& e)
+// Two uniforms in turn: the halves of one counter block.
+template <class Env>
+__device__ __forceinline__ void arms_u2(Env& e, double (&u)[2])
 {
-    const uint32_t k = e.k++;
-    const U4 x = draw_block(e.seed, e.site, e.iteration, kStreamArms | ((k >> 1) << 8), e.chain);
-    const uint32_t hi = (k & 1u) ? x.x[2] : x.x[0], lo = (k & 1u) ? x.x[3] : x.x[1];
-    const uint64_t w = ((uint64_t)hi << 32) | lo;
-    return ((double)(w >> 11) + 0.5) * 1.1102230246251565404e-16;
+    const U4 x = draw_block(e.seed, e.site, e.iteration, kStreamArms | ((e.k >> 1) << 8), e.chain);
+    e.k += 2;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint64_t w = ((uint64_t)x.x[2 * i] << 32) | x.x[2 * i + 1];
+        u[i] = ((double)(w >> 11) + 0.5) * 1.1102230246251565404e-16;
+    }
 }
 
 __device__ __forceinline__ double arms_expshift(double y, double y0)
@@ -142,7 +160,8 @@ __device__ __forceinline__ double arms_logshift(double y, double y0) { return lo
 // Nonzero on a convexity violation or a misplaced intersection. Reads only
 // evaluated points, so every intersection may be recomputed at once: one whose
 // neighbours did not change gets the same value again.
-__device__ __forceinline__ int arms_meet_at(ArmsEnv& e, int q)
+template <class Env>
+__device__ __forceinline__ int arms_meet_at(Env& e, int q)
 {
     const int n = e.n;
     double gl = 0, gr = 0, grl = 0, dl = 0, dr = 0;
@@ -184,7 +203,8 @@ __device__ __forceinline__ int arms_meet_at(ArmsEnv& e, int q)
 }
 
 // every intersection of the wave's envelope; nonzero if any fails
-__device__ __forceinline__ int arms_meet_all(ArmsEnv& e, int lane)
+template <class Env>
+__device__ __forceinline__ int arms_meet_all(Env& e, int lane)
 {
     bool bad = false;
 #pragma unroll
@@ -198,7 +218,8 @@ __device__ __forceinline__ int arms_meet_all(ArmsEnv& e, int lane)
 // exponentiate and integrate the envelope (BayesW_arms.cpp:672-703, 812-834):
 // ey and the areas in parallel, the running sum in position order as the
 // reference accumulates it
-__device__ __forceinline__ void arms_cumulate(ArmsEnv& e, int lane)
+template <class Env>
+__device__ __forceinline__ void arms_cumulate(Env& e, int lane)
 {
     const int n = e.n;
     double m = -__builtin_inf();
@@ -225,30 +246,34 @@ __device__ __forceinline__ void arms_cumulate(ArmsEnv& e, int lane)
             e.ey[q] = eyq[h];
         }
     }
+    // running sums in position order, as the reference accumulates them: the areas come from their lanes'
+    // registers (1.5 us for a dozen positions when each went through LDS)
+    double cum[2] = {0.0, 0.0}, c = 0.0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+        if (64 * h >= n) break;
         const int q = lane + 64 * h;
+        const double up = __shfl_up(eyq[h], 1, 64);
+        const double eyl = h && lane == 0 ? lane_read(eyq[0], 63) : up;
+        double a = 0.0;
         if (q >= 1 && q < n) {
-            const double eyl = arms_expshift(e.y[q - 1], ymax);   // the value its left neighbour stored
-            double a;
             if (e.x[q - 1] == e.x[q]) a = 0.0;
             else if (fabs(e.y[q] - e.y[q - 1]) < 0.1) a = 0.5 * (eyq[h] + eyl) * (e.x[q] - e.x[q - 1]);
             else a = ((eyq[h] - eyl) / (e.y[q] - e.y[q - 1])) * (e.x[q] - e.x[q - 1]);
-            e.area[q] = a;
         }
-    }
-    double c = 0.0;
-    e.cum[0] = 0.0;
-    for (int q = 1; q < n; ++q) {
-        c = c + e.area[q];
-        e.cum[q] = c;
+        for (int i = h ? 0 : 1; i < 64 && 64 * h + i < n; ++i) {
+            c = c + lane_read(a, i);
+            if (lane == i) cum[h] = c;
+        }
+        if (q < n) e.cum[q] = cum[h];
     }
     e.ymax = ymax;
 }
 
 // the x whose envelope cumulative probability is prob, into the working point
 // (BayesW_arms.cpp:364-425); it falls between positions q - 1 and q, q = e.wq
-__device__ __forceinline__ int arms_invert(ArmsEnv& e, double prob, int lane)
+template <class Env>
+__device__ __forceinline__ int arms_invert(Env& e, double prob, int lane)
 {
     const int n = e.n;
     const double u = prob * e.cum[n - 1];
@@ -295,7 +320,8 @@ enum : int { kAsInit = 0, kAsSample = 1, kAsEvalW = 2, kAsEvalQ = 3 };
 
 // Sets up one draw (arms with ninit = 4, npoint = 100, nsamp = 1 and no
 // Metropolis step, BayesW_arms.cpp:133-340); 0 or the reference's error code.
-__device__ __forceinline__ int arms_begin(ArmsEnv& e, const double (&xinit)[4], double xl, double xr, uint64_t seed,
+template <class Env>
+__device__ __forceinline__ int arms_begin(Env& e, const double (&xinit)[4], double xl, double xr, uint64_t seed,
                                           uint32_t site, uint32_t iteration, uint32_t chain, int lane)
 {
     constexpr int ninit = 4, mpoint = 2 * ninit + 1;
@@ -322,11 +348,12 @@ __device__ __forceinline__ int arms_begin(ArmsEnv& e, const double (&xinit)[4], 
 // asked for. Returns kArmsEval with e.xout the next point to evaluate, kArmsDone
 // with e.xout the sample, or an error code (>= 1000). Every lane of a wave calls
 // it with the same arguments on the wave's own envelope.
-__device__ __forceinline__ int arms_step(ArmsEnv& e, double y, int lane)
+template <class Env>
+__device__ __forceinline__ int arms_step(Env& e, double y, int lane)
 {
     constexpr int mpoint = 9;
     if (e.state == kAsInit) {
-        if (e.kinit > 0) e.y[2 * e.kinit - 1] = y;
+        if (e.kinit > 0) e.y[2 * e.kinit - 1] = y;   // (the last of those evaluated side by side, too)
         if (e.kinit < 4) {
             e.xout = e.x[2 * e.kinit + 1];
             e.kinit++;
@@ -402,9 +429,11 @@ __device__ __forceinline__ int arms_step(ArmsEnv& e, double y, int lane)
     }
     // sample and squeeze (BayesW_arms.cpp:344-360, 429-503)
     if (++e.guard > 100000) return 2001;
-    const int err = arms_invert(e, arms_u(e), lane);
+    double u[2];
+    arms_u2(e, u);
+    const int err = arms_invert(e, u[0], lane);
     if (err) return err;
-    e.yu = arms_logshift(arms_u(e) * e.wey, e.ymax);
+    e.yu = arms_logshift(u[1] * e.wey, e.ymax);
     const int wq = e.wq, n = e.n;
     if (wq - 2 >= 0 && wq + 1 <= n - 1) {
         const int ql = ((wq - 1) & 1) ? wq - 1 : wq - 2;
@@ -426,15 +455,26 @@ __device__ __noinline__ int arms_step_call(ArmsEnv& e, double y, int lane) { ret
 
 // One draw from log density f (inlined at the call site, where it may run
 // grid-wide sums: every thread of the grid takes the same path). 0 or an error.
+// kInline: f is a function of the lane's own point, and the four initial points
+// are evaluated side by side.
 template <bool kInline, class F>
-__device__ __forceinline__ int arms_draw(ArmsEnv& e, const double (&xinit)[4], double xl, double xr, uint64_t seed,
+__device__ __forceinline__ int arms_draw(ArmsEnv& env, const double (&xinit)[4], double xl, double xr, uint64_t seed,
                                          uint32_t site, uint32_t iteration, uint32_t chain, F&& f, double* out)
 {
     const int lane = threadIdx.x & 63;
+    typename std::conditional<kInline, ArmsRegs, ArmsEnv&>::type e(env);
     int st = arms_begin(e, xinit, xl, xr, seed, site, iteration, chain, lane);
     if (st) return st;
     double y = 0.0;
-    while ((st = kInline ? arms_step(e, y, lane) : arms_step_call(e, y, lane)) == kArmsEval) y = f(e.xout);
+    if constexpr (kInline) {
+        const double ys = f(e.x[2 * (lane & 3) + 1]);
+        if (lane < 4) e.y[2 * lane + 1] = ys;
+        y = lane_read(ys, 3);
+        e.kinit = 4;
+        while ((st = arms_step(e, y, lane)) == kArmsEval) y = f(e.xout);
+    } else {
+        while ((st = arms_step_call(e, y, lane)) == kArmsEval) y = f(e.xout);
+    }
     if (st != kArmsDone) return st;
     *out = e.xout;
     return 0;
@@ -624,9 +664,9 @@ bayesw_sweep_kernel(BwParams p)
     constexpr int kPer = kDense ? 3 : 2;   // per-code sums published per slot (codes 2, 0 [, 1])
     __shared__ BwShared<R> L;
     const uint32_t w = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
+    int tid = threadIdx.x;
+    int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lo = w * p.S;
     const uint32_t hi = min(lo + p.S, p.N);
     const int K = (int)p.K;
@@ -894,6 +934,8 @@ bayesw_sweep_kernel(BwParams p)
 
             int pos = 0;
             while (pos < nb) {
+                // (no address is kept over the rounds: spilled, each reload waits for all loads before it)
+                asm volatile("" : "+v"(tid), "+v"(lane));
                 // h: the first slot from pos whose marker is in the model (beta_old != 0).
                 // Its step starts from eps + x beta_old. When h == pos the round is
                 // that marker's own; otherwise the round publishes the sums of slots
@@ -1057,8 +1099,9 @@ bayesw_sweep_kernel(BwParams p)
                 BW_TICK(2);
 
                 // ---- decisions. Class likelihoods of the slots [pos, h] (or h alone in
-                // its own round): first the weighted integrand terms (slot, slab class,
-                // node) over all threads, then each (slot, class) sum in the reference's
+                // its own round): sigma of each (slot, slab class), formed once instead of at
+                // every node, the weighted integrand terms (slot, slab class, node) over all
+                // threads, then each (slot, class) sum in the reference's
                 // order, then the pick (wave 0, lane = slot). Slot h always stops the
                 // round: its step changes eps whatever its class.
                 // Sums of slot sl: (vi_sum, vi_1, vi_2) at xv[0], xv[1 + 2 sl], xv[2 + 2 sl],
@@ -1066,32 +1109,6 @@ bayesw_sweep_kernel(BwParams p)
                 {
                     const int ncls = K - 1, nn = (int)p.nq - 1, per = ncls * nn;
                     const int ns = breaker ? 1 : (spec ? h + 1 - pos : nb - pos);
-                    for (int t = tid; t < ns * per; t += kThreads) {
-                        const int sl = t / per, rem = t - sl * per, i = rem / nn, n = rem - i * nn;
-                        const int k = pos + sl;
-                        const bool sh = spec && k == h;
-                        const int b = sh ? V0 + 1 : 1 + kPer * sl;
-                        const double vs = sh ? xv[V0] : xv[0];
-                        const double s1 = xv[b], s2 = xv[b + 1];
-                        const double Ck = L.cls[i];
-                        const double sq = sqrt(2 * Ck * L.sigma_b);
-                        double f;
-                        if constexpr (kDense) {
-                            const double s3 = xv[b + 2];
-                            const BwGroups g{{vs - s1 - s2 - s3, s1, s2, s3},
-                                             {L.tab[k][3], L.tab[k][2], L.tab[k][0], L.tab[k][1]}};
-                            const double sigma =
-                                1.0 / sqrt(1 + L.alpha * L.alpha * L.sigma_b * Ck * bw_dense_exp_sum(g));
-                            f = bw_dense_integrand(sigma * L.ghx[n], L.alpha, sq, L.sumf[k], g);
-                        } else {
-                            const BwSums v{vs, vs - s1 - s2, s1, s2};
-                            const double mean = L.mean[k], sd = L.sd[k];
-                            const double sigma = bw_sigma(L.alpha, L.sigma_b, Ck, mean, sd, v);
-                            f = bw_integrand(sigma * L.ghx[n], L.alpha, sq, L.sumf[k], mean / sd, sd, v);
-                        }
-                        L.gv[sl][i][n] = L.ghw[n] * f;
-                    }
-                    __syncthreads();
                     for (int t = tid; t < ns * ncls; t += kThreads) {
                         const int sl = t / ncls, i = t - sl * ncls;
                         const int k = pos + sl;
@@ -1099,20 +1116,46 @@ bayesw_sweep_kernel(BwParams p)
                         const int b = sh ? V0 + 1 : 1 + kPer * sl;
                         const double vs = sh ? xv[V0] : xv[0];
                         const double s1 = xv[b], s2 = xv[b + 1];
-                        double sigma;
                         if constexpr (kDense) {
                             const double s3 = xv[b + 2];
                             const BwGroups g{{vs - s1 - s2 - s3, s1, s2, s3},
                                              {L.tab[k][3], L.tab[k][2], L.tab[k][0], L.tab[k][1]}};
-                            sigma = 1.0 / sqrt(1 + L.alpha * L.alpha * L.sigma_b * L.cls[i] * bw_dense_exp_sum(g));
+                            L.sg[sl][i] = 1.0 / sqrt(1 + L.alpha * L.alpha * L.sigma_b * L.cls[i] * bw_dense_exp_sum(g));
                         } else {
                             const BwSums v{vs, vs - s1 - s2, s1, s2};
-                            sigma = bw_sigma(L.alpha, L.sigma_b, L.cls[i], L.mean[k], L.sd[k], v);
+                            L.sg[sl][i] = bw_sigma(L.alpha, L.sigma_b, L.cls[i], L.mean[k], L.sd[k], v);
                         }
+                    }
+                    __syncthreads();
+                    for (int t = tid; t < ns * per; t += kThreads) {
+                        const int sl = t / per, rem = t - sl * per, i = rem / nn, n = rem - i * nn;
+                        const int k = pos + sl;
+                        const bool sh = spec && k == h;
+                        const int b = sh ? V0 + 1 : 1 + kPer * sl;
+                        const double vs = sh ? xv[V0] : xv[0];
+                        const double s1 = xv[b], s2 = xv[b + 1];
+                        const double sq = sqrt(2 * L.cls[i] * L.sigma_b);
+                        const double x = L.sg[sl][i] * L.ghx[n];
+                        double f;
+                        if constexpr (kDense) {
+                            const double s3 = xv[b + 2];
+                            const BwGroups g{{vs - s1 - s2 - s3, s1, s2, s3},
+                                             {L.tab[k][3], L.tab[k][2], L.tab[k][0], L.tab[k][1]}};
+                            f = bw_dense_integrand(x, L.alpha, sq, L.sumf[k], g);
+                        } else {
+                            const BwSums v{vs, vs - s1 - s2, s1, s2};
+                            const double mean = L.mean[k], sd = L.sd[k];
+                            f = bw_integrand(x, L.alpha, sq, L.sumf[k], mean / sd, sd, v);
+                        }
+                        L.gv[sl][i][n] = L.ghw[n] * f;
+                    }
+                    __syncthreads();
+                    for (int t = tid; t < ns * ncls; t += kThreads) {
+                        const int sl = t / ncls, i = t - sl * ncls;
                         double temp = L.gv[sl][i][0];
                         for (int n = 1; n < nn; ++n) temp = temp + L.gv[sl][i][n];
                         temp = temp + L.ghwc;
-                        L.ml[sl][i + 1] = L.pi[i + 1] * (sigma * temp);
+                        L.ml[sl][i + 1] = L.pi[i + 1] * (L.sg[sl][i] * temp);
                     }
                     __syncthreads();
                     if (wave == 0) {
