@@ -40,6 +40,8 @@ using namespace brr;
 // 16 of counters, 1 of the order flag (a copy of the scratch words from the
 // control words on)
 constexpr int kStatusWords = 4 + 16 + 1;
+constexpr size_t kStagePiece = 64 * 1024;          // pinned stage of small host arrays: one array, all of a call's
+constexpr size_t kStageBytes = 4 * kStagePiece;
 
 // device counters of a launch: [0] rounds, [1] changes, [2..7] phase ticks,
 // batched kernel also [8] decision rounds (summed over waves), [10..15] phase ticks 6..11
@@ -76,7 +78,7 @@ struct brr_hip_ctx {
     size_t gram_cap = 0;         // rows
     int32_t* d_gram_acc = nullptr;
     size_t gram_acc_cap = 0;     // rows x products
-    uint64_t* h_status = nullptr; // pinned: control words, counters and order flag of brr_hip_sweep_noalloc
+    uint64_t* h_status = nullptr; // pinned: control words, counters, the order flag of brr_hip_sweep_noalloc, then the stage
     bool record_num = false;
     uint32_t refresh_markers = 1024;
     double change_rate = 1.0;    // beta changes per marker visit in the last chain launch
@@ -577,6 +579,49 @@ void shape_stats(brr_hip_ctx* c)
     c->stats.storage = c->codes ? 2u : 1u;
 }
 
+// Small host arrays go through the context's pinned stage and its stream, with one wait for all of a call's: each
+// hipMemcpy of its own is a wait (12 us for 4 KB), and a small sweep has eleven of them. Larger ones are copied
+// directly. The stage is free again after each call's wait.
+struct Stage {
+    brr_hip_ctx* c;
+    size_t used = 0;
+    struct { void* dst; size_t at, bytes; } back[4] = {};
+    int n = 0;
+
+    uint8_t* take(size_t bytes)
+    {
+        if (bytes > kStagePiece || used + bytes > kStageBytes) return nullptr;
+        uint8_t* at = (uint8_t*)(c->h_status + kStatusWords) + used;
+        used += (bytes + 63) / 64 * 64;
+        return at;
+    }
+    hipError_t to_device(void* dst, const void* src, size_t bytes)
+    {
+        if (uint8_t* at = take(bytes)) {
+            std::memcpy(at, src, bytes);
+            return hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, c->stream);
+        }
+        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    }
+    // arrives with finish()
+    hipError_t to_host(void* dst, const void* src, size_t bytes)
+    {
+        uint8_t* at = n < 4 ? take(bytes) : nullptr;
+        if (!at) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+        back[n++] = {dst, (size_t)(at - (uint8_t*)(c->h_status + kStatusWords)), bytes};
+        return hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, c->stream);
+    }
+    hipError_t finish()
+    {
+        if (!used) return hipSuccess;
+        const hipError_t e = hipStreamSynchronize(c->stream);
+        if (e == hipSuccess)
+            for (int i = 0; i < n; ++i)
+                std::memcpy(back[i].dst, (const uint8_t*)(c->h_status + kStatusWords) + back[i].at, back[i].bytes);
+        return e;
+    }
+};
+
 int reset_exchange(brr_hip_ctx* c)
 {
     HIP_TRY(c, hipMemsetAsync(c->d_xchg1, 0, sizeof(uint64_t) * c->x1_words, c->stream));
@@ -596,13 +641,16 @@ int run_launches(brr_hip_ctx* c, Enqueue&& enqueue)
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     HIP_TRY(c, enqueue());
     HIP_TRY(c, hipEventRecord(c->ev1, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    float ms = 0.f;
-    HIP_TRY(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     uint32_t ctl[4] = {0, 0, 0, 0};
     unsigned long long counters[kCounters] = {};
-    HIP_TRY(c, hipMemcpy(ctl, c->d_ctl, sizeof(ctl), hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(counters, c->d_counters, sizeof(counters), hipMemcpyDeviceToHost));
+    static_assert(sizeof(ctl) <= 4 * sizeof(uint64_t) && kCounters + 4 <= kStatusWords, "pinned words");
+    HIP_TRY(c, hipMemcpyAsync(c->h_status, c->d_ctl, sizeof(ctl), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(c->h_status + 4, c->d_counters, sizeof(counters), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    std::memcpy(ctl, c->h_status, sizeof(ctl));
+    std::memcpy(counters, c->h_status + 4, sizeof(counters));
+    float ms = 0.f;
+    HIP_TRY(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     std::memcpy(c->last_counters, counters, sizeof(counters));
     c->stats.kernel_ms = ms;
     c->stats.rounds = counters[0];
@@ -1080,15 +1128,15 @@ int brr_hip_create(const brr_hip_config* cfg, brr_hip_ctx** out)
     }
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_status, sizeof(uint64_t) * kStatusWords) != hipSuccess) {
+        hipHostMalloc((void**)&c->h_status, sizeof(uint64_t) * kStatusWords + kStageBytes) != hipSuccess) {
         brr_hip_destroy(c);
         return BRR_HIP_EDEVICE;
     }
-    (void)hipMemset(c->d_eps, 0, sizeof(double) * N * Tn);
-    (void)hipMemset(c->d_beta, 0, sizeof(double) * M * Tn);
-    (void)hipMemset(c->d_comp, 0, sizeof(int32_t) * M * Tn);
-    (void)hipMemset(c->d_acum, 0, sizeof(double) * M * Tn);
-    (void)hipMemset(c->d_scal, 0, sizeof(double) * SL.size() * Tn);
+    (void)hipMemsetAsync(c->d_eps, 0, sizeof(double) * N * Tn, c->stream);
+    (void)hipMemsetAsync(c->d_beta, 0, sizeof(double) * M * Tn, c->stream);
+    (void)hipMemsetAsync(c->d_comp, 0, sizeof(int32_t) * M * Tn, c->stream);
+    (void)hipMemsetAsync(c->d_acum, 0, sizeof(double) * M * Tn, c->stream);
+    (void)hipMemsetAsync(c->d_scal, 0, sizeof(double) * SL.size() * Tn, c->stream);
     c->x1_cap = c->x1_words;
     if (reset_exchange(c) != BRR_HIP_OK) { brr_hip_destroy(c); return BRR_HIP_EDEVICE; }
     *out = c;
@@ -1879,9 +1927,11 @@ int brr_hip_set_state(brr_hip_ctx* c, const double* eps, const double* beta, con
     if (!c) return BRR_HIP_EINVAL;
     HIP_TRY(c, hipSetDevice(c->device));
     const size_t N = c->cfg.num_inds, M = c->cfg.num_snps, Tn = c->Tn;
-    if (eps) HIP_TRY(c, hipMemcpy(c->d_eps, eps, sizeof(double) * N * Tn, hipMemcpyHostToDevice));
-    if (beta) HIP_TRY(c, hipMemcpy(c->d_beta, beta, sizeof(double) * M * Tn, hipMemcpyHostToDevice));
-    if (comp) HIP_TRY(c, hipMemcpy(c->d_comp, comp, sizeof(int32_t) * M * Tn, hipMemcpyHostToDevice));
+    Stage st{c};
+    if (eps) HIP_TRY(c, st.to_device(c->d_eps, eps, sizeof(double) * N * Tn));
+    if (beta) HIP_TRY(c, st.to_device(c->d_beta, beta, sizeof(double) * M * Tn));
+    if (comp) HIP_TRY(c, st.to_device(c->d_comp, comp, sizeof(int32_t) * M * Tn));
+    HIP_TRY(c, st.finish());
     return BRR_HIP_OK;
 }
 
@@ -1915,10 +1965,12 @@ int brr_hip_get_state(brr_hip_ctx* c, double* eps, double* beta, int32_t* comp, 
     HIP_TRY(c, hipSetDevice(c->device));
     const size_t N = c->cfg.num_inds, M = c->cfg.num_snps, Tn = c->Tn;
     if (acum && c->bw) return fail(c, BRR_HIP_EINVAL, "a BayesW context keeps no acum");
-    if (eps) HIP_TRY(c, hipMemcpy(eps, c->d_eps, sizeof(double) * N * Tn, hipMemcpyDeviceToHost));
-    if (beta) HIP_TRY(c, hipMemcpy(beta, c->d_beta, sizeof(double) * M * Tn, hipMemcpyDeviceToHost));
-    if (comp) HIP_TRY(c, hipMemcpy(comp, c->d_comp, sizeof(int32_t) * M * Tn, hipMemcpyDeviceToHost));
-    if (acum) HIP_TRY(c, hipMemcpy(acum, c->d_acum, sizeof(double) * M * Tn, hipMemcpyDeviceToHost));
+    Stage st{c};
+    if (eps) HIP_TRY(c, st.to_host(eps, c->d_eps, sizeof(double) * N * Tn));
+    if (beta) HIP_TRY(c, st.to_host(beta, c->d_beta, sizeof(double) * M * Tn));
+    if (comp) HIP_TRY(c, st.to_host(comp, c->d_comp, sizeof(int32_t) * M * Tn));
+    if (acum) HIP_TRY(c, st.to_host(acum, c->d_acum, sizeof(double) * M * Tn));
+    HIP_TRY(c, st.finish());
     return BRR_HIP_OK;
 }
 
@@ -1966,9 +2018,10 @@ int brr_hip_sweep(brr_hip_ctx* c, const uint32_t* order, const double* u, const 
         if ((rc = dalloc(c, &c->d_order, M))) return rc;
         c->order_cap = M;
     }
-    HIP_TRY(c, hipMemcpy(c->d_order, order, sizeof(uint32_t) * M, hipMemcpyHostToDevice));
-    HIP_TRY(c, hipMemcpy(c->d_u, u, sizeof(double) * M * c->Tn, hipMemcpyHostToDevice));
-    HIP_TRY(c, hipMemcpy(c->d_z, z, sizeof(double) * M * c->Tn, hipMemcpyHostToDevice));
+    Stage st{c};   // (the launch waits for its copies)
+    HIP_TRY(c, st.to_device(c->d_order, order, sizeof(uint32_t) * M));
+    HIP_TRY(c, st.to_device(c->d_u, u, sizeof(double) * M * c->Tn));
+    HIP_TRY(c, st.to_device(c->d_z, z, sizeof(double) * M * c->Tn));
     SweepParams p = base_params(c);
     p.mode = kModeSweep;
     p.iterations = 1;
@@ -1976,6 +2029,7 @@ int brr_hip_sweep(brr_hip_ctx* c, const uint32_t* order, const double* u, const 
     p.u = c->d_u;
     p.z = c->d_z;
     rc = launch_any(c, p);
+    if (rc) (void)st.finish();
     c->stats.markers = (uint64_t)M * c->Tn;
     return rc;
 }
@@ -2287,14 +2341,15 @@ int brr_hip_bw_create(const brr_hip_bw_config* cfg, brr_hip_ctx** out)
         return rc;
     }
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
+        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_status, sizeof(uint64_t) * kStatusWords + kStageBytes) != hipSuccess) {
         brr_hip_destroy(c);
         return BRR_HIP_EDEVICE;
     }
-    (void)hipMemset(c->d_eps, 0, sizeof(double) * N);
-    (void)hipMemset(c->d_beta, 0, sizeof(double) * M);
-    (void)hipMemset(c->d_comp, 0, sizeof(int32_t) * M);
-    (void)hipMemset(c->d_scal, 0, sizeof(double) * nscal);
+    (void)hipMemsetAsync(c->d_eps, 0, sizeof(double) * N, c->stream);
+    (void)hipMemsetAsync(c->d_beta, 0, sizeof(double) * M, c->stream);
+    (void)hipMemsetAsync(c->d_comp, 0, sizeof(int32_t) * M, c->stream);
+    (void)hipMemsetAsync(c->d_scal, 0, sizeof(double) * nscal, c->stream);
     if (reset_exchange(c) != BRR_HIP_OK) { brr_hip_destroy(c); return BRR_HIP_EDEVICE; }
     *out = c;
     return BRR_HIP_OK;
