@@ -802,13 +802,16 @@ bayesr_batch_kernel(BatchParams p)
             }
             BRR_BTICK(2);
 
-            // ---- 3. decisions, wave q for its traits 16q .. 16q+15 (traits are
-            // independent chains, so each wave resolves its tile without
-            // workgroup barriers). Rounds: every pending (slot, trait) pair is
+            // ---- 3. decisions, wave q for its quarter of the traits (traits are
+            // independent chains, so each wave resolves its own without
+            // workgroup barriers; by matrix-core tiles of 16, five traits would take
+            // eight trips of one wave instead of one trip of three). Rounds: every pending (slot, trait) pair is
             // drawn in parallel; each trait accepts its pairs up to its first beta
             // change, the dots of its later slots are corrected by delta * Gram
             // row (BayesRBase.cpp:370-378) and those slots are drawn again.
-            if (wave < (int)p.nq) {
+            const int tw = (T + kWaves - 1) / kWaves;      // traits of a wave, at most 16
+            if (wave * tw < T) {
+                const uint32_t inv = (65536u + (uint32_t)tw - 1u) / (uint32_t)tw;   // e / tw = e inv >> 16 for e < 512
                 // the traits whose outputs of this block this workgroup writes: t with
                 // (t + 7 blk) % P == w (one division per block, not one per trait)
                 unsigned long long own = 0;
@@ -816,8 +819,8 @@ bayesr_batch_kernel(BatchParams p)
                     const uint32_t sh = (blk * 7u) % p.P;
                     for (uint32_t t = w >= sh ? w - sh : w + p.P - sh; t < (uint32_t)T; t += p.P) own |= 1ull << t;
                 }
-                const int tt = 16 * wave + tq;             // trait of this lane's accept work
-                const bool tok = tt < T;
+                const int tt = tw * wave + tq;             // trait of this lane's accept work
+                const bool tok = tq < tw && tt < T;
                 const bool mine = tok && ((own >> tt) & 1ull);   // output workgroup
                 const bool single_out = p.T <= p.P;   // then a workgroup outputs at most one trait per block
                 uint16_t* plist = L.plist + wave * (kBB * 16);
@@ -835,12 +838,12 @@ bayesr_batch_kernel(BatchParams p)
                     if (!first && kq == 0)
                         for (int i = 0; i < cnt; ++i) plist[incl - cnt + i] = (uint16_t)(((p0 + i) << 8) | tt);
                     wave_lds_sync();
-                    const int span = first ? nb * 16 : total;
+                    const int span = first ? nb * tw : total;
                     for (int e = lane; e < span; e += 64) {
                         int k, t;
                         if (first) {
-                            k = e >> 4;
-                            t = 16 * wave + (e & 15);
+                            k = (int)(((uint32_t)e * inv) >> 16);
+                            t = tw * wave + (e - k * tw);
                             if (t >= T) continue;
                         } else {
                             const int kt = plist[e];
@@ -879,7 +882,7 @@ bayesr_batch_kernel(BatchParams p)
                                     st_agent((uint64_t*)(p.acum + o), double_as_bits(ac));
                                 }
                                 L.cd[k][tt] = (k == c) ? dl : 0.0;
-                                if (k == c) atomicOr(&L.flag[k >> 2], 1u << wave);
+                                if (k == c) atomicOr(&L.flag[k >> 2], 1u << (tt >> 4));
                             } else {
                                 L.cd[k][tt] += dl * L.gm[c][k];
                             }
@@ -915,8 +918,11 @@ bayesr_batch_kernel(BatchParams p)
                     }
                     L.betasqn[tt] = bs;
                 }
-                // ---- 4. eps_t += sum_k delta_{k,t} u_k on the matrix cores, for the
-                // 4-marker steps holding a change of this wave's traits
+            }
+            if (tw < 16) __syncthreads();   // (with 16, a wave's traits are its tile's)
+            // ---- 4. eps_t += sum_k delta_{k,t} u_k on the matrix cores (wave q: traits 16q..16q+15),
+            // for the 4-marker steps holding a change of this wave's traits
+            if (wave < (int)p.nq) {
                 uint32_t fmask = 0u;
 #pragma unroll
                 for (int p4 = 0; p4 < kBB / 4; ++p4)
