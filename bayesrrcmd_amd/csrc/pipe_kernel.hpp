@@ -9,13 +9,19 @@
 //     dots become dot_k + dBeta_h G[h][k] and they are decided again at once, on one wave, without the grid;
 //   - the dots of block b + 1 are formed and exchanged from the residual before block b's changes while block
 //     b is decided, and corrected the same way, so the exchange is off the critical path.
-// A workgroup is ten waves with one role each, in lockstep by one barrier per block (step b):
+// A workgroup is twelve waves with one role each, in lockstep by one barrier per block (step b):
 //   waves 0-7   apply block b - 1's changes to their copy of the residual slice, form and publish the partial
-//               dots of 8 slots each of block b + 1, then store the prefetched columns of block b + 2, the Gram
-//               rows of block b + 1's in-model slots and the outputs of block b - 1;
+//               dots of 8 slots each of block b + 1;
 //   wave 8      waits for block b's totals, corrects and decides them (lane = slot) change by change;
-//   wave 9      reduces the slots of block b that belong to this workgroup (slot k to workgroup k mod P) and
-//               draws block b + 1's u and z.
+//   wave 9      reduces this workgroup's slots of block b + 1 and gathers its totals, as far as they arrive before
+//               block b is decided;
+//   wave 10     loads the columns of block b + 2 and the Gram rows of block b + 1's in-model slots into LDS and
+//               draws block b + 1's u and z;
+//   wave 11     constants and pair table of block b + 2, ids of block b + 3, outputs of block b - 1.
+// Waves 8 to 11 have a higher wave priority than the dot waves: as the youngest of their SIMDs they were served last
+// (a gather took 7.5 us while the dot waves had work, 1.5 us now). A step takes 3.9 us at N = 60,000 dense FP64
+// (6.2 us with ten waves at one priority, scattered partials and spilled addresses), 4.3 us at 100,000 ragged FP32:
+// apply and dots 2.4 us, their exchange 2.5 us beside the 1.3 us of block b's decisions.
 // With at most 16 workgroups every workgroup sums all partials itself and the reduce hop is left out.
 // Every workgroup decides from the same totals with the same instructions, so all hold the same bits.
 #pragma once
@@ -33,7 +39,9 @@ constexpr int kDotThreads = 64 * kDotWaves;
 constexpr int kPipeThreads = kDotThreads + 256;
 constexpr int kSlotsPerWave = kMaxB / kDotWaves;
 constexpr int kRing = 4;                 // blocks of columns and constants held at once
-constexpr uint32_t kDirectP = 16;        // workgroups up to which the partials are summed without a reduce hop
+// Workgroups up to which the partials are summed without a reduce hop. An exchange of 64 slots alone takes 2.1 us at
+// 16 workgroups so (2.4 with the hop) and 2.8 us at 24 (2.5 with it): each workgroup reads all partials.
+constexpr uint32_t kDirectP = 16;
 
 // Gram rows of a block kept in LDS: those of its first in-model slots; others are loaded when needed. As many
 // as 160 KB hold beside the columns and, but for the ragged layout, the pair tables.

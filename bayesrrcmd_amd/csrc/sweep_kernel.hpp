@@ -1,4 +1,6 @@
-// sweep_kernel.hpp -- persistent gfx950 kernel for the BayesR per-marker Gibbs sweep.
+// sweep_kernel.hpp -- persistent gfx950 kernel for the BayesR per-marker Gibbs sweep, round by round: index lists,
+// asynchronous windows, single-marker blocks and slices of more than two lane runs. Sequential sweeps over 2-bit columns
+// are pipe_kernel.hpp's, which shares the parameters, the exchange words and the iteration scalars of this file.
 //
 // What it computes: BayesRBase::processColumn (BayesRBase.cpp:287-392) over a
 // marker order, i.e. for each marker j in sequence
@@ -1139,8 +1141,7 @@ __device__ __forceinline__ void ragged_store(const SweepParams& p, Shared<R>& L,
 // re-rounded from it. The decisions, the scalar draws, updateMu, the fixed
 // effects and |eps|^2 are FP64 throughout.
 // The sweep of one context by one of its P workgroups (w), with the LDS of
-// the workgroup passed in: the body of bayesr_sweep_kernel and of the cohort
-// kernel below, which runs several contexts side by side in one launch.
+// the workgroup passed in: the body of bayesr_sweep_kernel.
 template <int R, int kLay, bool kCodes, bool kAsync, bool kF32>
 __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, RefreshLog<kF32, R>& RL,
                                            const uint32_t w)
