@@ -1347,7 +1347,9 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
     (void)hipEventElapsedTime(&ms_unpack, c->ev0, c->ev1);
     if (dense) {
         if (!hip_ok(hipEventRecord(c->ev0, c->stream), "hipEventRecord")) return BRR_HIP_EDEVICE;
-        bed_dense_table_kernel<<<(M + kBedThreads / 64 - 1) / (kBedThreads / 64), kBedThreads, 0, c->stream>>>(
+        const bool waves = bed_wave_sums(N, M);
+        const uint32_t per = waves ? kBedThreads / 64 : kBedThreads;
+        (waves ? bed_dense_table_kernel<true> : bed_dense_table_kernel<false>)<<<(M + per - 1) / per, kBedThreads, 0, c->stream>>>(
             c->d_dense, c->col_words, N, M, d_cnt, c->d_lut);
         if (!hip_ok(hipGetLastError(), "bed_dense_table_kernel") ||
             !hip_ok(hipEventRecord(c->ev1, c->stream), "hipEventRecord") ||

@@ -114,19 +114,50 @@ bed_unpack_kernel(const uint32_t* __restrict__ src, uint64_t cb, uint32_t N, uin
     }
 }
 
+// The running FP64 sum of tab(v) over the values v of one column's individuals
+// 0..N-1, added one at a time in individual order. tab(v) = tabl[v * kBedThreads]:
+// the calling thread's entries in LDS, one plane per value so that the lanes of
+// a wave read distinct banks whatever their values.
+__device__ __forceinline__ double bed_ordered_sum_lane(const uint4* col, uint32_t N, const double* tabl)
+{
+    double acc = 0.0;
+    const uint32_t nfull = N / 64u;
+    uint4 next = nfull ? col[0] : make_uint4(0u, 0u, 0u, 0u);
+    for (uint32_t q = 0; q < nfull; ++q) {
+        const uint4 w = next;
+        if (q + 1u < nfull) next = col[q + 1u];
+        const uint32_t xs[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < 16u; ++e) acc = acc + tabl[((xs[k] >> (2u * e)) & 3u) * kBedThreads];
+    }
+    uint32_t rest = N - 64u * nfull;
+    if (rest) {
+        const uint4 w = col[nfull];
+        const uint32_t xs[4] = {w.x, w.y, w.z, w.w};
+        for (int k = 0; k < 4 && rest; ++k) {
+            const uint32_t n = rest < 16u ? rest : 16u;
+            for (uint32_t e = 0; e < n; ++e) acc = acc + tabl[((xs[k] >> (2u * e)) & 3u) * kBedThreads];
+            rest -= n;
+        }
+    }
+    return acc;
+}
+
 // The running FP64 sum of x[v] >= 0 over the values v of one column's individuals 0..N-1, added one at a time in
 // individual order, by one wave; n[v] > 0 tells which values occur. While the sum stays in one binade it is a multiple
 // of that binade's unit and each addition adds x[v] rounded to the unit, whatever came before: the sum over a
 // stretch is an exact combination of the counts. Only a value half a unit off looks at the last bit (it rounds to
 // even, so the bit is 0 after it); the lanes then follow that bit through their individuals for both its values.
 // Lane l counts the values of 64 individuals, a scan over the lanes finds the first 64 that leave the binade, and
-// only those are added one by one: about a dozen times a column. One lane adding a whole column took
-// 2.46 ms for 8,000 columns of 100,000 individuals (60 cycles an addition); this takes 0.50 ms.
+// only those are added one by one: about a dozen times a column.
 __device__ __forceinline__ double bed_ordered_sum(const uint4* col, uint32_t N, const double (&x)[4],
                                                   const uint32_t (&n)[4], int lane)
 {
     const uint32_t chunks = (N + 63u) / 64u;
-    const double x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+    // (scalar registers: the one-by-one additions then choose their value beside the vector unit)
+    const double x0 = lane_read(x[0], 0), x1 = lane_read(x[1], 0), x2 = lane_read(x[2], 0), x3 = lane_read(x[3], 0);
     double acc = 0.0;
     for (uint32_t c0 = 0; c0 < chunks; c0 += 64u) {
         const uint32_t at = c0 + (uint32_t)lane;
@@ -237,42 +268,64 @@ __device__ __forceinline__ double bed_ordered_sum(const uint4* col, uint32_t N, 
 }
 
 // DenseMarkerBuilder::endColumn from the counts and the codes: one wave per
-// marker. The table holds the standardised value of dosage 0, 1, 2 and of a
+// marker (kWave) or one lane. The table holds the standardised value of dosage 0, 1, 2 and of a
 // missing call. The mean of the non-missing dosages and, without missing calls,
 // the column mean are integer sums (exact from the counts); with missing calls
 // the column sum, and always the squared norm, are summed in individual order.
+template <bool kWave>
 static __global__ void __launch_bounds__(kBedThreads)
 bed_dense_table_kernel(const uint32_t* __restrict__ codes, uint64_t col_words, uint32_t N, uint32_t M,
                        const uint32_t* __restrict__ counts, double* __restrict__ lut)
 {
+    __shared__ double tab[kWave ? 1 : 4 * kBedThreads];   // a lane's entries, value v at [v * kBedThreads]
     const int lane = (int)(threadIdx.x & 63u);
-    const uint32_t j = blockIdx.x * (kBedThreads / 64u) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t j = kWave ? blockIdx.x * (kBedThreads / 64u) +
+                                   (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))
+                             : blockIdx.x * kBedThreads + threadIdx.x;
     if (j >= M) return;
     const uint4* col = reinterpret_cast<const uint4*>(codes + (size_t)j * col_words);
     const uint32_t n2 = counts[4 * (size_t)j + 0];   // value 0: dosage 2
     const uint32_t nm = counts[4 * (size_t)j + 1];   // value 1: missing
     const uint32_t n1 = counts[4 * (size_t)j + 2];   // value 2: dosage 1
-    const uint32_t n[4] = {n2, nm, n1, N - n2 - nm - n1};
+    auto ordered_sum = [&](double x0, double x1, double x2, double x3) {
+        if constexpr (kWave) {
+            const double x[4] = {x0, x1, x2, x3};
+            const uint32_t n[4] = {n2, nm, n1, N - n2 - nm - n1};
+            return bed_ordered_sum(col, N, x, n, lane);
+        } else {
+            double* t = tab + threadIdx.x;
+            t[0 * kBedThreads] = x0;
+            t[1 * kBedThreads] = x1;
+            t[2 * kBedThreads] = x2;
+            t[3 * kBedThreads] = x3;
+            return bed_ordered_sum_lane(col, N, t);
+        }
+    };
     const double numInds = (double)N;
     const double sum = (double)((uint64_t)n1 + 2u * (uint64_t)n2);
     const double mean = sum / (numInds - (double)nm);
     double s = sum;                                   // integer terms: the index-order sum is exact
-    if (nm) {
-        const double x[4] = {2.0, mean, 1.0, 0.0};
-        s = bed_ordered_sum(col, N, x, n, lane);
-    }
+    if (nm) s = ordered_sum(2.0, mean, 1.0, 0.0);
     const double cmean = s / numInds;
     const double d0 = 0.0 - cmean, d1 = 1.0 - cmean, d2 = 2.0 - cmean, dm = mean - cmean;
-    const double x[4] = {d2 * d2, dm * dm, d1 * d1, d0 * d0};
-    const double sqn = bed_ordered_sum(col, N, x, n, lane);
+    const double sqn = ordered_sum(d2 * d2, dm * dm, d1 * d1, d0 * d0);
     const double sigma = 1.0 / (sqrt(sqn / (numInds - 1.0)));
-    if (lane == 0) {
+    if (!kWave || lane == 0) {
         double* o = lut + 4 * (size_t)j;
         o[0] = d0 * sigma;
         o[1] = d1 * sigma;
         o[2] = d2 * sigma;
         o[3] = dm * sigma;
     }
+}
+
+// A wave per column against a lane per column. A lane takes 13 ns an individual whatever the number of columns (up to
+// about 65,000, a wave per SIMD); waves take 27 us and, with the chip full, 8.5 ns + 0.16 ns per 1,000 individuals
+// a column more. Measured, wave against lane: 8,000 columns of 100,000 individuals 0.24 / 1.3 ms, 40,000 0.98 / 1.34,
+// 100,000 2.45 / 1.95; 8,000 of 3,000 0.105 / 0.044, 500 of 500 0.030 / 0.012.
+inline bool bed_wave_sums(uint32_t N, uint32_t M)
+{
+    return 13.0 * N > 27000.0 + M * (8.5 + 1.6e-4 * N);
 }
 
 } // namespace brr
