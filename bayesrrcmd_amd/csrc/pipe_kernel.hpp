@@ -623,7 +623,10 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
             }
         }
         if (wave < kDotWaves) {
-            int due = (int)q->refresh_blocks;   // blocks until the FP32 slice is re-rounded
+            // blocks until the FP32 slice is re-rounded: half the interval asked for, since the re-rounding reaches
+            // the dots two steps after the block that it follows
+            const int every = (int)max((q->refresh_blocks + 1u) / 2u, 1u);
+            int due = every;
             bool fresh = false;
             for (int b = -2; b < nblocks; ++b) {
                 asm volatile("" : "+s"(q), "+v"(lane));
@@ -643,7 +646,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                     apply(b - 1);
                     if constexpr (kF32) {
                         fresh = --due == 0;
-                        if (fresh) due = (int)q->refresh_blocks;
+                        if (fresh) due = every;
                         if (fresh)
 #pragma unroll
                             for (int r = 0; r < R; ++r) L.fs[b & 1][r * kRun + tid] = (float)e64[r];
