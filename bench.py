@@ -994,12 +994,12 @@ def main():
                                "column's device bytes, 4 N one FP32 residual pass (whatever precision the kernel "
                                "computes in), delta_j = 1 when beta_j changed; the residual passes are served from "
                                "registers, so HBM moves only the columns and the exchange words"),
-            "kernel": "brr::bayesr_sweep_kernel (one launch per iteration)",
+            "kernel": "brr::bayesr_pipe_kernel (one launch per iteration, with its Gram launch)",
             "avg_launch_ms": avg_ms, "algorithmic_bytes_per_launch": bytes_per_launch,
             "column_bytes_per_launch": float(m) * ((n + 3) // 4) if stats["storage"] == 2 else None,
             "column_GBps": (float(m) * ((n + 3) // 4) / (avg_ms * 1e-3) / 1e9) if stats["storage"] == 2 else None,
             "limiter": {
-                "kind": "latency: exchange rounds (one per block of markers plus one per other beta change)",
+                "kind": "latency: one exchange per block of markers, with the steps around it",
                 "rounds_per_launch": float(np.mean(rounds)),
                 "exchange_us_per_round_probe": probe_us,
                 "exchange_floor_ms": (float(np.mean(rounds)) * probe_us * 1e-3) if probe_us else None,

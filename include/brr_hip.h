@@ -380,7 +380,9 @@ int brr_hip_last_stats(const brr_hip_ctx* ctx, brr_hip_stats* stats);
 
 /* Device time of workgroup 0 in each phase of the last launch, ms (n <= 12
  * values written). Single chain: block load, partial dots, exchange,
- * decisions, commit/update, per-iteration scalars. Batched: block commit, dot
+ * decisions, commit/update, per-iteration scalars; where the sweep is pipelined
+ * the phases overlap: block load is the dot waves' wait for the step to end,
+ * exchange and decisions are the deciding wave's. Batched: block commit, dot
  * tiles, exchange gather, decision draws, residual update, per-iteration
  * scalars, Gram tiles, u/z draws, exchange reduce, accept/correct, block-end
  * barrier, spare. */
