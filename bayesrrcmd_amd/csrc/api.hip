@@ -40,7 +40,10 @@ using namespace brr;
 // 16 of counters, 1 of the order flag (a copy of the scratch words from the
 // control words on)
 constexpr int kStatusWords = 4 + 16 + 1;
-constexpr size_t kStagePiece = 64 * 1024;          // pinned stage of small host arrays: one array, all of a call's
+// Pinned stage of small host arrays: the largest of them, and all of a call's. A 3,000 x 1,500 call takes 275 us so, 311 us
+// with pieces of at most 16 KB; staging up to 1 MB as well changed calls of 12,000 to 100,000 individuals by less than
+// their runs differ (2 to 6%), for sixteen times the pinned memory.
+constexpr size_t kStagePiece = 64 * 1024;
 constexpr size_t kStageBytes = 4 * kStagePiece;
 
 // device counters of a launch: [0] rounds, [1] changes, [2..7] phase ticks,

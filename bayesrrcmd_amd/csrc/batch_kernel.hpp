@@ -570,7 +570,8 @@ bayesr_batch_kernel(BatchParams p)
             // and the partial Gram tiles (0,0), (0,1), (1,1) on waves 0, 1, 2. A step's operand
             // is looked up in the marker's four values in LDS: selected from registers it costs
             // seven VALU operations, more than the product itself (16 lanes' values lie in
-            // different banks, equal ones are broadcast).
+            // different banks, equal ones are broadcast). 25 FP32 tiles, 64 traits: 9.9 us a block
+            // looked up where they are used, 6.5 us a tile ahead, 28 us selected.
             {
                 const ET* tw0;
                 const ET* tw1;
@@ -805,7 +806,8 @@ bayesr_batch_kernel(BatchParams p)
             // ---- 3. decisions, wave q for its quarter of the traits (traits are
             // independent chains, so each wave resolves its own without
             // workgroup barriers; by matrix-core tiles of 16, five traits would take
-            // eight trips of one wave instead of one trip of three). Rounds: every pending (slot, trait) pair is
+            // eight trips of one wave instead of one trip of three; draws of 20 traits, N = 7,003,
+            // 0.63 -> 0.33 ms of a pass). Rounds: every pending (slot, trait) pair is
             // drawn in parallel; each trait accepts its pairs up to its first beta
             // change, the dots of its later slots are corrected by delta * Gram
             // row (BayesRBase.cpp:370-378) and those slots are drawn again.

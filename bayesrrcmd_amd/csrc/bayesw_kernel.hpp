@@ -90,7 +90,8 @@ struct ArmsEnv {
 };
 
 // The same run with its scalars in registers and the envelope in the ArmsEnv's arrays, for the per-marker draws:
-// in LDS every scalar costs its latency at every use.
+// in LDS every scalar costs its latency at every use (a draw took 14.3 us; 11.6 us with this, the initial points side
+// by side and the areas summed from registers).
 struct ArmsRegs {
     double *x, *y, *ey, *cum, *area;
     double ymax, yu, ynew;
