@@ -726,6 +726,7 @@ int gram_reserve(brr_hip_ctx* c, uint32_t iterations)
         c->gram_acc_cap = 0;
         if ((rc = dalloc(c, &c->d_gram_acc, acc * kGramCols))) return rc;
         HIP_TRY(c, hipMemsetAsync(c->d_gram_acc, 0, sizeof(int32_t) * acc * kGramCols, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));   // (cohorts use it on another context's stream)
         c->gram_acc_cap = acc;
     }
     return BRR_HIP_OK;
@@ -789,9 +790,7 @@ int prepare_pipe(brr_hip_ctx* c, bool counted)
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         c->missing = got != 0;
     }
-    if ((rc = gram_reserve(c, 1))) return rc;
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    return BRR_HIP_OK;
+    return gram_reserve(c, 1);
 }
 
 int launch(brr_hip_ctx* c, SweepParams& p)
@@ -1335,9 +1334,8 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
         cleanup();
         return rc;
     }
-    uint32_t* d_bad = d_cnt + 4 * (size_t)M;   // first unusable marker; whether any call is missing
-    if (!hip_ok(hipMemsetAsync(d_bad, 0xFF, sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
-        !hip_ok(hipMemsetAsync(d_bad + 1, 0, sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
+    uint32_t* d_bad = d_cnt + 4 * (size_t)M;   // first unusable marker; 0 if any call is missing
+    if (!hip_ok(hipMemsetAsync(d_bad, 0xFF, 2 * sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
         !hip_ok(hipEventRecord(c->ev0, c->stream), "hipEventRecord"))
         return BRR_HIP_EDEVICE;
     bed_unpack_kernel<<<M, kBedThreads, 0, c->stream>>>(d_stage, cb, N, c->col_words, c->d_dense, d_cnt,
@@ -1360,10 +1358,10 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
             return BRR_HIP_EDEVICE;
         (void)hipEventElapsedTime(&ms_table, c->ev0, c->ev1);
     }
-    uint32_t found[2] = {0xFFFFFFFFu, 0u};
+    uint32_t found[2] = {0xFFFFFFFFu, 0xFFFFFFFFu};
     if (!hip_ok(hipMemcpy(found, d_bad, sizeof(found), hipMemcpyDeviceToHost), "hipMemcpy")) return BRR_HIP_EDEVICE;
     const uint32_t bad = found[0];
-    c->missing = found[1] != 0;
+    c->missing = found[1] == 0;
     cleanup();
     c->stats = brr_hip_stats{};
     shape_stats(c);
