@@ -688,40 +688,18 @@ int launch_fn(brr_hip_ctx* c, const void* fn, void* param, uint32_t threads = kT
 
 // ------------------------------------------------------ pipelined sweep --
 
-// Rows of the Gram workspace one launch may fill when it runs several iterations (1 KB a row): what bounds the
-// workspace of a long chain (a chain of more is split into launches), and a thousand blocks fill the chip.
-constexpr size_t kGramRowsPerLaunch = 65536;
-// Blocks from which a Gram launch is not split over the individuals. At N = 100,000 a sweep of 125 blocks takes
-// 648 us with its Gram launch split in two (716 unsplit, and 219 instead of 70 at 4 blocks); of 250 blocks 1,265 us
-// unsplit and 1,332 split: the products then go through memory and a second launch.
-constexpr uint32_t kGramBlocks = 128;
-
-uint32_t gram_iterations(const brr_hip_ctx* c, uint32_t iterations)
-{
-    return (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, kGramRowsPerLaunch / c->cfg.num_snps));
-}
-
-uint32_t gram_splits(const brr_hip_ctx* c, uint32_t iterations)
-{
-    const uint32_t blocks = iterations * ((c->cfg.num_snps + c->B - 1) / c->B);
-    const uint32_t chunks = (c->cfg.num_inds + kGramChunk - 1) / kGramChunk;
-    return blocks >= kGramBlocks ? 1u : std::max(1u, std::min(2 * kGramBlocks / blocks, chunks));
-}
-
 int gram_products_of(const brr_hip_ctx* c) { return c->missing ? gram_products(c->layout) : 1; }
 
-// The workspace of a launch of `iterations` iterations.
-int gram_reserve(brr_hip_ctx* c, uint32_t iterations)
+// The workspace of `plan`'s launches: its Gram rows, and the shared counts if its blocks are split.
+int gram_reserve(brr_hip_ctx* c, const GramPlan& plan)
 {
-    const size_t rows = (size_t)iterations * c->cfg.num_snps;
     int rc;
-    if (c->gram_cap < rows) {
+    if (c->gram_cap < plan.rows) {
         c->gram_cap = 0;
-        if ((rc = dalloc(c, &c->d_gram, rows * kGramCols))) return rc;
-        c->gram_cap = rows;
+        if ((rc = dalloc(c, &c->d_gram, plan.rows * kGramCols))) return rc;
+        c->gram_cap = plan.rows;
     }
-    // (a block is at most 64 rows; whether it is split depends on the block size, which may change later)
-    const size_t acc = rows <= (size_t)kGramBlocks * kMaxB ? rows * gram_products_of(c) : 0;
+    const size_t acc = plan.acc_rows * gram_products_of(c);
     if (c->gram_acc_cap < acc) {
         c->gram_acc_cap = 0;
         if ((rc = dalloc(c, &c->d_gram_acc, acc * kGramCols))) return rc;
@@ -732,7 +710,13 @@ int gram_reserve(brr_hip_ctx* c, uint32_t iterations)
     return BRR_HIP_OK;
 }
 
-GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t iterations, const uint32_t* gate)
+GramPlan gram_plan_of(const brr_hip_ctx* c, uint32_t iterations)
+{
+    return gram_plan(c->cfg.num_inds, c->cfg.num_snps, c->B, iterations);
+}
+
+GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t iterations, uint32_t splits,
+                       const uint32_t* gate)
 {
     GramParams g{};
     g.N = c->cfg.num_inds;
@@ -740,7 +724,7 @@ GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t ite
     g.B = c->B;
     g.iterations = iterations;
     g.layout = c->layout;
-    g.splits = gram_splits(c, iterations);
+    g.splits = splits;
     g.codes = c->d_dense;
     g.col_words = c->col_words;
     g.counts = c->d_counts;
@@ -753,11 +737,13 @@ GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t ite
     return g;
 }
 
-// The Gram rows of `iterations` iterations, then the pipelined kernel over them.
-hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, uint32_t iterations)
+// The Gram rows of `iterations` iterations in blocks of `splits` workgroups, then the pipelined kernel over them.
+hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, uint32_t iterations, uint32_t splits)
 {
     if (p.mode == kModeSweep || p.mode == kModeChain) {
-        GramParams g = gram_params(c, p.order, iterations, p.gate);
+        const size_t rows = (size_t)iterations * c->cfg.num_snps;
+        if (rows > c->gram_cap || (splits > 1 && rows * gram_products_of(c) > c->gram_acc_cap)) return hipErrorInvalidValue;
+        GramParams g = gram_params(c, p.order, iterations, splits, p.gate);
         const uint32_t items = iterations * ((g.M + g.B - 1) / g.B) * g.splits;
         if (c->missing) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
         else gram_kernel<false><<<items, kGramThreads, 0, c->stream>>>(g);
@@ -790,7 +776,10 @@ int prepare_pipe(brr_hip_ctx* c, bool counted)
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         c->missing = got != 0;
     }
-    return gram_reserve(c, 1);
+    // (the block size may change before a sweep that cannot allocate: counts for whatever few blocks it then has)
+    GramPlan plan = gram_plan_of(c, 1);
+    plan.acc_rows = M <= kGramBlocks * (uint32_t)kMaxB ? M : 0;
+    return gram_reserve(c, plan);
 }
 
 int launch(brr_hip_ctx* c, SweepParams& p)
@@ -801,21 +790,18 @@ int launch(brr_hip_ctx* c, SweepParams& p)
                                        "(ragged_storage 0 or 2)");
     const SweepKernel k = kernel_of(c);
     if (!k.pipe) return launch_fn(c, k.fn, &p, k.threads);
-    if (p.mode != kModeChain) {
-        if (int rc = gram_reserve(c, 1)) return rc;
-        return run_launches(c, [&] { return enqueue_pipe(c, k, p, 1); });
-    }
+    const GramPlan plan = gram_plan_of(c, p.mode == kModeChain ? p.iterations : 1u);
+    if (int rc = gram_reserve(c, plan)) return rc;
+    if (p.mode != kModeChain) return run_launches(c, [&] { return enqueue_pipe(c, k, p, 1, plan.splits); });
     // a chain in launches of as many iterations as the Gram workspace holds
-    const uint32_t total = p.iterations, step = gram_iterations(c, total);
-    if (int rc = gram_reserve(c, step)) return rc;
     return run_launches(c, [&] {
-        for (uint32_t it = 0; it < total; it += step) {
+        for (uint32_t it = 0; it < plan.total; it += plan.step) {
             SweepParams q = p;
-            q.iterations = std::min(step, total - it);
+            q.iterations = plan.iterations(it);
             q.iter_base = p.iter_base + it;
             q.order = p.order + (size_t)it * p.M;
             q.hist = p.hist ? p.hist + (size_t)it * (4 + p.G) : nullptr;
-            if (hipError_t e = enqueue_pipe(c, k, q, q.iterations)) return e;
+            if (hipError_t e = enqueue_pipe(c, k, q, q.iterations, plan.splits)) return e;
         }
         return hipSuccess;
     });
@@ -1616,8 +1602,11 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
     }
     const uint32_t step = (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, 8 * kGramRowsPerLaunch / rows1));
     const uint32_t steps = (iterations + step - 1) / step;
-    for (uint32_t q = 0; q < n; ++q)
-        if ((rc = gram_reserve(ctxs[q], step))) return fail(c0, rc, ctxs[q]->err);
+    for (uint32_t q = 0; q < n; ++q) {
+        GramPlan plan{};   // (no block is split: the cohorts' blocks fill a launch together)
+        plan.rows = (size_t)step * ctxs[q]->cfg.num_snps;
+        if ((rc = gram_reserve(ctxs[q], plan))) return fail(c0, rc, ctxs[q]->err);
+    }
     HIP_TRY(c0, hipDeviceSynchronize());
     // parameter blocks by step in launch order, on the device; the Gram entries of all cohorts of a step in one launch
     std::vector<SweepParams> packed;
@@ -1635,8 +1624,7 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
                 p.hist += (size_t)it0 * (4 + p.G);
                 p.gram = c->d_gram;
                 packed.push_back(p);
-                GramEntry g{gram_params(c, p.order, its, nullptr), gram_items[st]};
-                g.p.splits = 1;
+                GramEntry g{gram_params(c, p.order, its, 1, nullptr), gram_items[st]};
                 grams.push_back(g);
                 gram_items[st] += its * ((g.p.M + g.p.B - 1) / g.p.B);
             }
@@ -2079,7 +2067,7 @@ int brr_hip_sweep_noalloc(brr_hip_ctx* c, const uint32_t* d_order, const double*
     p.refresh_blocks = std::max(1u, c->refresh_markers / c->B);
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     if (k.pipe) {
-        HIP_TRY(c, enqueue_pipe(c, k, p, 1));   // (the Gram workspace was allocated with the markers)
+        HIP_TRY(c, enqueue_pipe(c, k, p, 1, gram_plan_of(c, 1).splits));   // (its workspace was allocated with the markers)
     } else {
         void* args[] = {&p};
         HIP_TRY(c, hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream));

@@ -21,13 +21,13 @@
 // are the same in any order) and gram_finish_kernel forms the entries.
 #pragma once
 
+#include "gram_plan.hpp"
 #include "sweep_kernel.hpp"
 
 namespace brr {
 
 constexpr int kGramThreads = 512;
 constexpr int kGramCols = 2 * kMaxB;              // entries per row: the block's slots, then the next block's
-constexpr uint32_t kGramChunk = 1024;             // individuals staged at once
 constexpr uint32_t kGramChunkBytes = kGramChunk / 4;
 constexpr uint32_t kGramStride = kGramChunkBytes + 16;   // LDS bytes per column: rows start in shifted banks
 

@@ -1,0 +1,56 @@
+"""How a chain's Gram launches are cut (gram_plan.hpp, compiled here for the host): no launch of a call uses more rows
+of the Gram workspace or of the shared counts than the plan reserves for it."""
+import ctypes as C
+import itertools
+import subprocess
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parents[1] / "bayesrrcmd_amd" / "csrc"
+SHIM = """
+#include "gram_plan.hpp"
+extern "C" void plan(uint32_t N, uint32_t M, uint32_t B, uint32_t total, uint64_t* out)
+{
+    const brr::GramPlan p = brr::gram_plan(N, M, B, total);
+    out[0] = p.step; out[1] = p.splits; out[2] = p.rows; out[3] = p.acc_rows;
+    out[4] = out[5] = out[6] = out[7] = 0;   // iterations, launches, largest rows, rows of split launches
+    for (uint32_t it = 0; it < p.total; it += p.step) {
+        const uint64_t rows = (uint64_t)p.iterations(it) * M;
+        out[4] += p.iterations(it);
+        out[5] += 1;
+        if (rows > out[6]) out[6] = rows;
+        if (p.splits > 1 && rows > out[7]) out[7] = rows;
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("gram_plan")
+    (d / "shim.cpp").write_text(SHIM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{CSRC}", str(d / "shim.cpp"), "-o",
+                    str(d / "shim.so")], check=True)
+    lib = C.CDLL(str(d / "shim.so"))
+
+    def call(n, m, b, total):
+        out = (C.c_uint64 * 8)()
+        lib.plan(n, m, b, total, out)
+        return dict(zip(("step", "splits", "rows", "acc_rows", "iterations", "launches", "used", "used_acc"), out))
+    return call
+
+
+# the last launch of a chain is shorter than the others and may hold few blocks
+@pytest.mark.parametrize("n", [500, 5000, 100000])
+def test_launches_stay_inside_their_workspace(plan, n):
+    ms = [1, 63, 64, 65, 200, 500, 700, 1000, 3000, 4095, 8128, 8192, 9000, 33000, 65536, 65537, 300000]
+    for m, b, total in itertools.product(ms, [1, 2, 33, 64], [1, 2, 3, 7, 9, 23, 67, 100, 200, 400, 1000, 5000]):
+        p = plan(n, m, b, total)
+        at = (n, m, b, total, p)
+        assert p["iterations"] == total, at
+        assert p["used"] <= p["rows"] <= max(m, 65536), at
+        assert p["used_acc"] <= p["acc_rows"], at
+        assert p["acc_rows"] == 0 or p["acc_rows"] <= 128 * 64, at
+        # nearly equal launches, no more of them than their bound asks for
+        assert p["launches"] <= -(-total // max(1, 65536 // m)), at
