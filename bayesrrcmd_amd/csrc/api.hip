@@ -73,10 +73,11 @@ struct brr_hip_ctx {
     SweepParams* d_cohort = nullptr;   // brr_hip_run_cohorts: the cohorts' parameter blocks
     GramEntry* d_cohort_gram = nullptr;
     uint32_t cohort_cap = 0;
-    // pipelined sweep (gram_kernel.hpp): individuals per 2-bit value of each column, whether a call is missing,
-    // and the Gram rows (with shared counts where few blocks split the individuals) kept between launches
+    // pipelined sweep (gram_kernel.hpp): individuals per 2-bit value of each column, the markers' share in the Gram
+    // entries and the most bases of one, and the Gram rows (with shared counts where few blocks split the individuals) kept between launches
     uint32_t* d_counts = nullptr;
-    bool missing = false;
+    GramMarker* d_markers = nullptr;
+    int bases = 1;
     double* d_gram = nullptr;
     size_t gram_cap = 0;         // rows
     int32_t* d_gram_acc = nullptr;
@@ -688,7 +689,7 @@ int launch_fn(brr_hip_ctx* c, const void* fn, void* param, uint32_t threads = kT
 
 // ------------------------------------------------------ pipelined sweep --
 
-int gram_products_of(const brr_hip_ctx* c) { return c->missing ? gram_products(c->layout) : 1; }
+int gram_products_of(const brr_hip_ctx* c) { return gram_products(c->layout, c->bases); }
 
 // The workspace of `plan`'s launches: its Gram rows, and the shared counts if its blocks are split.
 int gram_reserve(brr_hip_ctx* c, const GramPlan& plan)
@@ -725,11 +726,10 @@ GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t ite
     g.iterations = iterations;
     g.layout = c->layout;
     g.splits = splits;
+    g.bases = c->bases;
     g.codes = c->d_dense;
     g.col_words = c->col_words;
-    g.counts = c->d_counts;
-    g.lut = c->d_lut;
-    g.stats = c->d_stats;
+    g.markers = c->d_markers;
     g.order = order;
     g.gram = c->d_gram;
     g.acc = c->d_gram_acc;
@@ -745,11 +745,11 @@ hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, ui
         if (rows > c->gram_cap || (splits > 1 && rows * gram_products_of(c) > c->gram_acc_cap)) return hipErrorInvalidValue;
         GramParams g = gram_params(c, p.order, iterations, splits, p.gate);
         const uint32_t items = iterations * ((g.M + g.B - 1) / g.B) * g.splits;
-        if (c->missing) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
+        if (c->bases > 1) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
         else gram_kernel<false><<<items, kGramThreads, 0, c->stream>>>(g);
         if (hipError_t e = hipGetLastError()) return e;
         if (g.splits > 1) {
-            gram_finish_kernel<<<iterations * g.M, kGramCols, 0, c->stream>>>(g, gram_products_of(c));
+            gram_finish_kernel<<<iterations * g.M, kGramCols, 0, c->stream>>>(g);
             if (hipError_t e = hipGetLastError()) return e;
         }
     }
@@ -758,8 +758,8 @@ hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, ui
     return hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream);
 }
 
-// Per-marker counts of the columns just stored, and the Gram workspace of a sweep (so that sweeps allocate
-// nothing). `counted`: the caller has the counts in place (and `missing` set).
+// The markers' share in the Gram entries, from the columns just stored, and the Gram workspace of a sweep (so that
+// sweeps allocate nothing). `counted`: the caller has the counts per code in place.
 int prepare_pipe(brr_hip_ctx* c, bool counted)
 {
     if (c->T || c->bw || !c->codes) return BRR_HIP_OK;
@@ -767,15 +767,19 @@ int prepare_pipe(brr_hip_ctx* c, bool counted)
     const uint32_t M = c->cfg.num_snps;
     if (!counted) {
         if ((rc = dalloc(c, &c->d_counts, (size_t)4 * M + 1))) return rc;
-        uint32_t* any = c->d_counts + 4 * (size_t)M;
-        uint32_t got = 0;
-        HIP_TRY(c, hipMemsetAsync(any, 0, sizeof(uint32_t), c->stream));
-        marker_counts_kernel<<<M, 256, 0, c->stream>>>(c->d_dense, c->col_words, c->cfg.num_inds, c->d_counts, any);
+        marker_counts_kernel<<<M, 256, 0, c->stream>>>(c->d_dense, c->col_words, c->cfg.num_inds, c->d_counts);
         HIP_TRY(c, hipGetLastError());
-        HIP_TRY(c, hipMemcpyAsync(&got, any, sizeof(got), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-        c->missing = got != 0;
     }
+    if ((rc = dalloc(c, &c->d_markers, (size_t)M))) return rc;
+    uint32_t* most = c->d_counts + 4 * (size_t)M;
+    uint32_t got = 0;
+    HIP_TRY(c, hipMemsetAsync(most, 0, sizeof(uint32_t), c->stream));
+    gram_markers_kernel<<<(M + 255) / 256, 256, 0, c->stream>>>(M, c->layout, c->d_lut, c->d_stats, c->d_counts,
+                                                                c->d_markers, most);
+    HIP_TRY(c, hipGetLastError());
+    HIP_TRY(c, hipMemcpyAsync(&got, most, sizeof(got), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    c->bases = (int)got;
     // (the block size may change before a sweep that cannot allocate: counts for whatever few blocks it then has)
     GramPlan plan = gram_plan_of(c, 1);
     plan.acc_rows = M <= kGramBlocks * (uint32_t)kMaxB ? M : 0;
@@ -1149,7 +1153,7 @@ void brr_hip_destroy(brr_hip_ctx* c)
     dfree(c->d_scal); dfree(c->d_hist); dfree(c->d_order); dfree(c->d_u); dfree(c->d_z);
     dfree(c->d_xchg1); dfree(c->d_xchg2); dfree(c->d_ctl); dfree(c->d_counters); dfree(c->d_tmp);
     dfree(c->d_fail); dfree(c->d_sumf); dfree(c->d_num); dfree(c->d_keps); dfree(c->d_cohort);
-    dfree(c->d_cohort_gram); dfree(c->d_counts); dfree(c->d_gram); dfree(c->d_gram_acc);
+    dfree(c->d_cohort_gram); dfree(c->d_counts); dfree(c->d_markers); dfree(c->d_gram); dfree(c->d_gram_acc);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1295,7 +1299,7 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
     uint32_t* d_stage = nullptr;
     uint32_t*& d_cnt = c->d_counts;
     int rc;
-    if ((rc = dalloc(c, &d_stage, stage_words)) || (rc = dalloc(c, &d_cnt, (size_t)4 * M + 2))) {
+    if ((rc = dalloc(c, &d_stage, stage_words)) || (rc = dalloc(c, &d_cnt, (size_t)4 * M + 1))) {
         dfree(d_stage);
         return rc;
     }
@@ -1320,8 +1324,8 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
         cleanup();
         return rc;
     }
-    uint32_t* d_bad = d_cnt + 4 * (size_t)M;   // first unusable marker; 0 if any call is missing
-    if (!hip_ok(hipMemsetAsync(d_bad, 0xFF, 2 * sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
+    uint32_t* d_bad = d_cnt + 4 * (size_t)M;
+    if (!hip_ok(hipMemsetAsync(d_bad, 0xFF, sizeof(uint32_t), c->stream), "hipMemsetAsync") ||
         !hip_ok(hipEventRecord(c->ev0, c->stream), "hipEventRecord"))
         return BRR_HIP_EDEVICE;
     bed_unpack_kernel<<<M, kBedThreads, 0, c->stream>>>(d_stage, cb, N, c->col_words, c->d_dense, d_cnt,
@@ -1344,10 +1348,8 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
             return BRR_HIP_EDEVICE;
         (void)hipEventElapsedTime(&ms_table, c->ev0, c->ev1);
     }
-    uint32_t found[2] = {0xFFFFFFFFu, 0xFFFFFFFFu};
-    if (!hip_ok(hipMemcpy(found, d_bad, sizeof(found), hipMemcpyDeviceToHost), "hipMemcpy")) return BRR_HIP_EDEVICE;
-    const uint32_t bad = found[0];
-    c->missing = found[1] == 0;
+    uint32_t bad = 0xFFFFFFFFu;
+    if (!hip_ok(hipMemcpy(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost), "hipMemcpy")) return BRR_HIP_EDEVICE;
     cleanup();
     c->stats = brr_hip_stats{};
     shape_stats(c);
@@ -1595,10 +1597,10 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
     // Iterations per launch: as many as fit the cohorts' Gram workspaces (together at most eight launches' worth of
     // one context, at least one iteration)
     size_t rows1 = 0;
-    bool missing = false;
+    bool many = false;
     for (uint32_t q = 0; q < n; ++q) {
         rows1 += ctxs[q]->cfg.num_snps;
-        missing = missing || ctxs[q]->missing;
+        many = many || ctxs[q]->bases > 1;
     }
     const uint32_t step = (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, 8 * kGramRowsPerLaunch / rows1));
     const uint32_t steps = (iterations + step - 1) / step;
@@ -1664,7 +1666,7 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
         if (hipError_t e2 = hipGetLastError()) return e2;
         for (uint32_t st = 0; st < steps; ++st) {
             const GramEntry* g = c0->d_cohort_gram + (size_t)st * n;
-            if (missing) gram_cohort_kernel<true><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
+            if (many) gram_cohort_kernel<true><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
             else gram_cohort_kernel<false><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
             if (hipError_t e2 = hipGetLastError()) return e2;
             for (size_t l = 0; l < launches.size(); ++l) {

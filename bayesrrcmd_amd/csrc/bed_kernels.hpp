@@ -34,7 +34,7 @@ __device__ __forceinline__ uint32_t bed_wave_sum_u32(uint32_t v)
 // codes + j * col_words: the column's cb bytes, then zeros. counts[4j + v] =
 // number of individuals i < N whose value is v (pad bits ignored). When stats is
 // not null, stats[4j..4j+3] = {mean, sd, sqrdZ, Zsum} of SparseMarker and the
-// first marker without genotype 1 or 2 calls lowers *bad; bad[1] becomes 0 if any call is missing. eigen = 1: the
+// first marker without genotype 1 or 2 calls lowers *bad. eigen = 1: the
 // EigenSparse statistics instead (missing calls imputed at the mean,
 // eigensparsemarkerbuilder.cpp:41-59), and only a marker without any nonzero
 // call (eigensparsemarker.cpp:60-71) lowers *bad.
@@ -89,7 +89,6 @@ bed_unpack_kernel(const uint32_t* __restrict__ src, uint64_t cb, uint32_t N, uin
         counts[4 * (size_t)j + 1] = n[1];
         counts[4 * (size_t)j + 2] = n[2];
         counts[4 * (size_t)j + 3] = N - n[0] - n[1] - n[2];
-        if (n[1]) bad[1] = 0u;
         if (stats) {
             // SparseMarker::updateStatistics sums the values 1 and 2 in
             // individual order; the sums are integers, so the counts give them

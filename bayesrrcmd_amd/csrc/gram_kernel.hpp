@@ -7,9 +7,11 @@
 // weight (sparsebayesrkernel.cpp:24-27, eigenbayesrkernel.cpp:10-20). They depend on the genotypes and on the
 // marker order alone, so one kernel ahead of the sweep forms them for a whole iteration.
 //
-// With x the dosage (0 for a missing call) and m the missing-call indicator, u and w are linear in (1, x, m),
-// so G follows in FP64 from per-marker sums and the integer products XX = sum x_h x_k, XM = sum x_h m_k,
-// MX = sum m_h x_k, MM = sum m_h m_k, which the i8 matrix cores give exactly.
+// u and w are combinations of 1 and at most three small integers per 2-bit code, the marker's bases: G follows in
+// FP64 from per-marker sums and the products of the bases' integers, which the i8 matrix cores give exactly. Sparse
+// columns have the dosage (0 for a missing call) and the missing-call indicator. Dense columns hold whatever four
+// values the caller's table has, so their bases are found from the table: three values at equal steps share one (the
+// dosages of a standardised column, under any numbering of its codes), every other value that occurs has its own.
 //
 // One workgroup per block of up to 64 markers: the 2-bit codes of the block's and the next block's columns
 // (128 columns) are staged through LDS in chunks of 1,024 individuals, each of the 8 waves takes 128
@@ -31,67 +33,135 @@ constexpr int kGramCols = 2 * kMaxB;              // entries per row: the block'
 constexpr uint32_t kGramChunkBytes = kGramChunk / 4;
 constexpr uint32_t kGramStride = kGramChunkBytes + 16;   // LDS bytes per column: rows start in shifted banks
 
+constexpr int kGramBases = 3;
+// Bytes per 2-bit code of the sparse columns' bases: 0 -> dosage 2, 1 missing, 2 -> 1, 3 -> 0.
+constexpr uint32_t kDosageTab = 0x00010002u;
+constexpr uint32_t kMissingTab = 0x00000100u;
+
+// A marker's share in its row and column entries: value of code v = a + sum_b c[b] (byte v of tab[b]).
+struct GramMarker {
+    double a, c[kGramBases];        // sparse: mean; 1 / sd, the others unused
+    double s[kGramBases];           // sums of the bytes over the individuals
+    uint32_t tab[kGramBases];
+    int n;                          // bases in use
+};
+
 struct GramParams {
     uint32_t N, M, B, iterations;
     int layout;
     uint32_t splits;                // workgroups per block (1: the entries are formed here)
     const uint32_t* codes;          // 2-bit columns, column j at codes + j * col_words
     uint64_t col_words;
-    const uint32_t* counts;         // M x 4: individuals per 2-bit value
-    const double* lut;              // dense: M x 4 by dosage 0, 1, 2, missing
-    const double* stats;            // ragged / EigenSparse: M x 4 {mean, sd, sqrdZ, Zsum}
+    const GramMarker* markers;      // M
+    int bases;                      // most bases of a marker of the context
     const uint32_t* order;          // iterations x M
     double* gram;                   // (iterations x M) rows of kGramCols
     int32_t* acc;                   // splits > 1: products x (iterations x M) x kGramCols, zero between launches
     const uint32_t* gate;           // null, or a word that must be 0 for the launch to run
 };
 
-// A marker's share in its row and column entries.
-struct GramMarker {
-    double x, m;       // sums of x and of the missing calls
-    double a, d, e;    // dense: value = a + d x + e m; sparse: mean, 1 / sd, unused
-};
-
-__device__ __forceinline__ GramMarker gram_marker(const GramParams& p, uint32_t j)
+// The bases of a dense column from its table (by dosage 0, 1, 2, missing) and counts per code. Codes that do not occur
+// have no value: whatever the table holds for them stays out of the sums. Steps count as equal up to the roundings of
+// (dosage - mean) / sd, at most 2^-50 of the largest value.
+__device__ __forceinline__ void dense_bases(const double* lt, const uint32_t* cnt, GramMarker& g)
 {
-    GramMarker g;
-    const uint32_t* c = p.counts + 4 * (size_t)j;
-    g.x = (double)c[2] + 2.0 * (double)c[0];
-    g.m = (double)c[1];
-    if (p.layout == kLayoutDense) {
-        const double* lt = p.lut + 4 * (size_t)j;
-        g.a = lt[0];
-        g.d = 0.5 * (lt[2] - lt[0]);
-        g.e = lt[3] - lt[0];
-    } else {
-        const double* st = p.stats + 4 * (size_t)j;
-        g.a = st[0];
-        g.d = 1.0 / st[1];
-        g.e = 0.0;
+    const double v[4] = {lt[2], lt[3], lt[1], lt[0]};
+    // low, middle and high code of three values at equal steps: a builder's table first
+    constexpr uint32_t kTriple[12] = {0x320, 0x312, 0x310, 0x321, 0x301, 0x302, 0x230, 0x231, 0x132, 0x130, 0x031, 0x012};
+    g.n = 0;
+    uint32_t left = 0u;             // codes that still need a value
+#pragma unroll
+    for (int c = 0; c < 4; ++c) left |= cnt[c] ? 1u << c : 0u;
+    auto value = [&](uint32_t c) { return c == 0u ? v[0] : c == 1u ? v[1] : c == 2u ? v[2] : v[3]; };
+    auto add = [&](double c, uint32_t tab) {
+#pragma unroll
+        for (int b = 0; b < kGramBases; ++b) {
+            g.c[b] = g.n == b ? c : g.c[b];
+            g.tab[b] = g.n == b ? tab : g.tab[b];
+        }
+        ++g.n;
+    };
+    bool steps = false;
+    for (int t = 0; t < 12 && !steps; ++t) {
+        const uint32_t lo = kTriple[t] >> 8, mid = (kTriple[t] >> 4) & 3u, hi = kTriple[t] & 3u;
+        const uint32_t three = 1u << lo | 1u << mid | 1u << hi;
+        if ((left & three) != three) continue;
+        const double x = value(lo), y = value(mid), z = value(hi);
+        if (!(fabs(2.0 * y - x - z) <= 1.7763568394002505e-15 * fmax(fabs(x), fmax(fabs(y), fabs(z))))) continue;   // 2^-49
+        g.a = x;
+        add(0.5 * (z - x), 1u << (8u * mid) | 2u << (8u * hi));
+        left &= ~three;
+        steps = true;
     }
-    return g;
+    if (!steps) {
+        const uint32_t base = left & 8u ? 3u : (uint32_t)__builtin_ctz(left | 8u);
+        g.a = value(base);
+        left &= ~(1u << base);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (((left >> c) & 1u) && v[c] != g.a) add(v[c] - g.a, 1u << (8 * c));
+    if (g.n == 0) g.n = 1;          // (a column of one value)
 }
 
-// The entry's part that does not depend on the products, and each product's factor (0 XX, 1 MX, 2 XM, 3 MM).
+// Every marker's GramMarker, and in *bases (0 before) the most bases of a marker.
+static __global__ void __launch_bounds__(256)
+gram_markers_kernel(uint32_t M, int layout, const double* lut, const double* stats, const uint32_t* counts, GramMarker* out,
+                    uint32_t* bases)
+{
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    if (j >= M) return;
+    GramMarker g;
+    const uint32_t* cnt = counts + 4 * (size_t)j;
+#pragma unroll
+    for (int b = 0; b < kGramBases; ++b) {
+        g.c[b] = 0.0;
+        g.tab[b] = 0u;
+    }
+    if (layout == kLayoutDense) {
+        dense_bases(lut + 4 * (size_t)j, cnt, g);
+    } else {
+        const double* st = stats + 4 * (size_t)j;
+        g.a = st[0];
+        g.c[0] = 1.0 / st[1];
+        g.tab[0] = kDosageTab;
+        g.tab[1] = kMissingTab;
+        g.n = cnt[1] ? 2 : 1;
+    }
+#pragma unroll
+    for (int b = 0; b < kGramBases; ++b) {
+        g.s[b] = 0.0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) g.s[b] += (double)cnt[v] * (double)((g.tab[b] >> (8 * v)) & 255u);
+    }
+    out[j] = g;
+    if (*(volatile uint32_t*)bases < (uint32_t)g.n) atomicMax(bases, (uint32_t)g.n);
+}
+
+// The entry's part that does not depend on the products, and the factor of the product of h's base i and k's base j.
 __device__ __forceinline__ double gram_base(int layout, double N, const GramMarker& h, const GramMarker& k)
 {
     if (layout == kLayoutDense)
-        return N * h.a * k.a + h.a * (k.d * k.x + k.e * k.m) + k.a * (h.d * h.x + h.e * h.m);
-    if (layout == kLayoutEigen) return -h.a * (k.x + k.a * k.m) * h.d;
-    return -h.a * k.x * h.d;
+        return N * h.a * k.a + h.a * (k.c[0] * k.s[0] + k.c[1] * k.s[1] + k.c[2] * k.s[2]) +
+               k.a * (h.c[0] * h.s[0] + h.c[1] * h.s[1] + h.c[2] * h.s[2]);
+    if (layout == kLayoutEigen) return -h.a * (k.s[0] + k.a * k.s[1]) * h.c[0];
+    return -h.a * k.s[0] * h.c[0];
 }
-__device__ __forceinline__ double gram_factor(int layout, int prod, const GramMarker& h, const GramMarker& k)
+__device__ __forceinline__ double gram_factor(int layout, int i, int j, const GramMarker& h, const GramMarker& k)
 {
     if (layout == kLayoutDense) {
-        const double fh = (prod & 1) ? h.e : h.d, fk = (prod & 2) ? k.e : k.d;
+        const double fh = i == 0 ? h.c[0] : i == 1 ? h.c[1] : h.c[2];
+        const double fk = j == 0 ? k.c[0] : j == 1 ? k.c[1] : k.c[2];
         return fh * fk;
     }
-    if (prod == 0) return h.d;
-    if (prod == 1) return h.a * h.d;
-    return (prod == 2 ? k.a : h.a * k.a) * h.d;   // EigenSparse
+    const double d = h.c[0];
+    if (j == 0) return i == 0 ? d : h.a * d;
+    return (i == 0 ? k.a : h.a * k.a) * d;   // EigenSparse
 }
-// Products a layout needs when calls are missing.
-__host__ __device__ constexpr int gram_products(int layout) { return layout == kLayoutRagged ? 2 : 4; }
+// Products of contexts whose markers have up to `bases` bases, product i + bases j from h's base i and k's base j: the
+// ragged dot weight is the dosage alone.
+__host__ __device__ constexpr int gram_weights(int layout, int bases) { return layout == kLayoutRagged ? 1 : bases; }
+__host__ __device__ constexpr int gram_products(int layout, int bases) { return bases * gram_weights(layout, bases); }
 
 typedef int int4v __attribute__((ext_vector_type(4)));
 typedef int int16v __attribute__((ext_vector_type(16)));
@@ -114,12 +184,13 @@ struct GramShared {
     };
     uint32_t id[kGramCols];
     GramMarker mk[kGramCols];
-    int any_miss;
+    uint32_t tab[kGramBases][kGramCols];   // the bases' bytes per code
+    int bases;                             // most bases of the block's and the next block's markers
 };
 
-// Work item `item` (block of an iteration, times its split). kMiss: some call of the context is missing (then the
-// blocks that hold one form the other products too).
-template <bool kMiss>
+// Work item `item` (block of an iteration, times its split). kMany: some marker of the context has more than one base
+// (then the blocks that hold one form the other products too).
+template <bool kMany>
 __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, uint32_t item)
 {
     if (p.gate && __hip_atomic_load(p.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
@@ -132,7 +203,7 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
     const int nb = (int)min(p.B, p.M - b0);
     const int nn = b0 + p.B < p.M ? (int)min(p.B, p.M - b0 - p.B) : 0;
     const uint32_t* order = p.order + (size_t)it * p.M;
-    if (tid == 0) L.any_miss = 0;
+    if (tid == 0) L.bases = 1;
     __syncthreads();
     if (tid < kGramCols) {
         const int k = tid & (kMaxB - 1);
@@ -142,10 +213,14 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
         if (ok) {
             const uint32_t j = order[b0 + (next ? p.B : 0u) + (uint32_t)k];
             L.id[tid] = j;
-            L.mk[tid] = gram_marker(p, j);
-            if (L.mk[tid].m != 0.0) L.any_miss = 1;
+            const GramMarker g = p.markers[j];
+            L.mk[tid] = g;
+#pragma unroll
+            for (int b = 0; b < kGramBases; ++b) L.tab[b][tid] = g.tab[b];
+            if (kMany && g.n > 1) atomicMax(&L.bases, g.n);
         } else {
-            L.mk[tid] = GramMarker{0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int b = 0; b < kGramBases; ++b) L.tab[b][tid] = 0u;
         }
     }
     __syncthreads();
@@ -153,7 +228,9 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
     const uint32_t c0 = (uint32_t)((uint64_t)nchunk * split / p.splits);
     const uint32_t c1 = (uint32_t)((uint64_t)nchunk * (split + 1) / p.splits);
     const uint64_t colb = p.col_words * 4;
-    const int nprod = (kMiss && L.any_miss) ? gram_products(p.layout) : 1;
+    const int nu = kMany ? min(L.bases, p.bases) : 1, nw = gram_weights(p.layout, nu);
+    // individuals past the last one, staged as code 3, of which the sums know nothing
+    const int32_t pads = (int32_t)(nchunk * kGramChunk - p.N);
     const size_t row0 = (size_t)it * p.M + b0;
 
     // 16-byte pieces of a chunk: thread tid takes pieces tid + 512 q: column (tid >> 4) + 32 q, part tid & 15
@@ -169,7 +246,7 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
             if (!ok) pre[q] = make_uint4(~0u, ~0u, ~0u, ~0u);
         }
     };
-    // code 3 (dosage 0, not missing) past the last individual
+    // code 3 past the last individual
     auto stage = [&](uint32_t c, int buf) {
         const int64_t left = (int64_t)p.N - (int64_t)c * kGramChunk - 64 * (int64_t)part;   // individuals of this piece
 #pragma unroll
@@ -187,10 +264,14 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
         }
     };
 
-    constexpr uint32_t kDosage = 0x00010002u;   // byte per code: 0 -> 2, 1 (missing) -> 0, 2 -> 1, 3 -> 0
-    constexpr uint32_t kMissing = 0x00000100u;
-    for (int prod = 0; prod < nprod; ++prod) {
-        const uint32_t ta = (prod & 1) ? kMissing : kDosage, tb = (prod & 2) ? kMissing : kDosage;
+    for (int prod = 0; prod < nu * nw; ++prod) {
+        const int bu = prod % nu, bw = prod / nu;
+        uint32_t tw[4], tu[2];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            tw[g] = L.tab[kMany ? bw : 0][32 * g + (lane & 31)];
+            if (g < 2) tu[g] = kMany ? L.tab[bu][32 * g + (lane & 31)] : tw[g];
+        }
         int16v acc[7];
 #pragma unroll
         for (int t = 0; t < 7; ++t)
@@ -214,8 +295,8 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const uint32_t x = s == 0 ? w[g].x : s == 1 ? w[g].y : s == 2 ? w[g].z : w[g].w;
-                    fb[g] = gram_expand(x, tb);
-                    if (g < 2) fa[g] = kMiss ? gram_expand(x, ta) : fb[g];
+                    fb[g] = gram_expand(x, tw[g]);
+                    if (g < 2) fa[g] = kMany ? gram_expand(x, tu[g]) : fb[g];
                 }
                 acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[0], fb[0], acc[0], 0, 0, 0);
                 acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[0], fb[1], acc[1], 0, 0, 0);
@@ -244,14 +325,15 @@ __device__ __forceinline__ void gram_body(const GramParams& p, GramShared& L, ui
             const bool need = h < nb && (k < kMaxB ? (k > h && k < nb) : k - kMaxB < nn);
             if (!need) continue;
             const size_t at = (row0 + (size_t)h) * kGramCols + (size_t)k;
-            const int32_t s = L.sum[h][k];
+            int32_t s = L.sum[h][k];
+            if (c1 == nchunk) s -= pads * (int32_t)(L.tab[bu][h] >> 24) * (int32_t)(L.tab[bw][k] >> 24);
             if (p.splits > 1) {
-                atomicAdd(p.acc + (size_t)prod * p.iterations * p.M * kGramCols + at, s);
+                atomicAdd(p.acc + (size_t)(bu + p.bases * bw) * p.iterations * p.M * kGramCols + at, s);
             } else {
                 const GramMarker& mh = L.mk[h];
                 const GramMarker& mk = L.mk[k];
                 const double prev = prod == 0 ? gram_base(p.layout, (double)p.N, mh, mk) : p.gram[at];
-                p.gram[at] = prev + gram_factor(p.layout, prod, mh, mk) * (double)s;
+                p.gram[at] = prev + gram_factor(p.layout, bu, bw, mh, mk) * (double)s;
             }
         }
         __syncthreads();
@@ -265,12 +347,12 @@ __device__ __forceinline__ uint32_t gram_item()
     return x8 * n8 + min(x8, r8) + blockIdx.x / 8;
 }
 
-template <bool kMiss>
+template <bool kMany>
 __global__ void __launch_bounds__(kGramThreads)
 gram_kernel(GramParams p)
 {
     __shared__ GramShared L;
-    gram_body<kMiss>(p, L, gram_item());
+    gram_body<kMany>(p, L, gram_item());
 }
 
 // The blocks of several contexts (cohorts) in one launch: item i belongs to the last entry with first <= i.
@@ -279,7 +361,7 @@ struct GramEntry {
     uint32_t first;
 };
 
-template <bool kMiss>
+template <bool kMany>
 __global__ void __launch_bounds__(kGramThreads)
 gram_cohort_kernel(const GramEntry* tab, uint32_t n)
 {
@@ -288,12 +370,12 @@ gram_cohort_kernel(const GramEntry* tab, uint32_t n)
     uint32_t c = 0;
     while (c + 1 < n && item >= tab[c + 1].first) ++c;
     const GramParams p = tab[c].p;
-    gram_body<kMiss>(p, L, item - tab[c].first);
+    gram_body<kMany>(p, L, item - tab[c].first);
 }
 
 // splits > 1: the entries from the shared counts, which are left zero. One workgroup per row.
 static __global__ void __launch_bounds__(kGramCols)
-gram_finish_kernel(GramParams p, int products)
+gram_finish_kernel(GramParams p)
 {
     if (p.gate && __hip_atomic_load(p.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
     const uint32_t it = blockIdx.x / p.M, pos = blockIdx.x % p.M;
@@ -303,21 +385,21 @@ gram_finish_kernel(GramParams p, int products)
     const int h = (int)(pos - b0), k = (int)threadIdx.x;
     if (!(k < kMaxB ? (k > h && k < nb) : k - kMaxB < nn)) return;
     const uint32_t* order = p.order + (size_t)it * p.M;
-    const GramMarker mh = gram_marker(p, order[pos]);
-    const GramMarker mk = gram_marker(p, order[k < kMaxB ? b0 + (uint32_t)k : b0 + p.B + (uint32_t)(k - kMaxB)]);
+    const GramMarker& mh = p.markers[order[pos]];
+    const GramMarker& mk = p.markers[order[k < kMaxB ? b0 + (uint32_t)k : b0 + p.B + (uint32_t)(k - kMaxB)]];
     const size_t at = (size_t)blockIdx.x * kGramCols + (size_t)k;
     double g = gram_base(p.layout, (double)p.N, mh, mk);
-    for (int prod = 0; prod < products; ++prod) {
+    for (int prod = 0; prod < gram_products(p.layout, p.bases); ++prod) {
         int32_t* s = p.acc + (size_t)prod * p.iterations * p.M * kGramCols + at;
-        g += gram_factor(p.layout, prod, mh, mk) * (double)*s;
+        g += gram_factor(p.layout, prod % p.bases, prod / p.bases, mh, mk) * (double)*s;
         *s = 0;
     }
     p.gram[at] = g;
 }
 
-// Individuals per 2-bit value of each column (one workgroup per marker), and whether any call is missing.
+// Individuals per 2-bit value of each column (one workgroup per marker).
 static __global__ void __launch_bounds__(256)
-marker_counts_kernel(const uint32_t* codes, uint64_t col_words, uint32_t N, uint32_t* counts, uint32_t* any_miss)
+marker_counts_kernel(const uint32_t* codes, uint64_t col_words, uint32_t N, uint32_t* counts)
 {
     __shared__ uint32_t red[3][4];
     const uint32_t* col = codes + (size_t)blockIdx.x * col_words;
@@ -344,7 +426,6 @@ marker_counts_kernel(const uint32_t* codes, uint64_t col_words, uint32_t N, uint
         o[1] = n[1];
         o[2] = n[2];
         o[3] = N - n[0] - n[1] - n[2];
-        if (n[1]) *any_miss = 1u;
     }
 }
 

@@ -132,7 +132,9 @@ const char* brr_hip_last_error(const brr_hip_ctx* ctx);
  * starting at bed + j * column_stride (the .bed payload after the 3 magic
  * bytes has column_stride = ceil(N/4)). lut: M x 4 doubles, the standardised
  * column value for dosage 0, 1, 2 and for a missing call, as DenseMarkerBuilder
- * computes them (src/densemarkerbuilder.cpp:43-60). */
+ * computes them (src/densemarkerbuilder.cpp:43-60). Any four values per column
+ * are swept as they stand (brr_dense_read_ppbed numbers its values by first
+ * appearance); tables whose dosage values are at equal steps are the fastest. */
 int brr_hip_upload_dense(brr_hip_ctx* ctx, const uint8_t* bed, uint64_t column_stride,
                          const double* lut);
 
