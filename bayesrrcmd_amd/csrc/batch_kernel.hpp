@@ -434,6 +434,11 @@ bayesr_batch_kernel(BatchParams p)
     }
     if (tid < kMaxK) L.cva[tid] = (tid >= 1 && tid < K) ? p.cva[tid - 1] : 0.0;
     for (int e = tid; e < kBB * kMaxT; e += kThreads) (&L.cd[0][0])[e] = 0.0;
+    // (tiles past the slice hold code 0 throughout: a code that no individual has may have no number in the table)
+    for (int e = tid; e < kBB * kBRow / 4; e += kThreads) {
+        ((uint32_t*)L.blk[0].codes)[e] = 0u;
+        ((uint32_t*)L.blk[1].codes)[e] = 0u;
+    }
     if (tid == 0) L.abort = 0;
     uint32_t rnd = __hip_atomic_load(p.ctl + kCtlRound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned long long n_rounds = 0, n_changes = 0, n_drounds = 0;
