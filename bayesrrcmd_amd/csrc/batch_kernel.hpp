@@ -343,11 +343,11 @@ struct BDraw {
     int sel;
 };
 
-template <int kK, bool kExact>
+template <int kK>
 __device__ __forceinline__ BDraw bdraw_k(const BShared& L, int t, int K, double num, double beta_old, double u,
                                        uint64_t zw, bool zwords)
 {
-    const MixDraw m = mix_draw<kK, kExact>(K, num * num, u, [&](int c) { return L.dg[c][t]; },
+    const MixDraw m = mix_draw<kK, false, true>(K, num * num, u, [&](int c) { return L.dg[c][t]; },
                                    [&](int c) { return L.hk[c][t]; }, [&](int c) { return L.gc[c][t]; });
     BDraw r{beta_old, m.acum0(), m.sel};
     if (r.sel == 0) {
@@ -359,12 +359,14 @@ __device__ __forceinline__ BDraw bdraw_k(const BShared& L, int t, int K, double 
     return r;
 }
 
-// Four components (the usual mixture) as straight-line code, else room for kMaxK.
+// Straight-line code for up to four components and for more; the constants are padded. Draws of 64 traits, 1,000 markers,
+// 3 iterations at N = 2,000, with a run-time K where it is not 4, and padded: K = 2 4.94 / 3.63 ms, 3 6.00 / 4.19, 5 7.77 /
+// 6.03, 8 12.1 / 8.4. A body for each of 2, 3 and 4 spills in the kernels of 25 and 32 tiles (100,000 individuals, 600
+// markers, K = 4: 4.6 -> 6.4 ms).
 __device__ __forceinline__ BDraw bdraw(const BShared& L, int t, int K, double num, double beta_old, double u,
                                        uint64_t zw, bool zwords)
 {
-    return K == 4 ? bdraw_k<4, true>(L, t, K, num, beta_old, u, zw, zwords)
-                  : bdraw_k<kMaxK, false>(L, t, K, num, beta_old, u, zw, zwords);
+    return K <= 4 ? bdraw_k<4>(L, t, K, num, beta_old, u, zw, zwords) : bdraw_k<kMaxK>(L, t, K, num, beta_old, u, zw, zwords);
 }
 
 // -------------------------------------------------------------------- kernel --
@@ -432,6 +434,12 @@ bayesr_batch_kernel(BatchParams p)
             for (int k = 0; k < K; ++k) L.pi[k][t] = sc[SL.pi() + k];
         }
     }
+    for (int e = tid; e < kMaxK * kMaxT; e += kThreads)   // (mix_draw's padding, for the components past the last)
+        if (const int k = e / kMaxT, t = e % kMaxT; k >= K) {
+            L.gc[k][t] = -__builtin_inf();
+            L.dg[k][t] = kPadDg;
+            L.hk[k][t] = 0.0;
+        }
     if (tid < kMaxK) L.cva[tid] = (tid >= 1 && tid < K) ? p.cva[tid - 1] : 0.0;
     for (int e = tid; e < kBB * kMaxT; e += kThreads) (&L.cd[0][0])[e] = 0.0;
     // (tiles past the slice hold code 0 throughout: a code that no individual has may have no number in the table)

@@ -57,10 +57,15 @@ struct MixDraw {
 // wave whenever one lane needed them). u <= acum is decided as u sum_i e_i <= e_0 + .. + e_c, so that no
 // reciprocal stands before the choice. kExact: K == kK, so that the exponentials are straight-line code and
 // overlap (with a run-time K each became a branch of its own: 900 cycles a draw on one wave instead of 300).
-template <int kK, bool kExact, class Dg, class Hk, class Lc>
+// kPad: straight-line code for any K <= kK. The constants of components K .. kK - 1 are kPadDg, 0 and -infinity: they add
+// exp(kPadDg) to a sum of at least 1, which leaves its bits as they are, or 0, and are never drawn.
+constexpr double kPadDg = -300.0;
+
+template <int kK, bool kExact, bool kPad = false, class Dg, class Hk, class Lc>
 __device__ __forceinline__ MixDraw mix_draw(int Krt, double n2, double u, Dg&& dg, Hk&& hk, Lc&& lc)
 {
-    const int K = kExact ? kK : Krt;
+    const int Kg = kExact ? kK : Krt;          // components that the guards look at
+    const int K = kPad ? kK : Kg;
     double x[kK];
     bool far = false;
 #pragma unroll
@@ -89,7 +94,7 @@ __device__ __forceinline__ MixDraw mix_draw(int Krt, double n2, double u, Dg&& d
             for (int c = 0; c < kK; ++c)
 #pragma unroll
                 for (int i = 1; i < kK; ++i)
-                    if (i != c && c < K && i < K && fabs(x[i] - x[c]) > 700.0) guard |= 1u << c;
+                    if (i != c && c < Kg && i < Kg && fabs(x[i] - x[c]) > 700.0) guard |= 1u << c;
 #pragma unroll
             for (int c = 0; c < kK; ++c)
                 if (c < K) x[c] = x[c] - m;
