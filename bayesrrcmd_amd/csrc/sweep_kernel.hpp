@@ -334,7 +334,16 @@ struct IntC {
     static constexpr int value = N;
 };
 
-// f(IntC<kK>, BoolC<exact>) for K mixture components: exact for the usual sizes, else room for kMaxK
+// Constant c of a group's K, or mix_draw's padding.
+template <bool kExact>
+__device__ __forceinline__ double padded(const double* of, int c, int K, double pad)
+{
+    const double v = of[kExact || c < K ? c : K - 1];
+    return kExact || c < K ? v : pad;
+}
+
+// f(IntC<kK>, BoolC<exact>) for K mixture components: exact for the usual sizes, else kMaxK with padded constants (lists of
+// N = 20,000, M = 2,000, two iterations with K = 5: 1.86 ms with a run-time K, 1.76 padded)
 template <class F>
 __device__ __forceinline__ void with_components(int K, F&& f)
 {
@@ -1582,9 +1591,11 @@ __device__ __forceinline__ void sweep_body(const SweepParams& p, Shared<R>& L, R
                                 num = beta_old * (dN - 1.0) - mean * eS * rsd + dotk * rsd;
                             }
                             numk = num;
-                            const MixDraw md = mix_draw<kK, decltype(exact)::value>(
-                                K, num * num, L.uu[k], [&](int c) { return L.gdg[g * K + c]; },
-                                [&](int c) { return L.ghk[g * K + c]; }, [&](int c) { return L.gc[g * K + c]; });
+                            constexpr bool ex = decltype(exact)::value;
+                            const MixDraw md = mix_draw<kK, ex, !ex>(
+                                K, num * num, L.uu[k], [&](int c) { return padded<ex>(L.gdg + g * K, c, K, kPadDg); },
+                                [&](int c) { return padded<ex>(L.ghk + g * K, c, K, 0.0); },
+                                [&](int c) { return padded<ex>(L.gc + g * K, c, K, -__builtin_inf()); });
                             sel = md.sel;
                             acum0 = md.acum0();
                             // the beta draw of the chosen component (BayesRBase.cpp:343-352)
