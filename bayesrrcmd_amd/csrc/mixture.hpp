@@ -45,7 +45,9 @@ __device__ __forceinline__ double rcp_draw(double s)
 struct MixDraw {
     double e0, s;   // the zero component's probability (acum of processColumn) is e0 / s
     int sel;        // the component drawn; -1: none (u beyond the guarded sum)
-    __device__ __forceinline__ double acum0() const { return e0 * rcp_draw(s); }
+    __device__ __forceinline__ double acum0() const { return prob0(e0, s); }
+    // (a guarded component stays at 0 where the sum is no number: num^2 past the largest double)
+    __device__ static __forceinline__ double prob0(double e0, double s) { return e0 == 0.0 ? 0.0 : e0 * rcp_draw(s); }
 };
 
 // The draw from n2 = num^2 and the uniform u. Constants per component c (any callables):

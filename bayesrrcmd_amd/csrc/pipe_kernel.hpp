@@ -603,7 +603,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
             }
             if (act0) {
                 L.ob[par][k] = bnew;
-                L.oa[par][k] = e0 * rcp_draw(es);
+                L.oa[par][k] = MixDraw::prob0(e0, es);
                 L.on[par][k] = numk;
                 L.os[par][k] = sel;
             }
