@@ -533,11 +533,10 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
             while (start < nb) {
                 const bool act = lane >= start && act0;
                 const double num = dense ? dot + base : __builtin_fma(dot - w0 * eS, w3, base);
-                constexpr bool ex = decltype(exact)::value;
-                const MixDraw md = mix_draw<kK, ex, !ex>(
-                    K, num * num, u, [&](int c) { return kRegs ? dg[kRegs ? c : 0] : padded<ex>(L.gdg + gk, c, K, kPadDg); },
-                    [&](int c) { return kRegs ? hk[kRegs ? c : 0] : padded<ex>(L.ghk + gk, c, K, 0.0); },
-                    [&](int c) { return kRegs ? lc[kRegs ? c : 0] : padded<ex>(L.gc + gk, c, K, -__builtin_inf()); });
+                const MixDraw md = mix_draw<kK, decltype(exact)::value>(
+                    K, num * num, u, [&](int c) { return kRegs ? dg[kRegs ? c : 0] : L.gdg[gk + c]; },
+                    [&](int c) { return kRegs ? hk[kRegs ? c : 0] : L.ghk[gk + c]; },
+                    [&](int c) { return kRegs ? lc[kRegs ? c : 0] : L.gc[gk + c]; });
                 // the beta draw of the chosen component (BayesRBase.cpp:343-352)
                 double bn = md.sel == 0 ? 0.0 : bo;
                 if constexpr (kRegs) {
