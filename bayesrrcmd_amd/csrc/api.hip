@@ -78,6 +78,7 @@ struct brr_hip_ctx {
     uint32_t* d_counts = nullptr;
     GramMarker* d_markers = nullptr;
     int bases = 1;
+    bool many = false;           // some marker has another base than the dosage
     double* d_gram = nullptr;
     size_t gram_cap = 0;         // rows
     int32_t* d_gram_acc = nullptr;
@@ -745,7 +746,7 @@ hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, ui
         if (rows > c->gram_cap || (splits > 1 && rows * gram_products_of(c) > c->gram_acc_cap)) return hipErrorInvalidValue;
         GramParams g = gram_params(c, p.order, iterations, splits, p.gate);
         const uint32_t items = iterations * ((g.M + g.B - 1) / g.B) * g.splits;
-        if (c->bases > 1) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
+        if (c->many) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
         else gram_kernel<false><<<items, kGramThreads, 0, c->stream>>>(g);
         if (hipError_t e = hipGetLastError()) return e;
         if (g.splits > 1) {
@@ -771,15 +772,16 @@ int prepare_pipe(brr_hip_ctx* c, bool counted)
         HIP_TRY(c, hipGetLastError());
     }
     if ((rc = dalloc(c, &c->d_markers, (size_t)M))) return rc;
-    uint32_t* most = c->d_counts + 4 * (size_t)M;
+    uint32_t* kind = c->d_counts + 4 * (size_t)M;
     uint32_t got = 0;
-    HIP_TRY(c, hipMemsetAsync(most, 0, sizeof(uint32_t), c->stream));
+    HIP_TRY(c, hipMemsetAsync(kind, 0, sizeof(uint32_t), c->stream));
     gram_markers_kernel<<<(M + 255) / 256, 256, 0, c->stream>>>(M, c->layout, c->d_lut, c->d_stats, c->d_counts,
-                                                                c->d_markers, most);
+                                                                c->d_markers, kind);
     HIP_TRY(c, hipGetLastError());
-    HIP_TRY(c, hipMemcpyAsync(&got, most, sizeof(got), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(&got, kind, sizeof(got), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    c->bases = (int)got;
+    c->bases = (int)(got >> 1);
+    c->many = got > 2u;
     // (the block size may change before a sweep that cannot allocate: counts for whatever few blocks it then has)
     GramPlan plan = gram_plan_of(c, 1);
     plan.acc_rows = M <= kGramBlocks * (uint32_t)kMaxB ? M : 0;
@@ -1600,7 +1602,7 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
     bool many = false;
     for (uint32_t q = 0; q < n; ++q) {
         rows1 += ctxs[q]->cfg.num_snps;
-        many = many || ctxs[q]->bases > 1;
+        many = many || ctxs[q]->many;
     }
     const uint32_t step = (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, 8 * kGramRowsPerLaunch / rows1));
     const uint32_t steps = (iterations + step - 1) / step;

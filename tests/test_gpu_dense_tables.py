@@ -42,6 +42,22 @@ def free_tables(pr, seed, three=False):
     return pr.bed, (lut - x.mean(axis=1)[:, None]) / x.std(axis=1, ddof=1)[:, None]
 
 
+def two_dosages(pr, seed):
+    """Columns in which one dosage does not occur, beside some with one value only; a builder's tables."""
+    d = np.abs(spec_dosage(pr.bed, pr.n))
+    for j in range(pr.m):
+        a, b = [(2, 1), (0, 1), (1, 2)][j % 3]
+        d[j][d[j] == a] = b
+    codes = np.zeros((pr.m, 4 * pr.bed.shape[1]), dtype=np.uint8)
+    codes[:, :pr.n] = np.array([3, 2, 0], dtype=np.uint8)[d]
+    q = codes.reshape(pr.m, -1, 4)
+    bed = q[..., 0] | q[..., 1] << 2 | q[..., 2] << 4 | q[..., 3] << 6
+    lut = brr.build_dense(bed, pr.n)
+    lut[0] = 0.0
+    lut[~np.isfinite(lut).all(axis=1)] = 0.0      # (columns of one value have no standard deviation)
+    return bed, lut
+
+
 def pair(pr, bed, lut, **kw):
     o = orc.OracleProblem(pr.n, pr.m, orc.DENSE, 4, 1, S4, bed=bed, lut=lut)
     o.init(pr.y, 11)
@@ -58,11 +74,12 @@ def pair(pr, bed, lut, **kw):
 
 # (N, M, block): Gram launches split over the individuals and not, blocks with a next one and without
 @pytest.mark.parametrize("n,m,block", [(700, 61, 0), (1025, 129, 33), (5001, 200, 0), (400, 8300, 0)])
-@pytest.mark.parametrize("tables", ["ppbed", "ppbed-missing", "three", "four"])
+@pytest.mark.parametrize("tables", ["ppbed", "ppbed-missing", "three", "four", "two"])
 def test_sweep_follows_the_table(gpu_lib, n, m, block, tables):
     miss = 0.0 if tables == "ppbed" else 0.03
     pr = make_problem(n, m, seed=n + m, causal_frac=0.05, maf=(0.1, 0.5), miss=miss)
-    bed, lut = ppbed(pr) if tables.startswith("ppbed") else free_tables(pr, n, tables == "three")
+    bed, lut = (ppbed(pr) if tables.startswith("ppbed") else two_dosages(pr, n) if tables == "two" else
+                free_tables(pr, n, tables == "three"))
     o, h = pair(pr, bed, lut, block_markers=block)
     order = np.arange(m, dtype=np.uint32)
     for it in range(2):
