@@ -79,6 +79,8 @@ struct brr_hip_ctx {
     GramMarker* d_markers = nullptr;
     int bases = 1;
     bool many = false;           // some marker has another base than the dosage
+    bool counted = false;        // d_counts and ..
+    bool have_shares = false;    // .. d_markers are those of the columns held
     double* d_gram = nullptr;
     size_t gram_cap = 0;         // rows
     int32_t* d_gram_acc = nullptr;
@@ -692,37 +694,59 @@ int launch_fn(brr_hip_ctx* c, const void* fn, void* param, uint32_t threads = kT
 
 int gram_products_of(const brr_hip_ctx* c) { return gram_products(c->layout, c->bases); }
 
-// The workspace of `plan`'s launches: its Gram rows, and the shared counts if its blocks are split.
-int gram_reserve(brr_hip_ctx* c, const GramPlan& plan)
+// The shared counts of `rows` rows, clear. False if the device has no room for them (blocks are then not split).
+bool gram_reserve_acc(brr_hip_ctx* c, size_t rows)
 {
-    int rc;
-    if (c->gram_cap < plan.rows) {
-        c->gram_cap = 0;
-        if ((rc = dalloc(c, &c->d_gram, plan.rows * kGramCols))) return rc;
-        c->gram_cap = plan.rows;
+    const size_t acc = rows * gram_products_of(c);
+    if (c->gram_acc_cap >= acc) return true;
+    c->gram_acc_cap = 0;
+    if (dalloc(c, &c->d_gram_acc, acc * kGramCols) ||
+        hipMemsetAsync(c->d_gram_acc, 0, sizeof(int32_t) * acc * kGramCols, c->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
     }
-    const size_t acc = plan.acc_rows * gram_products_of(c);
-    if (c->gram_acc_cap < acc) {
-        c->gram_acc_cap = 0;
-        if ((rc = dalloc(c, &c->d_gram_acc, acc * kGramCols))) return rc;
-        HIP_TRY(c, hipMemsetAsync(c->d_gram_acc, 0, sizeof(int32_t) * acc * kGramCols, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));   // (cohorts use it on another context's stream)
-        c->gram_acc_cap = acc;
+    c->gram_acc_cap = acc;
+    return true;
+}
+
+// Room for `rows` Gram rows, or for at least kGramRowsLeast where the device has no more.
+int gram_reserve_rows(brr_hip_ctx* c, size_t rows)
+{
+    while (c->gram_cap < rows) {
+        c->gram_cap = 0;
+        const int rc = dalloc(c, &c->d_gram, rows * kGramCols);
+        if (!rc) {
+            c->gram_cap = rows;
+        } else {
+            (void)hipGetLastError();
+            if (rows <= kGramRowsLeast) return rc;
+            rows = std::max(rows / 2, kGramRowsLeast);
+        }
     }
     return BRR_HIP_OK;
 }
 
-GramPlan gram_plan_of(const brr_hip_ctx* c, uint32_t iterations)
+GramPlan gram_plan_of(const brr_hip_ctx* c, uint32_t iterations, size_t most)
 {
-    return gram_plan(c->cfg.num_inds, c->cfg.num_snps, c->B, iterations);
+    return gram_plan(c->cfg.num_inds, c->cfg.num_snps, c->B, iterations, most);
 }
 
-GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t iterations, uint32_t splits,
-                       const uint32_t* gate)
+// How `iterations` iterations run in the workspace that could be had for them.
+int gram_reserve(brr_hip_ctx* c, uint32_t iterations, GramPlan* plan)
+{
+    *plan = gram_plan_of(c, iterations, kGramRowsMost);
+    if (int rc = gram_reserve_rows(c, plan->rows)) return rc;
+    if (c->gram_cap < plan->rows) *plan = gram_plan_of(c, iterations, c->gram_cap);
+    if (plan->acc_rows && !gram_reserve_acc(c, plan->acc_rows)) plan->splits = 1;
+    return BRR_HIP_OK;
+}
+
+// The Gram rows of a launch's iterations `p`.
+GramParams gram_params(const brr_hip_ctx* c, const SweepParams& p, uint32_t iterations, uint32_t splits)
 {
     GramParams g{};
-    g.N = c->cfg.num_inds;
-    g.M = c->cfg.num_snps;
+    g.N = p.N;
+    g.M = p.M;
     g.B = c->B;
     g.iterations = iterations;
     g.layout = c->layout;
@@ -731,10 +755,10 @@ GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t ite
     g.codes = c->d_dense;
     g.col_words = c->col_words;
     g.markers = c->d_markers;
-    g.order = order;
+    g.order = p.order;
     g.gram = c->d_gram;
     g.acc = c->d_gram_acc;
-    g.gate = gate;
+    g.gate = p.gate;
     return g;
 }
 
@@ -742,9 +766,9 @@ GramParams gram_params(const brr_hip_ctx* c, const uint32_t* order, uint32_t ite
 hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, uint32_t iterations, uint32_t splits)
 {
     if (p.mode == kModeSweep || p.mode == kModeChain) {
-        const size_t rows = (size_t)iterations * c->cfg.num_snps;
+        const size_t rows = (size_t)iterations * p.M;
         if (rows > c->gram_cap || (splits > 1 && rows * gram_products_of(c) > c->gram_acc_cap)) return hipErrorInvalidValue;
-        GramParams g = gram_params(c, p.order, iterations, splits, p.gate);
+        GramParams g = gram_params(c, p, iterations, splits);
         const uint32_t items = iterations * ((g.M + g.B - 1) / g.B) * g.splits;
         if (c->many) gram_kernel<true><<<items, kGramThreads, 0, c->stream>>>(g);
         else gram_kernel<false><<<items, kGramThreads, 0, c->stream>>>(g);
@@ -759,17 +783,34 @@ hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, ui
     return hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream);
 }
 
-// The markers' share in the Gram entries, from the columns just stored, and the Gram workspace of a sweep (so that
-// sweeps allocate nothing). `counted`: the caller has the counts per code in place.
-int prepare_pipe(brr_hip_ctx* c, bool counted)
+// The launches of `plan`: its iterations, or the parts of each.
+hipError_t enqueue_plan(brr_hip_ctx* c, const SweepKernel& k, const SweepParams& p, const GramPlan& plan)
 {
-    if (c->T || c->bw || !c->codes) return BRR_HIP_OK;
+    for (uint32_t it = 0; it < plan.total; it += plan.step)
+        for (uint32_t part = 0; part < plan.parts; ++part) {
+            SweepParams q = p;
+            q.M = plan.markers(p.M, part);
+            q.part = (part ? 1u : 0u) | (part + 1 < plan.parts ? 2u : 0u);
+            q.iterations = plan.iterations(it);
+            q.iter_base = p.iter_base + it;
+            q.order = p.order + (size_t)it * p.M + (size_t)part * plan.part;
+            q.hist = p.hist ? p.hist + (size_t)it * (4 + p.G) : nullptr;
+            if (hipError_t e = enqueue_pipe(c, k, q, q.iterations, plan.splits)) return e;
+        }
+    return hipSuccess;
+}
+
+// The markers' share in the Gram entries, once for the columns held.
+int prepare_shares(brr_hip_ctx* c)
+{
+    if (c->have_shares) return BRR_HIP_OK;
     int rc;
     const uint32_t M = c->cfg.num_snps;
-    if (!counted) {
+    if (!c->counted) {
         if ((rc = dalloc(c, &c->d_counts, (size_t)4 * M + 1))) return rc;
         marker_counts_kernel<<<M, 256, 0, c->stream>>>(c->d_dense, c->col_words, c->cfg.num_inds, c->d_counts);
         HIP_TRY(c, hipGetLastError());
+        c->counted = true;
     }
     if ((rc = dalloc(c, &c->d_markers, (size_t)M))) return rc;
     uint32_t* kind = c->d_counts + 4 * (size_t)M;
@@ -782,10 +823,24 @@ int prepare_pipe(brr_hip_ctx* c, bool counted)
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     c->bases = (int)(got >> 1);
     c->many = got > 2u;
-    // (the block size may change before a sweep that cannot allocate: counts for whatever few blocks it then has)
-    GramPlan plan = gram_plan_of(c, 1);
-    plan.acc_rows = M <= kGramBlocks * (uint32_t)kMaxB ? M : 0;
-    return gram_reserve(c, plan);
+    c->have_shares = true;
+    return BRR_HIP_OK;
+}
+
+// At the end of the set-up calls: a context whose sweeps are pipelined gets what they need, so that later sweeps
+// allocate nothing. Where the device has no room the call succeeds all the same; the sweep itself then says so.
+void prepare_sweeps(brr_hip_ctx* c)
+{
+    if (!c->have_markers || !c->have_model || c->T || c->bw || !kernel_of(c).pipe) return;
+    const std::string err = c->err;
+    GramPlan plan;
+    if (prepare_shares(c) || gram_reserve(c, 1, &plan)) {
+        (void)hipGetLastError();
+    } else if (c->cfg.num_snps <= kGramBlocks * (uint32_t)kMaxB) {
+        // (the block size may change before a sweep that cannot allocate: counts for whatever few blocks it then has)
+        (void)gram_reserve_acc(c, c->cfg.num_snps);
+    }
+    c->err = err;
 }
 
 int launch(brr_hip_ctx* c, SweepParams& p)
@@ -796,21 +851,11 @@ int launch(brr_hip_ctx* c, SweepParams& p)
                                        "(ragged_storage 0 or 2)");
     const SweepKernel k = kernel_of(c);
     if (!k.pipe) return launch_fn(c, k.fn, &p, k.threads);
-    const GramPlan plan = gram_plan_of(c, p.mode == kModeChain ? p.iterations : 1u);
-    if (int rc = gram_reserve(c, plan)) return rc;
-    if (p.mode != kModeChain) return run_launches(c, [&] { return enqueue_pipe(c, k, p, 1, plan.splits); });
-    // a chain in launches of as many iterations as the Gram workspace holds
-    return run_launches(c, [&] {
-        for (uint32_t it = 0; it < plan.total; it += plan.step) {
-            SweepParams q = p;
-            q.iterations = plan.iterations(it);
-            q.iter_base = p.iter_base + it;
-            q.order = p.order + (size_t)it * p.M;
-            q.hist = p.hist ? p.hist + (size_t)it * (4 + p.G) : nullptr;
-            if (hipError_t e = enqueue_pipe(c, k, q, q.iterations, plan.splits)) return e;
-        }
-        return hipSuccess;
-    });
+    if (p.mode != kModeSweep && p.mode != kModeChain) return run_launches(c, [&] { return enqueue_pipe(c, k, p, 1, 1); });
+    GramPlan plan;
+    if (int rc = prepare_shares(c)) return rc;
+    if (int rc = gram_reserve(c, p.mode == kModeChain ? p.iterations : 1u, &plan)) return rc;
+    return run_launches(c, [&] { return enqueue_plan(c, k, p, plan); });
 }
 
 // Batched contexts: the same launch with the sweep-mode / chain-mode fields of p.
@@ -1129,11 +1174,14 @@ int brr_hip_create(const brr_hip_config* cfg, brr_hip_ctx** out)
         brr_hip_destroy(c);
         return BRR_HIP_EDEVICE;
     }
-    (void)hipMemsetAsync(c->d_eps, 0, sizeof(double) * N * Tn, c->stream);
-    (void)hipMemsetAsync(c->d_beta, 0, sizeof(double) * M * Tn, c->stream);
-    (void)hipMemsetAsync(c->d_comp, 0, sizeof(int32_t) * M * Tn, c->stream);
-    (void)hipMemsetAsync(c->d_acum, 0, sizeof(double) * M * Tn, c->stream);
-    (void)hipMemsetAsync(c->d_scal, 0, sizeof(double) * SL.size() * Tn, c->stream);
+    // (on the null stream: a context's first .bed decode is 8 us slower after clearing on its own stream; waited for, since
+    // later copies go through that stream)
+    (void)hipMemset(c->d_eps, 0, sizeof(double) * N * Tn);
+    (void)hipMemset(c->d_beta, 0, sizeof(double) * M * Tn);
+    (void)hipMemset(c->d_comp, 0, sizeof(int32_t) * M * Tn);
+    (void)hipMemset(c->d_acum, 0, sizeof(double) * M * Tn);
+    (void)hipMemset(c->d_scal, 0, sizeof(double) * SL.size() * Tn);
+    (void)hipStreamSynchronize(nullptr);
     c->x1_cap = c->x1_words;
     if (reset_exchange(c) != BRR_HIP_OK) { brr_hip_destroy(c); return BRR_HIP_EDEVICE; }
     *out = c;
@@ -1179,6 +1227,7 @@ int brr_hip_upload_dense(brr_hip_ctx* c, const uint8_t* bed, uint64_t column_str
     HIP_TRY(c, hipSetDevice(c->device));
     c->col_bytes = col_bytes;
     c->col_words = (col_bytes + 15) / 16 * 4;   // 16-byte aligned columns
+    c->counted = c->have_shares = false;
     int rc = dalloc(c, &c->d_dense, (size_t)c->col_words * M);
     if (rc) return rc;
     if ((rc = dalloc(c, &c->d_lut, (size_t)4 * M))) return rc;
@@ -1186,7 +1235,6 @@ int brr_hip_upload_dense(brr_hip_ctx* c, const uint8_t* bed, uint64_t column_str
     HIP_TRY(c, hipMemcpy2D(c->d_dense, c->col_words * 4, bed, column_stride, col_bytes, M,
                            hipMemcpyHostToDevice));
     HIP_TRY(c, hipMemcpy(c->d_lut, lut, sizeof(double) * 4 * M, hipMemcpyHostToDevice));
-    if (!c->bw && (rc = prepare_pipe(c, false))) return rc;
     c->have_markers = true;
     if (c->bw) {
         // a BayesW context takes its layout from the markers it is given
@@ -1194,6 +1242,7 @@ int brr_hip_upload_dense(brr_hip_ctx* c, const uint8_t* bed, uint64_t column_str
         c->cfg.layout = BRR_HIP_LAYOUT_DENSE_2BIT;
         c->have_model = false;   // sum_failure depends on the columns
     }
+    prepare_sweeps(c);
     return BRR_HIP_OK;
 }
 
@@ -1230,6 +1279,7 @@ int brr_hip_upload_ragged(brr_hip_ctx* c, const int32_t* ones, const uint64_t* o
         }
     }
     HIP_TRY(c, hipSetDevice(c->device));
+    c->counted = c->have_shares = false;
     int rc;
     if ((rc = dalloc(c, &c->d_ones, n1)) || (rc = dalloc(c, &c->d_twos, n2)) ||
         (rc = dalloc(c, &c->d_miss, nm)) || (rc = dalloc(c, &c->d_ones_off, M + 1)) ||
@@ -1270,9 +1320,9 @@ int brr_hip_upload_ragged(brr_hip_ctx* c, const int32_t* ones, const uint64_t* o
         // BayesR kernels too, once the lists are gone)
         dfree(c->d_ones); dfree(c->d_twos); dfree(c->d_miss);
     }
-    if ((rc = prepare_pipe(c, false))) return rc;
     c->have_markers = true;
     c->have_model = c->have_model && !c->bw;   // sum_failure depends on the columns
+    prepare_sweeps(c);
     return BRR_HIP_OK;
 }
 
@@ -1293,7 +1343,7 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
     if (N < 2 || M == 0) return fail(c, BRR_HIP_EINVAL, "need N >= 2 and M >= 1");
     HIP_TRY(c, hipSetDevice(c->device));
     const bool dense = layout == BRR_HIP_LAYOUT_DENSE_2BIT;
-    c->have_markers = false;
+    c->have_markers = c->counted = c->have_shares = false;
     // the packed payload, with 32 zero bytes past its end for the unpacker's
     // five-word reads
     const uint64_t payload = cb * M;
@@ -1365,13 +1415,15 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
                                            (layout == BRR_HIP_LAYOUT_EIGEN_SPARSE ? " has no nonzero call"
                                                                                   : " has no genotype 1 or 2 calls"));
     c->codes = true;
-    if ((rc = prepare_pipe(c, true))) return rc;
+    c->counted = !c->T && !c->bw;
+    if (!c->counted) dfree(c->d_counts);
     if (c->bw) {
         c->layout = dense ? kLayoutDense : kLayoutRagged;
         c->cfg.layout = (uint32_t)layout;
         c->have_model = false;   // sum_failure depends on the columns
     }
     c->have_markers = true;
+    prepare_sweeps(c);
     return BRR_HIP_OK;
 }
 
@@ -1393,6 +1445,10 @@ int brr_hip_set_async(brr_hip_ctx* c, uint32_t window)
     if (window && c->f32) return fail(c, BRR_HIP_EINVAL, "the FP32 residual mode runs the sequential sweep only");
     c->async = window ? 1u : 0u;
     c->B = window ? window : c->B_seq;
+    if (!window) {
+        HIP_TRY(c, hipSetDevice(c->device));
+        prepare_sweeps(c);
+    }
     return BRR_HIP_OK;
 }
 
@@ -1417,6 +1473,8 @@ int brr_hip_set_precision(brr_hip_ctx* c, int precision, uint32_t refresh_marker
         return fail(c, BRR_HIP_EINVAL, "refresh interval must be 1..1024 markers");
     c->f32 = true;
     c->refresh_markers = refresh_markers;
+    HIP_TRY(c, hipSetDevice(c->device));
+    prepare_sweeps(c);
     return BRR_HIP_OK;
 }
 
@@ -1424,7 +1482,9 @@ int brr_hip_set_launch(brr_hip_ctx* c, uint32_t workgroups, uint32_t block_marke
 {
     if (int k = need_kind(c, false)) return k;
     HIP_TRY(c, hipSetDevice(c->device));
-    return configure_shape(c, workgroups, block_markers);
+    const int rc = configure_shape(c, workgroups, block_markers);
+    if (!rc) prepare_sweeps(c);
+    return rc;
 }
 
 int brr_hip_autotune(brr_hip_ctx* c, uint64_t seed, uint32_t iterations, brr_hip_tune_entry* table,
@@ -1606,11 +1666,8 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
     }
     const uint32_t step = (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, 8 * kGramRowsPerLaunch / rows1));
     const uint32_t steps = (iterations + step - 1) / step;
-    for (uint32_t q = 0; q < n; ++q) {
-        GramPlan plan{};   // (no block is split: the cohorts' blocks fill a launch together)
-        plan.rows = (size_t)step * ctxs[q]->cfg.num_snps;
-        if ((rc = gram_reserve(ctxs[q], plan))) return fail(c0, rc, ctxs[q]->err);
-    }
+    for (uint32_t q = 0; q < n; ++q)
+        if ((rc = gram_reserve_rows(ctxs[q], (size_t)step * ctxs[q]->cfg.num_snps))) return fail(c0, rc, ctxs[q]->err);
     HIP_TRY(c0, hipDeviceSynchronize());
     // parameter blocks by step in launch order, on the device; the Gram entries of all cohorts of a step in one launch
     std::vector<SweepParams> packed;
@@ -1628,7 +1685,7 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
                 p.hist += (size_t)it0 * (4 + p.G);
                 p.gram = c->d_gram;
                 packed.push_back(p);
-                GramEntry g{gram_params(c, p.order, its, 1, nullptr), gram_items[st]};
+                GramEntry g{gram_params(c, p, its, 1), gram_items[st]};
                 grams.push_back(g);
                 gram_items[st] += its * ((g.p.M + g.p.B - 1) / g.p.B);
             }
@@ -1917,6 +1974,7 @@ int brr_hip_set_model(brr_hip_ctx* c, const brr_hip_model* m)
     c->model.cva = c->cva.data();
     HIP_TRY(c, hipMemcpy(c->d_cva, m->cva, sizeof(double) * G * (K - 1), hipMemcpyHostToDevice));
     c->have_model = true;
+    prepare_sweeps(c);
     return BRR_HIP_OK;
 }
 
@@ -2049,6 +2107,8 @@ int brr_hip_sweep_noalloc(brr_hip_ctx* c, const uint32_t* d_order, const double*
                                        "(ragged_storage 0 or 2)");
     const SweepKernel k = kernel_of(c);
     if (!k.fn) return fail(c, BRR_HIP_EINVAL, "unsupported slice size");
+    if (k.pipe && (!c->have_shares || c->gram_cap < (size_t)std::min(M, c->B)))
+        return fail(c, BRR_HIP_ENOMEM, "brr_hip_sweep_noalloc: the device had no room for the context's Gram rows at set-up");
     HIP_TRY(c, hipSetDevice(c->device));
     uint64_t* base = nullptr;
     if ((rc = scratch_for(c, &base))) return rc;
@@ -2071,7 +2131,9 @@ int brr_hip_sweep_noalloc(brr_hip_ctx* c, const uint32_t* d_order, const double*
     p.refresh_blocks = std::max(1u, c->refresh_markers / c->B);
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     if (k.pipe) {
-        HIP_TRY(c, enqueue_pipe(c, k, p, 1, gram_plan_of(c, 1).splits));   // (its workspace was allocated with the markers)
+        GramPlan plan = gram_plan_of(c, 1, std::min(c->gram_cap, kGramRowsMost));
+        if (plan.acc_rows * gram_products_of(c) > c->gram_acc_cap) plan.splits = 1;
+        HIP_TRY(c, enqueue_plan(c, k, p, plan));
     } else {
         void* args[] = {&p};
         HIP_TRY(c, hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream));
@@ -2344,10 +2406,11 @@ int brr_hip_bw_create(const brr_hip_bw_config* cfg, brr_hip_ctx** out)
         brr_hip_destroy(c);
         return BRR_HIP_EDEVICE;
     }
-    (void)hipMemsetAsync(c->d_eps, 0, sizeof(double) * N, c->stream);
-    (void)hipMemsetAsync(c->d_beta, 0, sizeof(double) * M, c->stream);
-    (void)hipMemsetAsync(c->d_comp, 0, sizeof(int32_t) * M, c->stream);
-    (void)hipMemsetAsync(c->d_scal, 0, sizeof(double) * nscal, c->stream);
+    (void)hipMemset(c->d_eps, 0, sizeof(double) * N);
+    (void)hipMemset(c->d_beta, 0, sizeof(double) * M);
+    (void)hipMemset(c->d_comp, 0, sizeof(int32_t) * M);
+    (void)hipMemset(c->d_scal, 0, sizeof(double) * nscal);
+    (void)hipStreamSynchronize(nullptr);   // (as in brr_hip_create)
     if (reset_exchange(c) != BRR_HIP_OK) { brr_hip_destroy(c); return BRR_HIP_EDEVICE; }
     *out = c;
     return BRR_HIP_OK;

@@ -199,11 +199,11 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
     }
     for (uint32_t t = tid; t < p.G; t += kPipeThreads) {
         L.sigmaG[t] = p.scal[SL.sigmaG() + t];
-        L.betasqn[t] = 0.0;
+        L.betasqn[t] = (q->part & 1u) ? p.scal[SL.betasqn() + t] : 0.0;
     }
     for (uint32_t t = tid; t < p.G * p.K; t += kPipeThreads) {
         L.pi[t] = p.scal[SL.pi() + t];
-        L.v[t] = 0.0;
+        L.v[t] = (q->part & 1u) ? p.scal[SL.v() + t] : 0.0;
     }
     for (uint32_t t = tid; t < p.G * (p.K - 1); t += kPipeThreads) L.cva[t] = p.cva[t];
     for (uint32_t t = tid; t < p.F; t += kPipeThreads) {
@@ -378,7 +378,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                 goto done;
             break;
         }
-        if (p.mode == kModeChain) {
+        if (p.mode == kModeChain && !(q->part & 1u)) {
             // ---- updateMu (DenseBayesRRmz.cpp:36-42 / SparseBayesRRG.cpp:106-113)
             const double old_mu = L.mu;
             double new_mu = 0.0;
@@ -855,7 +855,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
 
-        if (p.mode == kModeChain) {
+        if (p.mode == kModeChain && !(q->part & 2u)) {
             double e2 = 0.0;
             const bool ok = fp64_region([&](double (&ed)[R][8]) {
                 // ---- fixed effects (BayesRBase.cpp:212-235)

@@ -98,6 +98,7 @@ struct SweepParams {
     const uint32_t* dense;
     uint64_t col_words, col_bytes;
     const double* gram;           // pipelined sweep: the Gram rows of the launch's iterations (gram_kernel.hpp)
+    uint32_t part;                // pipelined sweep: 1: M markers from inside an iteration's order, 2: not its last ones
     const double* lut;            // M x 4, by dosage 0,1,2,missing
     // ragged arena
     const int32_t* ones;

@@ -353,16 +353,24 @@ int brr_hip_sweep(brr_hip_ctx* ctx, const uint32_t* order, const double* u, cons
  * M doubles, caller-owned, read only) and the kernel's exchange words, control
  * words and counters, and a bitmap that checks the order on the device, live
  * in the library's file-scope device scratch (1.53 MiB per GPU, held until the
- * process ends). Limits: single-chain BayesR contexts, M <= 4,194,304 markers
- * (BRR_HIP_EINVAL beyond); an order that is not a permutation is refused with
- * BRR_HIP_EINVAL before the sweep touches the state. Calls that overlap on one
+ * process ends). A context whose sweeps are pipelined (2-bit columns, slices of
+ * up to 1024 individuals) also uses its own Gram rows, 1 KB a marker for up to
+ * 262,144 markers, which the set-up calls allocate: markers and model, then
+ * brr_hip_set_launch, _set_async and _set_precision. Limits: single-chain
+ * BayesR contexts, M <= 4,194,304 markers (BRR_HIP_EINVAL beyond);
+ * BRR_HIP_ENOMEM if the device had no room for the Gram rows at set-up; an
+ * order that is not a permutation is refused with BRR_HIP_EINVAL before the
+ * sweep touches the state. Calls that overlap on one
  * GPU race on its scratch; calls in sequence (each is synchronous) are safe.
  * Outputs: the context's state, read as after brr_hip_sweep. */
 int brr_hip_sweep_noalloc(brr_hip_ctx* ctx, const uint32_t* d_order, const double* d_u, const double* d_z);
 
 /* A device-resident chain: `iterations` full runGibbs iterations (updateMu,
- * sweep, sigmaE / sigmaG / pi draws) in one persistent launch, drawing u, z
- * and the scalars from the counter-based stream (seed, chain). orders holds
+ * sweep, sigmaE / sigmaG / pi draws) without a return to the host, drawing u, z
+ * and the scalars from the counter-based stream (seed, chain): persistent
+ * launches of up to 65,536 markers' visits, each after the launch that forms
+ * its Gram entries (more than 262,144 markers: an iteration in several); all
+ * iterations in one launch where the sweep is not pipelined. orders holds
  * the marker order of each iteration (iterations x M). hist (may be NULL)
  * receives iterations x (4 + G) doubles {mu, sigmaE, m0, |eps|^2, sigmaG[G]}.
  * Batched context: trait t draws from stream (seed, chain + t) and hist is

@@ -5,6 +5,8 @@ import numpy as np
 import pytest
 
 import bayesrrcmd_amd as brr
+import _oracle as orc
+import test_zz_no_alloc as na
 from _data import make_problem
 
 pytestmark = pytest.mark.gpu
@@ -75,4 +77,54 @@ def test_reload_that_gains_missing_calls(gpu_lib):
     for k, x in fresh.get_state().items():
         assert np.array_equal(h.get_state()[k], x), k
     fresh.close()
+    h.close()
+
+
+def rel(a, b):
+    a, b = np.asarray(a, float), np.asarray(b, float)
+    return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-30))
+
+
+# more markers than the Gram workspace has rows (262,144): each iteration in two launches. Sweeps against the oracle and
+# against the sweep that allocates nothing, then whole iterations against the oracle's. (262,144 + 65: the parts end inside
+# no block and the last one is short of a block)
+@pytest.mark.parametrize("layout,groups", [(DENSE, 1), (RAGGED, 2)], ids=["dense", "ragged-groups"])
+def test_iteration_in_parts(gpu_lib, layout, groups):
+    n, m = 64, 262144 + 65
+    pr = make_problem(n, m, seed=7, causal_frac=0.0001, maf=(0.3, 0.5))
+    S = np.tile(np.array(S4), (groups, 1))
+    group = (np.arange(m) % groups).astype(np.int32) if groups > 1 else None
+    kw = dict(bed=pr.bed, lut=pr.lut) if layout == DENSE else dict(ragged=pr.ragged)
+    o = orc.OracleProblem(n, m, layout, 4, groups, S, group=group, **kw)
+    o.init(pr.y, 9)
+    a, b = (context(pr, layout, brr.PRECISION_FP64, groups, 0) for _ in range(2))
+    order = np.arange(m, dtype=np.uint32)
+    for it in range(2):
+        brr.shuffle(5, it, 0, order)
+        u, z = brr.marker_uz(5, it, 0, m)
+        o.sweep(order, u, z, trace=False)
+        a.sweep(order, u, z)
+        assert na.noalloc(b, order, u, z) == 0, brr.lib().brr_hip_last_error(b.ctx)
+        sa, sb, ca, cb = a.get_state(), b.get_state(), a.get_scalars(), b.get_scalars()
+        assert np.count_nonzero(o.beta) > 100
+        assert np.array_equal(sa["comp"], o.comp) and np.array_equal(ca["v"].reshape(-1), o.v), it
+        for k, want in (("beta", o.beta), ("acum", o.acum), ("eps", o.eps)):
+            assert rel(sa[k], want) <= 1e-9, (it, k)
+        assert rel(ca["betasqn"], o.betasqn) <= 1e-9, it
+        for k in sa:
+            assert np.array_equal(sa[k], sb[k]), (it, k)
+        assert np.array_equal(ca["v"], cb["v"]) and np.array_equal(ca["betasqn"], cb["betasqn"])
+        assert a.stats()["rounds"] == 4097 + 1 and a.stats()["changes"] == b.stats()["changes"]
+    a.close()
+    b.close()
+    iters = 2
+    o = orc.OracleProblem(n, m, layout, 4, groups, S, group=group, **kw)
+    hist_o, _ = o.run_gibbs(pr.y, 9, iters)
+    cur = np.arange(m, dtype=np.uint32)
+    orders = np.stack([brr.shuffle(9, it, 0, cur).copy() for it in range(iters)])
+    h = context(pr, layout, brr.PRECISION_FP64, groups, 0)
+    hist = h.run_chain(9, 0, 0, orders)
+    assert np.array_equal(hist[:, 2], hist_o[:, 2]) and rel(hist, hist_o) <= 1e-8
+    st = h.get_state()
+    assert np.array_equal(st["comp"], o.comp) and rel(st["beta"], o.beta) <= 1e-8 and rel(st["eps"], o.eps) <= 1e-8
     h.close()

@@ -10,18 +10,20 @@ import pytest
 CSRC = Path(__file__).resolve().parents[1] / "bayesrrcmd_amd" / "csrc"
 SHIM = """
 #include "gram_plan.hpp"
-extern "C" void plan(uint32_t N, uint32_t M, uint32_t B, uint32_t total, uint64_t* out)
+extern "C" void plan(uint32_t N, uint32_t M, uint32_t B, uint32_t total, uint64_t most, uint64_t* out)
 {
-    const brr::GramPlan p = brr::gram_plan(N, M, B, total);
-    out[0] = p.step; out[1] = p.splits; out[2] = p.rows; out[3] = p.acc_rows;
-    out[4] = out[5] = out[6] = out[7] = 0;   // iterations, launches, largest rows, rows of split launches
-    for (uint32_t it = 0; it < p.total; it += p.step) {
-        const uint64_t rows = (uint64_t)p.iterations(it) * M;
-        out[4] += p.iterations(it);
-        out[5] += 1;
-        if (rows > out[6]) out[6] = rows;
-        if (p.splits > 1 && rows > out[7]) out[7] = rows;
-    }
+    const brr::GramPlan p = brr::gram_plan(N, M, B, total, most);
+    out[0] = p.step; out[1] = p.splits; out[2] = p.rows; out[3] = p.acc_rows; out[4] = p.parts;
+    out[5] = out[6] = out[7] = out[8] = 0;   // markers swept, launches, largest rows, rows of split launches
+    for (uint32_t it = 0; it < p.total; it += p.step)
+        for (uint32_t q = 0; q < p.parts; ++q) {
+            const uint64_t rows = (uint64_t)p.iterations(it) * p.markers(M, q);
+            out[5] += rows;
+            out[6] += 1;
+            if (rows == 0 || q * p.part % B) out[5] = ~0ull;   // an empty part, or one that starts inside a block
+            if (rows > out[7]) out[7] = rows;
+            if (p.splits > 1 && rows > out[8]) out[8] = rows;
+        }
 }
 """
 
@@ -34,10 +36,10 @@ def plan(tmp_path_factory):
                     str(d / "shim.so")], check=True)
     lib = C.CDLL(str(d / "shim.so"))
 
-    def call(n, m, b, total):
-        out = (C.c_uint64 * 8)()
-        lib.plan(n, m, b, total, out)
-        return dict(zip(("step", "splits", "rows", "acc_rows", "iterations", "launches", "used", "used_acc"), out))
+    def call(n, m, b, total, most=262144):
+        out = (C.c_uint64 * 9)()
+        lib.plan(n, m, b, total, C.c_uint64(most), out)
+        return dict(zip(("step", "splits", "rows", "acc_rows", "parts", "swept", "launches", "used", "used_acc"), out))
     return call
 
 
@@ -48,9 +50,21 @@ def test_launches_stay_inside_their_workspace(plan, n):
     for m, b, total in itertools.product(ms, [1, 2, 33, 64], [1, 2, 3, 7, 9, 23, 67, 100, 200, 400, 1000, 5000]):
         p = plan(n, m, b, total)
         at = (n, m, b, total, p)
-        assert p["iterations"] == total, at
-        assert p["used"] <= p["rows"] <= max(m, 65536), at
+        assert p["swept"] == total * m, at
+        assert p["used"] <= p["rows"] <= max(min(m, 262144), 65536), at
         assert p["used_acc"] <= p["acc_rows"], at
         assert p["acc_rows"] == 0 or p["acc_rows"] <= 128 * 64, at
         # nearly equal launches, no more of them than their bound asks for
-        assert p["launches"] <= -(-total // max(1, 65536 // m)), at
+        assert p["launches"] <= -(-total // max(1, 65536 // m)) * p["parts"], at
+        assert p["parts"] == 1 or m > 262144, at
+
+
+# a workspace smaller than an iteration: the iteration in parts of whole blocks
+@pytest.mark.parametrize("most", [64, 100, 4096, 8192, 65536, 262144])
+def test_parts_stay_inside_a_small_workspace(plan, most):
+    for m, b, total in itertools.product([1, 63, 64, 65, 129, 4097, 8192, 8193, 70000, 300001], [1, 2, 33, 64], [1, 2, 5]):
+        p = plan(5000, m, b, total, most)
+        at = (most, m, b, total, p)
+        assert p["swept"] == total * m, at
+        assert p["used"] <= p["rows"] <= most, at
+        assert p["used_acc"] <= p["acc_rows"] and (p["acc_rows"] == 0 or p["acc_rows"] <= 128 * 64), at
