@@ -1656,83 +1656,100 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
         launches[l].push_back(q);
         used[l] += ctxs[q]->P;
     }
-    // Iterations per launch: as many as fit the cohorts' Gram workspaces (together at most eight launches' worth of
-    // one context, at least one iteration)
+    // The Gram rows of all cohorts of a step in one launch and one workspace, the leading context's: as many iterations as
+    // fit eight launches' worth of one context, at least one, up to kCohortRowsMost rows. Where that is too little for
+    // an iteration, or the device has less room, an iteration is swept in parts.
     size_t rows1 = 0;
     bool many = false;
     for (uint32_t q = 0; q < n; ++q) {
+        if ((rc = prepare_shares(ctxs[q]))) return fail(c0, rc, ctxs[q]->err);
         rows1 += ctxs[q]->cfg.num_snps;
         many = many || ctxs[q]->many;
     }
-    const uint32_t step = (uint32_t)std::min<size_t>(iterations, std::max<size_t>(1, 8 * kGramRowsPerLaunch / rows1));
-    const uint32_t steps = (iterations + step - 1) / step;
-    for (uint32_t q = 0; q < n; ++q)
-        if ((rc = gram_reserve_rows(ctxs[q], (size_t)step * ctxs[q]->cfg.num_snps))) return fail(c0, rc, ctxs[q]->err);
-    HIP_TRY(c0, hipDeviceSynchronize());
-    // parameter blocks by step in launch order, on the device; the Gram entries of all cohorts of a step in one launch
-    std::vector<SweepParams> packed;
-    std::vector<GramEntry> grams;
-    std::vector<uint32_t> gram_items(steps, 0);
-    for (uint32_t st = 0; st < steps; ++st) {
-        const uint32_t it0 = st * step, its = std::min(step, iterations - it0);
-        for (auto& L : launches)
-            for (uint32_t q : L) {
-                const brr_hip_ctx* c = ctxs[q];
-                SweepParams p = params[q];
-                p.iterations = its;
-                p.iter_base += it0;
-                p.order += (size_t)it0 * p.M;
-                p.hist += (size_t)it0 * (4 + p.G);
-                p.gram = c->d_gram;
-                packed.push_back(p);
-                GramEntry g{gram_params(c, p, its, 1), gram_items[st]};
-                grams.push_back(g);
-                gram_items[st] += its * ((g.p.M + g.p.B - 1) / g.p.B);
-            }
+    CohortPlan plan;
+    for (size_t most = std::max(8 * kGramRowsPerLaunch, std::min(rows1, kCohortRowsMost));; most /= 2) {
+        std::vector<uint32_t> M(n), B(n);
+        for (uint32_t q = 0; q < n; ++q) { M[q] = ctxs[q]->cfg.num_snps; B[q] = ctxs[q]->B; }
+        plan = cohort_plan(M, B, iterations, most);
+        if ((rc = gram_reserve_rows(c0, plan.rows))) return rc;
+        if (c0->gram_cap >= plan.rows) break;
+        if (most <= kGramRowsLeast) return fail(c0, BRR_HIP_ENOMEM, "no room for the cohorts' Gram rows");
     }
+    // parameter blocks on the device: all cohorts' (for the reset), then by step and launch those with markers in the step
+    std::vector<SweepParams> packed(params);
+    std::vector<GramEntry> grams;
+    struct Launch { CohortTable t; const void* fn; size_t at; };   // at: its first parameter block
+    struct Step { size_t gram0; uint32_t grams, items; std::vector<Launch> launches; };
+    std::vector<Step> steps;
+    for (uint32_t it0 = 0; it0 < iterations; it0 += plan.step)
+        for (uint32_t part = 0; part < plan.parts; ++part) {
+            const uint32_t its = std::min(plan.step, iterations - it0);
+            Step st{grams.size(), 0, 0, {}};
+            size_t row = 0;
+            for (auto& L : launches) {
+                Launch la{};
+                const size_t first = packed.size();
+                uint32_t wg = 0, R = 1;
+                for (uint32_t q : L) {
+                    const brr_hip_ctx* c = ctxs[q];
+                    const uint32_t M = c->cfg.num_snps, m0 = plan.first(M, c->B, part), m1 = plan.first(M, c->B, part + 1);
+                    if (m0 == m1) continue;
+                    SweepParams p = params[q];
+                    p.M = m1 - m0;
+                    p.part = (m0 ? 1u : 0u) | (m1 < M ? 2u : 0u);
+                    p.iterations = its;
+                    p.iter_base += it0;
+                    p.order += (size_t)it0 * M + m0;
+                    p.hist += (size_t)it0 * (4 + p.G);
+                    p.gram = c0->d_gram + row * kGramCols;
+                    packed.push_back(p);
+                    GramEntry g{gram_params(c, p, its, 1), st.items};
+                    g.p.gram = c0->d_gram + row * kGramCols;
+                    grams.push_back(g);
+                    st.items += its * ((p.M + p.B - 1) / p.B);
+                    row += (size_t)its * p.M;
+                    la.t.first[la.t.n++] = wg;
+                    wg += c->P;
+                    // the launch's lane runs: the most any of its cohorts needs (a slice shorter than the kernel's
+                    // runs is masked at its end, as in any context's last workgroup)
+                    R = std::max(R, c->R);
+                }
+                if (!la.t.n) continue;
+                la.t.first[la.t.n] = wg;
+                la.at = first;
+                la.fn = cohort_kernel_for(R, c0->f32);
+                int occ = 0;
+                if (!la.fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, la.fn, kPipeThreads, 0) != hipSuccess ||
+                    (uint64_t)occ * c0->cus < wg)
+                    return fail(c0, BRR_HIP_EDEVICE, "a cohort launch does not fit the device");
+                st.launches.push_back(la);
+            }
+            st.grams = (uint32_t)(grams.size() - st.gram0);
+            if (!st.grams) continue;
+            if (row > c0->gram_cap) return fail(c0, BRR_HIP_EDEVICE, "cohort steps beyond their Gram rows");
+            steps.push_back(std::move(st));
+        }
     if (c0->cohort_cap < packed.size()) {
         c0->cohort_cap = 0;
-        if ((rc = dalloc(c0, &c0->d_cohort, packed.size())) || (rc = dalloc(c0, &c0->d_cohort_gram, grams.size()))) return rc;
+        if ((rc = dalloc(c0, &c0->d_cohort, packed.size())) || (rc = dalloc(c0, &c0->d_cohort_gram, packed.size()))) return rc;
         c0->cohort_cap = (uint32_t)packed.size();
     }
     HIP_TRY(c0, hipMemcpy(c0->d_cohort, packed.data(), sizeof(SweepParams) * packed.size(), hipMemcpyHostToDevice));
     HIP_TRY(c0, hipMemcpy(c0->d_cohort_gram, grams.data(), sizeof(GramEntry) * grams.size(), hipMemcpyHostToDevice));
     // the cooperative cohort kernel of each launch: recorded into one graph with the counters' reset and the Gram
     // launches (or, with BRR_HIP_COHORTS_DIRECT, launched one after another)
-    std::vector<CohortTable> tables(launches.size());
-    std::vector<const void*> fns(launches.size());
-    uint32_t base = 0;
-    for (size_t l = 0; l < launches.size(); ++l) {
-        CohortTable& t = tables[l];
-        t.params = c0->d_cohort + base;
-        t.n = (uint32_t)launches[l].size();
-        uint32_t wg = 0;
-        for (uint32_t i = 0; i < t.n; ++i) { t.first[i] = wg; wg += ctxs[launches[l][i]]->P; }
-        t.first[t.n] = wg;
-        // the launch's lane runs: the most any of its cohorts needs (a slice shorter than the
-        // kernel's runs is masked at its end, as in any context's last workgroup)
-        uint32_t R = 1;
-        for (uint32_t q : launches[l]) R = std::max(R, ctxs[q]->R);
-        fns[l] = cohort_kernel_for(R, c0->f32);
-        int occ = 0;
-        if (!fns[l] || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fns[l], kPipeThreads, 0) != hipSuccess ||
-            (uint64_t)occ * c0->cus < wg)
-            return fail(c0, BRR_HIP_EDEVICE, "a cohort launch does not fit the device");
-        base += t.n;
-    }
     auto enqueue = [&]() -> hipError_t {
         cohort_reset_kernel<<<n, 64, 0, c0->stream>>>(c0->d_cohort);
         if (hipError_t e2 = hipGetLastError()) return e2;
-        for (uint32_t st = 0; st < steps; ++st) {
-            const GramEntry* g = c0->d_cohort_gram + (size_t)st * n;
-            if (many) gram_cohort_kernel<true><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
-            else gram_cohort_kernel<false><<<gram_items[st], kGramThreads, 0, c0->stream>>>(g, n);
+        for (Step& st : steps) {
+            const GramEntry* g = c0->d_cohort_gram + st.gram0;
+            if (many) gram_cohort_kernel<true><<<st.items, kGramThreads, 0, c0->stream>>>(g, st.grams);
+            else gram_cohort_kernel<false><<<st.items, kGramThreads, 0, c0->stream>>>(g, st.grams);
             if (hipError_t e2 = hipGetLastError()) return e2;
-            for (size_t l = 0; l < launches.size(); ++l) {
-                CohortTable t = tables[l];
-                t.params += (size_t)st * n;
-                void* args[] = {&t};
-                const hipError_t e2 = hipLaunchCooperativeKernel(fns[l], dim3(t.first[t.n]), dim3(kPipeThreads), args, 0,
+            for (Launch& la : st.launches) {
+                la.t.params = c0->d_cohort + la.at;
+                void* args[] = {&la.t};
+                const hipError_t e2 = hipLaunchCooperativeKernel(la.fn, dim3(la.t.first[la.t.n]), dim3(kPipeThreads), args, 0,
                                                                  c0->stream);
                 if (e2 != hipSuccess) return e2;
             }

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <vector>
 
 namespace brr {
 
@@ -15,6 +16,8 @@ constexpr size_t kGramRowsPerLaunch = 65536;
 // Rows of the workspace at most: an iteration of more markers is swept in parts, a launch each. An iteration of 64
 // individuals and 300,000 markers takes 21.3 ms in two parts, 22.1 ms in one with 300 MB of rows.
 constexpr size_t kGramRowsMost = 262144;
+// Rows that a step of several contexts may take (8 GB; more markers in parts, which change a chain's roundings).
+constexpr size_t kCohortRowsMost = 8388608;
 // Rows below which a workspace that the device has no room for is not halved any more.
 constexpr size_t kGramRowsLeast = 8192;
 // Blocks from which a Gram launch is not split over the individuals. At N = 100,000 a sweep of 125 blocks takes
@@ -61,6 +64,44 @@ inline GramPlan gram_plan(uint32_t N, uint32_t M, uint32_t B, uint32_t total, si
     const uint64_t chunks = (N + kGramChunk - 1) / kGramChunk;
     p.splits = blocks >= kGramBlocks ? 1u : (uint32_t)std::max<uint64_t>(1, std::min(2 * kGramBlocks / blocks, chunks));
     p.acc_rows = p.splits > 1 ? p.rows : 0;
+    return p;
+}
+
+// The steps of a call over several contexts whose Gram rows share one workspace: `step` iterations each or, where one
+// iteration of all takes more than `most` rows, an iteration in `parts` of each context's blocks (a context with few blocks
+// sits out some of them).
+struct CohortPlan {
+    uint32_t step, parts;
+    size_t rows;          // rows of a step, at most
+
+    // first marker of part `part` of M markers in blocks of B (parts: M)
+    uint32_t first(uint32_t M, uint32_t B, uint32_t part) const
+    {
+        const uint64_t blocks = (M + B - 1) / B;
+        return (uint32_t)std::min<uint64_t>(M, blocks * part / parts * B);
+    }
+};
+
+inline CohortPlan cohort_plan(const std::vector<uint32_t>& M, const std::vector<uint32_t>& B, uint32_t total, size_t most)
+{
+    CohortPlan p{};
+    size_t rows1 = 0;
+    for (uint32_t m : M) rows1 += m;
+    if (rows1 <= most) {
+        const uint32_t fit = (uint32_t)std::min<size_t>(total, most / rows1);
+        const uint32_t steps = (total + fit - 1) / fit;
+        p.step = (total + steps - 1) / steps;
+        p.parts = 1;
+        p.rows = p.step * rows1;
+    } else {
+        p.step = 1;
+        p.parts = (uint32_t)((rows1 + most - 1) / most);
+        for (uint32_t part = 0; part < p.parts; ++part) {
+            size_t rows = 0;
+            for (size_t q = 0; q < M.size(); ++q) rows += p.first(M[q], B[q], part + 1) - p.first(M[q], B[q], part);
+            p.rows = std::max(p.rows, rows);
+        }
+    }
     return p;
 }
 

@@ -10,6 +10,22 @@ import pytest
 CSRC = Path(__file__).resolve().parents[1] / "bayesrrcmd_amd" / "csrc"
 SHIM = """
 #include "gram_plan.hpp"
+extern "C" void cohort_plan(uint32_t n, const uint32_t* M, const uint32_t* B, uint32_t total, uint64_t most, uint64_t* out)
+{
+    const brr::CohortPlan p = brr::cohort_plan(std::vector<uint32_t>(M, M + n), std::vector<uint32_t>(B, B + n), total, most);
+    out[0] = p.step; out[1] = p.parts; out[2] = p.rows;
+    out[3] = out[4] = 0;                     // markers of an iteration, largest rows of a step
+    for (uint32_t part = 0; part < p.parts; ++part) {
+        uint64_t rows = 0;
+        for (uint32_t q = 0; q < n; ++q) {
+            const uint32_t a = p.first(M[q], B[q], part), b = p.first(M[q], B[q], part + 1);
+            if (b < a || (b > a && a % B[q])) out[3] = 1ull << 62;
+            rows += b - a;
+        }
+        out[3] += rows;
+        if (rows * p.step > out[4]) out[4] = rows * p.step;
+    }
+}
 extern "C" void plan(uint32_t N, uint32_t M, uint32_t B, uint32_t total, uint64_t most, uint64_t* out)
 {
     const brr::GramPlan p = brr::gram_plan(N, M, B, total, most);
@@ -36,10 +52,17 @@ def plan(tmp_path_factory):
                     str(d / "shim.so")], check=True)
     lib = C.CDLL(str(d / "shim.so"))
 
+    def cohorts(ms, bs, total, most):
+        out = (C.c_uint64 * 5)()
+        arr = C.c_uint32 * len(ms)
+        lib.cohort_plan(len(ms), arr(*ms), arr(*bs), total, C.c_uint64(most), out)
+        return dict(zip(("step", "parts", "rows", "swept", "used"), out))
+
     def call(n, m, b, total, most=262144):
         out = (C.c_uint64 * 9)()
         lib.plan(n, m, b, total, C.c_uint64(most), out)
         return dict(zip(("step", "splits", "rows", "acc_rows", "parts", "swept", "launches", "used", "used_acc"), out))
+    call.cohorts = cohorts
     return call
 
 
@@ -68,3 +91,17 @@ def test_parts_stay_inside_a_small_workspace(plan, most):
         assert p["swept"] == total * m, at
         assert p["used"] <= p["rows"] <= most, at
         assert p["used_acc"] <= p["acc_rows"] and (p["acc_rows"] == 0 or p["acc_rows"] <= 128 * 64), at
+
+
+# the steps of several contexts: each holds every context's next iterations, or the next part of their blocks
+@pytest.mark.parametrize("most", [8192, 65536, 524288])
+def test_cohort_steps_stay_inside_their_workspace(plan, most):
+    for ms, bs in (([5], [64]), ([200, 4001, 64], [64, 64, 2]), ([20000] * 8, [64] * 8), ([300000, 1, 70000], [64, 64, 33]),
+                   ([100000] * 40, [64] * 40), ([64] * 9000, [64] * 9000), ([1] * 9000, [1] * 9000)):
+        for total in (1, 2, 3, 10, 1000):
+            p = plan.cohorts(ms, bs, total, most)
+            at = (most, ms[:4], len(ms), total, p)
+            assert 1 <= p["step"] <= total and (p["parts"] == 1 or p["step"] == 1), at
+            assert p["swept"] == sum(ms) and p["used"] == p["rows"], at
+            if max(ms) > 64 * len(ms):
+                assert p["rows"] <= most + 64 * len(ms), at
