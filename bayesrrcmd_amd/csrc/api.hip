@@ -807,12 +807,12 @@ int prepare_shares(brr_hip_ctx* c)
     int rc;
     const uint32_t M = c->cfg.num_snps;
     if (!c->counted) {
-        if ((rc = dalloc(c, &c->d_counts, (size_t)4 * M + 1))) return rc;
+        if (!c->d_counts && (rc = dalloc(c, &c->d_counts, (size_t)4 * M + 1))) return rc;
         marker_counts_kernel<<<M, 256, 0, c->stream>>>(c->d_dense, c->col_words, c->cfg.num_inds, c->d_counts);
         HIP_TRY(c, hipGetLastError());
         c->counted = true;
     }
-    if ((rc = dalloc(c, &c->d_markers, (size_t)M))) return rc;
+    if (!c->d_markers && (rc = dalloc(c, &c->d_markers, (size_t)M))) return rc;
     uint32_t* kind = c->d_counts + 4 * (size_t)M;
     uint32_t got = 0;
     HIP_TRY(c, hipMemsetAsync(kind, 0, sizeof(uint32_t), c->stream));
@@ -1351,7 +1351,7 @@ int brr_hip_load_bed(brr_hip_ctx* c, const uint8_t* bed_file, uint64_t file_byte
     uint32_t* d_stage = nullptr;
     uint32_t*& d_cnt = c->d_counts;
     int rc;
-    if ((rc = dalloc(c, &d_stage, stage_words)) || (rc = dalloc(c, &d_cnt, (size_t)4 * M + 1))) {
+    if ((rc = dalloc(c, &d_stage, stage_words)) || (!d_cnt && (rc = dalloc(c, &d_cnt, (size_t)4 * M + 1)))) {
         dfree(d_stage);
         return rc;
     }
