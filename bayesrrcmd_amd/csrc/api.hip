@@ -24,11 +24,14 @@ namespace brr {
 // instantiated in the kern_*.hip files
 BRR_SWEEP_SEQ_KERNELS(BRR_SWEEP_DECL)
 BRR_SWEEP_ASYNC_KERNELS(BRR_SWEEP_DECL)
-BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, false)
-BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, true)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, false, false)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, true, false)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, false, true)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_DECL, true, true)
 BRR_GRAM_DECL(false)
 BRR_GRAM_DECL(true)
-BRR_COHORT_KERNELS(BRR_COHORT_DECL)
+BRR_COHORT_KERNELS(BRR_COHORT_DECL, false)
+BRR_COHORT_KERNELS(BRR_COHORT_DECL, true)
 BRR_BATCH_KERNELS(BRR_BATCH_DECL)
 BRR_BATCH_F32_KERNELS(BRR_BATCH_DECL)
 BRR_BW_KERNELS(BRR_BW_DECL)
@@ -354,12 +357,12 @@ const void* async_kernel(int layout, bool codes)
                  : (const void*)bayesr_sweep_kernel<R, kLayoutRagged, false, true, false>;
 }
 
-template <int R, bool kF32>
+template <int R, bool kF32, bool kParts>
 const void* pipe_kernel(int layout)
 {
-    if (layout == kLayoutDense) return (const void*)bayesr_pipe_kernel<R, kLayoutDense, kF32>;
-    if (layout == kLayoutEigen) return (const void*)bayesr_pipe_kernel<R, kLayoutEigen, kF32>;
-    return (const void*)bayesr_pipe_kernel<R, kLayoutRagged, kF32>;
+    if (layout == kLayoutDense) return (const void*)bayesr_pipe_kernel<R, kLayoutDense, kF32, kParts>;
+    if (layout == kLayoutEigen) return (const void*)bayesr_pipe_kernel<R, kLayoutEigen, kF32, kParts>;
+    return (const void*)bayesr_pipe_kernel<R, kLayoutRagged, kF32, kParts>;
 }
 
 template <bool kF32>
@@ -375,6 +378,7 @@ struct SweepKernel {
     const void* fn;
     uint32_t threads;
     bool pipe;
+    const void* parts = nullptr;   // pipelined: of parts of an iteration
 };
 
 // Sequential sweeps over 2-bit codes take the pipelined kernel while a slice is one or two lane runs (four runs'
@@ -400,8 +404,10 @@ SweepKernel kernel_for(uint32_t R, int layout, bool codes, bool async, bool f32,
         }
     }
     switch (R) {
-    case 1: return {f32 ? pipe_kernel<1, true>(layout) : pipe_kernel<1, false>(layout), kPipeThreads, true};
-    case 2: return {f32 ? pipe_kernel<2, true>(layout) : pipe_kernel<2, false>(layout), kPipeThreads, true};
+    case 1: return {f32 ? pipe_kernel<1, true, false>(layout) : pipe_kernel<1, false, false>(layout), kPipeThreads, true,
+                    f32 ? pipe_kernel<1, true, true>(layout) : pipe_kernel<1, false, true>(layout)};
+    case 2: return {f32 ? pipe_kernel<2, true, false>(layout) : pipe_kernel<2, false, false>(layout), kPipeThreads, true,
+                    f32 ? pipe_kernel<2, true, true>(layout) : pipe_kernel<2, false, true>(layout)};
     case 4: return {f32 ? four_run_kernel<true>(layout) : four_run_kernel<false>(layout), kThreads, false};
     default: return {nullptr, kThreads, false};
     }
@@ -412,11 +418,12 @@ SweepKernel kernel_of(const brr_hip_ctx* c)
     return kernel_for(c->R, c->layout, c->codes, c->async != 0, c->f32, c->B);
 }
 
+template <bool kParts>
 const void* cohort_kernel_for(uint32_t R, bool f32)
 {
     switch (R) {
-    case 1: return f32 ? (const void*)bayesr_cohort_kernel<1, true> : (const void*)bayesr_cohort_kernel<1, false>;
-    case 2: return f32 ? (const void*)bayesr_cohort_kernel<2, true> : (const void*)bayesr_cohort_kernel<2, false>;
+    case 1: return f32 ? (const void*)bayesr_cohort_kernel<1, true, kParts> : (const void*)bayesr_cohort_kernel<1, false, kParts>;
+    case 2: return f32 ? (const void*)bayesr_cohort_kernel<2, true, kParts> : (const void*)bayesr_cohort_kernel<2, false, kParts>;
     default: return nullptr;
     }
 }
@@ -780,7 +787,7 @@ hipError_t enqueue_pipe(brr_hip_ctx* c, const SweepKernel& k, SweepParams& p, ui
     }
     p.gram = c->d_gram;
     void* args[] = {&p};
-    return hipLaunchCooperativeKernel(k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream);
+    return hipLaunchCooperativeKernel(p.part ? k.parts : k.fn, dim3(c->P), dim3(k.threads), args, 0, c->stream);
 }
 
 // The launches of `plan`: its iterations, or the parts of each.
@@ -1717,7 +1724,7 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
                 if (!la.t.n) continue;
                 la.t.first[la.t.n] = wg;
                 la.at = first;
-                la.fn = cohort_kernel_for(R, c0->f32);
+                la.fn = plan.parts > 1 ? cohort_kernel_for<true>(R, c0->f32) : cohort_kernel_for<false>(R, c0->f32);
                 int occ = 0;
                 if (!la.fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, la.fn, kPipeThreads, 0) != hipSuccess ||
                     (uint64_t)occ * c0->cus < wg)

@@ -4,5 +4,5 @@
 #include "kernels.hpp"
 
 namespace brr {
-BRR_COHORT_KERNELS(BRR_COHORT_INST)
+BRR_COHORT_KERNELS(BRR_COHORT_INST, false)
 } // namespace brr

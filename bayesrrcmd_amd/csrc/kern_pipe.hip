@@ -3,5 +3,5 @@
 #include "kernels.hpp"
 
 namespace brr {
-BRR_PIPE_KERNELS_OF(BRR_PIPE_INST, false)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_INST, false, false)
 } // namespace brr

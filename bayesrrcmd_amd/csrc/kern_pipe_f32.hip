@@ -4,5 +4,5 @@
 #include "kernels.hpp"
 
 namespace brr {
-BRR_PIPE_KERNELS_OF(BRR_PIPE_INST, true)
+BRR_PIPE_KERNELS_OF(BRR_PIPE_INST, true, false)
 } // namespace brr

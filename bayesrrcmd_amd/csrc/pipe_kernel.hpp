@@ -118,7 +118,9 @@ struct PipeShared {
 // lanes, at 300 moves a step; read again they cost a cached scalar load.
 typedef const __attribute__((address_space(4))) SweepParams* ConstParams;
 
-template <int R, int kLay, bool kF32>
+// kParts: launches of a part of an iteration (SweepParams::part). A body of their own: the tests of those flags moved the
+// whole one's registers about, 11% of a sweep at N = 100,000 with slices of 400 individuals.
+template <int R, int kLay, bool kF32, bool kParts>
 __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, PipeShared<R, kLay, kF32>& L,
                                           const uint32_t w)
 {
@@ -199,11 +201,11 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
     }
     for (uint32_t t = tid; t < p.G; t += kPipeThreads) {
         L.sigmaG[t] = p.scal[SL.sigmaG() + t];
-        L.betasqn[t] = (q->part & 1u) ? p.scal[SL.betasqn() + t] : 0.0;
+        L.betasqn[t] = kParts && (q->part & 1u) ? p.scal[SL.betasqn() + t] : 0.0;
     }
     for (uint32_t t = tid; t < p.G * p.K; t += kPipeThreads) {
         L.pi[t] = p.scal[SL.pi() + t];
-        L.v[t] = (q->part & 1u) ? p.scal[SL.v() + t] : 0.0;
+        L.v[t] = kParts && (q->part & 1u) ? p.scal[SL.v() + t] : 0.0;
     }
     for (uint32_t t = tid; t < p.G * (p.K - 1); t += kPipeThreads) L.cva[t] = p.cva[t];
     for (uint32_t t = tid; t < p.F; t += kPipeThreads) {
@@ -378,7 +380,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
                 goto done;
             break;
         }
-        if (p.mode == kModeChain && !(q->part & 1u)) {
+        if (p.mode == kModeChain && !(kParts && (q->part & 1u))) {
             // ---- updateMu (DenseBayesRRmz.cpp:36-42 / SparseBayesRRG.cpp:106-113)
             const double old_mu = L.mu;
             double new_mu = 0.0;
@@ -855,7 +857,7 @@ __device__ __forceinline__ void pipe_body(const SweepParams& p, ConstParams q, P
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
 
-        if (p.mode == kModeChain && !(q->part & 2u)) {
+        if (p.mode == kModeChain && !(kParts && (q->part & 2u))) {
             double e2 = 0.0;
             const bool ok = fp64_region([&](double (&ed)[R][8]) {
                 // ---- fixed effects (BayesRBase.cpp:212-235)
@@ -928,12 +930,12 @@ done:
     }
 }
 
-template <int R, int kLay, bool kF32>
+template <int R, int kLay, bool kF32, bool kParts>
 __global__ void __launch_bounds__(kPipeThreads)
 bayesr_pipe_kernel(SweepParams p)
 {
     __shared__ PipeShared<R, kLay, kF32> L;
-    pipe_body<R, kLay, kF32>(p, (ConstParams)__builtin_amdgcn_kernarg_segment_ptr(), L, blockIdx.x);
+    pipe_body<R, kLay, kF32, kParts>(p, (ConstParams)__builtin_amdgcn_kernarg_segment_ptr(), L, blockIdx.x);
 }
 
 // ------------------------------------------------------- cohorts in one launch --
@@ -950,7 +952,7 @@ struct CohortTable {
     uint32_t first[kMaxCohorts + 1];    // first workgroup of each cohort; first[n] = grid size
 };
 
-template <int R, bool kF32>
+template <int R, bool kF32, bool kParts>
 __global__ void __launch_bounds__(kPipeThreads)
 bayesr_cohort_kernel(CohortTable t)
 {
@@ -964,9 +966,9 @@ bayesr_cohort_kernel(CohortTable t)
     const SweepParams p = t.params[c];
     const ConstParams q = (ConstParams)(uint64_t)(t.params + c);   // (not written while the kernel runs)
     const uint32_t w = blockIdx.x - t.first[c];
-    if (p.layout == kLayoutDense) pipe_body<R, kLayoutDense, kF32>(p, q, L.d, w);
-    else if (p.layout == kLayoutEigen) pipe_body<R, kLayoutEigen, kF32>(p, q, L.e, w);
-    else pipe_body<R, kLayoutRagged, kF32>(p, q, L.r, w);
+    if (p.layout == kLayoutDense) pipe_body<R, kLayoutDense, kF32, kParts>(p, q, L.d, w);
+    else if (p.layout == kLayoutEigen) pipe_body<R, kLayoutEigen, kF32, kParts>(p, q, L.e, w);
+    else pipe_body<R, kLayoutRagged, kF32, kParts>(p, q, L.r, w);
 }
 
 } // namespace brr
