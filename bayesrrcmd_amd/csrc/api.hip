@@ -1642,18 +1642,18 @@ int brr_hip_run_cohorts(brr_hip_ctx* const* ctxs, uint32_t n, uint64_t seed, con
         p.refresh_blocks = std::max(1u, c->refresh_markers / c->B);
         params[q] = p;
     }
-    // launches: cohorts by decreasing estimated time of an iteration, first
+    // launches: cohorts by decreasing estimated chain length in exchange rounds, first
     // fit into launches of at most one workgroup per compute unit and kMaxCohorts
     // cohorts (so each launch's first cohort sets its length)
     std::vector<uint32_t> byLen(n);
     for (uint32_t q = 0; q < n; ++q) byLen[q] = q;
-    // an iteration takes about 4 us for each block, its one exchange included, and 0.7 us for each beta change (3.5 to 5.0
-    // and 0.68 to 0.75 from N = 700 to 100,000): the change rate of the context's last launch estimates the latter
-    auto length = [&](uint32_t q) {
+    // a chain's exchange rounds per iteration are about M / B + its beta changes: the
+    // change rate of the context's last launch estimates the latter
+    auto rounds_est = [&](uint32_t q) {
         const brr_hip_ctx* c = ctxs[q];
-        return (double)c->cfg.num_snps * (4.0 / (double)c->B + 0.7 * std::min(1.0, c->change_rate));
+        return (double)c->cfg.num_snps * (1.0 / (double)c->B + std::min(1.0, c->change_rate));
     };
-    std::stable_sort(byLen.begin(), byLen.end(), [&](uint32_t a, uint32_t b) { return length(a) > length(b); });
+    std::stable_sort(byLen.begin(), byLen.end(), [&](uint32_t a, uint32_t b) { return rounds_est(a) > rounds_est(b); });
     std::vector<std::vector<uint32_t>> launches;
     std::vector<uint32_t> used;
     for (uint32_t q : byLen) {
