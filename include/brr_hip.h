@@ -249,9 +249,10 @@ int brr_hip_autotune(brr_hip_ctx* ctx, uint64_t seed, uint32_t iterations, brr_h
  * iterations x (4 + G_q), chains[q]: NULL or each context's chain index). The
  * contexts are packed into persistent cooperative launches, each cohort on a
  * disjoint set of workgroups (its context's own count) with its own exchange,
- * at most one workgroup per compute unit and 64 cohorts per launch, longest
- * chains first (markers x (1 / block + the context's last change rate)); the
- * launches are captured into one hipGraph and run by one graph launch. All contexts: one device, single-chain sequential
+ * at most one workgroup per compute unit and 64 cohorts per launch, those likely
+ * to take longest first (markers x (1 / block + the context's last change rate)); the
+ * launches, with those that form the cohorts' Gram entries, are captured into one
+ * hipGraph and run by one graph launch. All contexts: one device, single-chain sequential
  * BayesR without fixed effects, columns held as 2-bit codes, one residual
  * precision, slices of at most 1024 individuals (one or two lane runs; a context
  * with more is refused with BRR_HIP_EINVAL; brr_hip_set_launch sets a context's);
