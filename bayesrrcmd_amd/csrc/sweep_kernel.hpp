@@ -721,7 +721,10 @@ __device__ __forceinline__ bool fixed_effects(const SweepParams& p, LDS& L, doub
                                               uint32_t lo, uint32_t hi, int lane, AllReduce&& allreduce)
 {
     const int tid = threadIdx.x;
-    if (tid == 0) {
+    // By all lanes of wave 0, which write the same words, and not by lane 0 alone: at the end of a loop of one lane the
+    // compiler has put spills and copies of other values ahead of the instruction that turns the other lanes on again,
+    // and they were lost in those.
+    if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
         for (uint32_t i = 1; i < p.F; ++i) {
             const U4 x = draw_block(p.seed, i, iteration, kStreamFixed, p.chain);
             const uint64_t r = ((uint64_t)x.x[0] << 32) | x.x[1];
