@@ -2488,6 +2488,7 @@ int brr_hip_bw_set_fixed(brr_hip_ctx* c, const float* X, uint32_t num_fixed)
     HIP_TRY(c, hipMemcpy(c->d_fixedX, X, sizeof(float) * N * num_fixed, hipMemcpyHostToDevice));
     HIP_TRY(c, hipMemset(c->d_fixed, 0, sizeof(double) * num_fixed));   // m_theta.setZero()
     HIP_TRY(c, hipMemset(c->d_sumf_fix, 0, sizeof(double) * num_fixed));
+    HIP_TRY(c, hipStreamSynchronize(nullptr));   // (the context's stream does not wait for the null stream)
     c->F = num_fixed;
     if (c->have_model) {
         bw_fixed_sumf_kernel<<<c->F, kThreads, 0, c->stream>>>(c->d_fixedX, N, c->d_fail, c->d_sumf_fix);
