@@ -1900,6 +1900,7 @@ int brr_hip_record_num(brr_hip_ctx* c, int enable)
         if (rc) return rc;
     }
     HIP_TRY(c, hipMemset(c->d_num, 0, sizeof(double) * c->cfg.num_snps));
+    HIP_TRY(c, hipStreamSynchronize(nullptr));   // (the context's stream does not wait for the null stream)
     c->record_num = true;
     return BRR_HIP_OK;
 }
